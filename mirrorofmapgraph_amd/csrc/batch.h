@@ -52,16 +52,17 @@ __device__ __forceinline__ M8 shfl_xor8(const M8 &x, int o) {
 }
 
 // Calls fn(v) for the set bits of a bitmap, block-uniformly: each round a
-// workgroup compacts BLK/2 words into LDS and hands them out BLK at a time (fn is
+// workgroup compacts slice_words words into LDS and hands them out BLK at a time (fn is
 // called by every thread, with v = -1 for padding).
 template <class Fn>
 __device__ void for_each_bit(const uint32_t *bm, int nwords, Fn fn) {
     constexpr int WPR = BLK / 2;
     __shared__ int s_q[WPR * 32];
     __shared__ int s_w[BLK / WAVE];
-    for (int w0 = blockIdx.x * WPR; w0 < nwords; w0 += gridDim.x * WPR) {
+    const int wpr = slice_words<BLK>(nwords);
+    for (int w0 = blockIdx.x * wpr; w0 < nwords; w0 += gridDim.x * wpr) {
         const int w = w0 + (int)threadIdx.x;
-        uint32_t word = (threadIdx.x < WPR && w < nwords) ? bm[w] : 0u;
+        uint32_t word = ((int)threadIdx.x < wpr && w < nwords) ? bm[w] : 0u;
         int total;
         int k = block_exclusive_scan<BLK>(__popc(word), s_w, &total);
         while (word) {
@@ -85,9 +86,10 @@ __device__ void for_each_bit_clear(uint32_t *bm, int nwords, Fn fn) {
     constexpr int WPR = BLK / 2;
     __shared__ int s_q[WPR * 32];
     __shared__ int s_w[BLK / WAVE];
-    for (int w0 = blockIdx.x * WPR; w0 < nwords; w0 += gridDim.x * WPR) {
+    const int wpr = slice_words<BLK>(nwords);
+    for (int w0 = blockIdx.x * wpr; w0 < nwords; w0 += gridDim.x * wpr) {
         const int w = w0 + (int)threadIdx.x;
-        uint32_t word = (threadIdx.x < WPR && w < nwords) ? bm[w] : 0u;
+        uint32_t word = ((int)threadIdx.x < wpr && w < nwords) ? bm[w] : 0u;
         if (word) bm[w] = 0;
         int total;
         int k = block_exclusive_scan<BLK>(__popc(word), s_w, &total);

@@ -548,7 +548,7 @@ int batch_dev_alloc(BatchDev &b, mg_graph *g, bool sssp, int slots) {
     b.S = slots;
     b.KS = (slots + 15) / 16 * 16;
     b.nwords = (int)(((n + 63) / 64) * 2);
-    b.G = sssp ? grid_blocks(std::max<int64_t>(g->n / 4, g->m / 16), BLK) : grid_blocks(std::max<int64_t>(g->n / 4, g->m / 64), BLK);
+    b.G = level_blocks(g->n, g->m, sssp ? 16 : 64, MAX_GRID);
     b.task_need = sssp ? g->m / SB_TASK + (int64_t)n + 64 : 2 * (g->m / TASK) + 64;
     b.task_cap = b.task_need;
     hipError_t e = hipSuccess;

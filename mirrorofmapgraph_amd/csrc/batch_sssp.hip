@@ -187,10 +187,11 @@ __device__ void for_each_bit_wave(uint32_t *bm, int nwords, bool clear, Fn fn) {
     __shared__ int s_q[WPR * 32];
     __shared__ int s_w[BLK / WAVE];
     const int lane = lane_id(), wv = (int)threadIdx.x / WAVE;
-    for (int w0 = blockIdx.x * WPR; w0 < nwords; w0 += gridDim.x * WPR) {
+    const int wpr = slice_words<BLK>(nwords);
+    for (int w0 = blockIdx.x * wpr; w0 < nwords; w0 += gridDim.x * wpr) {
         const int w = w0 + (int)threadIdx.x;
         uint32_t word = 0;
-        if (threadIdx.x < WPR && w < nwords) {
+        if ((int)threadIdx.x < wpr && w < nwords) {
             word = bm[w];
             if (clear && word) bm[w] = 0;
         }

@@ -589,7 +589,7 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
     a.depth = ws.vals;
     a.visited = ws.visited;
     a.hard = ws.hard;
-    a.G = o.level_grid > 0 ? o.level_grid : grid_blocks(std::max<int64_t>(g->n / 4, g->m / 64), BLK);
+    a.G = o.level_grid > 0 ? o.level_grid : level_blocks(g->n, g->m, 64, MAX_GRID);
     const long long m_views = g->m * a.fa.nviews;
 
     MG_HIP(hipEventRecord(g->ev0, g->stream));

@@ -218,6 +218,10 @@ void free_dev(void *p);
 int grid_blocks(int64_t work_items, int block);
 // As grid_blocks, capped at `cap` workgroups instead of MAX_GRID.
 int grid_blocks_cap(int64_t work_items, int block, int cap);
+// Workgroups of the level kernels of a search over n vertices and m edges: a thread per
+// four vertices or per_thread edges, and one per vertex while that is at most 1024
+// workgroups (four per CU), so graphs of up to 256K vertices are spread over the GPU.
+int level_blocks(int64_t n, int64_t m, int per_thread, int cap);
 
 // Per-call bookkeeping shared by the search entry points.
 struct CallTimer {

@@ -28,6 +28,11 @@ int grid_blocks_cap(int64_t work_items, int block, int cap) {
     return (int)b;
 }
 
+int level_blocks(int64_t n, int64_t m, int per_thread, int cap) {
+    const int64_t spread = std::min<int64_t>(n, 1024 * BLK);
+    return grid_blocks_cap(std::max({n / 4, m / per_thread, spread}), BLK, cap);
+}
+
 bool alloc_refused() {
     static std::mutex mu;
     static std::string armed;

@@ -369,17 +369,36 @@ __device__ void expand_tile_range(const FrontierArgs &fa, P &pol, int view, int 
     __syncthreads();
 }
 
+// Bitmap words a workgroup compacts per round: a share of the bitmap over up to 1024
+// workgroups, between BLOCK/32 words (BLOCK vertices: one tile when every bit is set) and
+// BLOCK/2 (the LDS list's size).  With rounds of BLOCK/2 words on every graph the small
+// ones left most of the GPU idle (16 of 128 workgroups had work at 64K vertices, 49 of
+// 196 at 200K) and each busy workgroup walked thousands of vertices; from 4M vertices up
+// the rounds are the same.  Smaller shares than 1/1024 cost the large graphs (4M vertices
+// in slices of 17 words: SSSP 1.2% slower).  Measured together with a thread per vertex
+// for the level kernels (level_blocks): BFS of 64K vertices 166 -> 156 us, directed SSSP
+// of 200K 652 -> 555 us, 100 batched SSSP sources on 250K vertices 9.92 -> 8.29 ms, 256
+// batched BFS sources on 1M 7.23 -> 5.76 ms, 64 batched SSSP sources on a 512^2 grid
+// 93.0 -> 76.1 ms.
+template <int BLOCK>
+__device__ __forceinline__ int slice_words(int nwords) {
+    const int wgs = min((int)gridDim.x, 1024);
+    const int share = (nwords + wgs - 1) / wgs;
+    return max(BLOCK / 32, min(share, BLOCK / 2));
+}
+
 // Multi-workgroup top-down over the frontier bitmap `fr`: each round a workgroup
-// compacts BLOCK/2 words (BLOCK*16 vertices) into LDS and expands them in tiles.
+// compacts slice_words words into LDS and expands them in tiles.
 template <int BLOCK, class P>
 __device__ void expand_bitmap(const FrontierArgs &fa, P &pol, int view, int L, const uint32_t *fr) {
     constexpr int WPR = BLOCK / 2;
     __shared__ int s_q[WPR * 32];
     __shared__ int s_wave2[BLOCK / WAVE];
     auto no_emit = [](int, bool) {};
-    for (int w0 = blockIdx.x * WPR; w0 < fa.nwords; w0 += gridDim.x * WPR) {
+    const int wpr = slice_words<BLOCK>(fa.nwords);
+    for (int w0 = blockIdx.x * wpr; w0 < fa.nwords; w0 += gridDim.x * wpr) {
         const int w = w0 + (int)threadIdx.x;
-        uint32_t word = (threadIdx.x < WPR && w < fa.nwords) ? fr[w] : 0u;
+        uint32_t word = ((int)threadIdx.x < wpr && w < fa.nwords) ? fr[w] : 0u;
         int total;
         int k = block_exclusive_scan<BLOCK>(__popc(word), s_wave2, &total);
         while (word) {
@@ -407,7 +426,7 @@ template <class P>
 struct policy_defers<P, std::void_t<decltype(std::declval<P &>().defer(0, 0))>> : std::true_type {};
 
 // Multi-workgroup push over the frontier bitmap `fr` without workgroup barriers in
-// the edge loop: each round a workgroup compacts BLOCK/2 bitmap words into LDS; a
+// the edge loop: each round a workgroup compacts slice_words bitmap words into LDS; a
 // lane walks the edges of each listed vertex of degree <= LANE_T itself, longer
 // lists become TASK-edge task records (one reservation atomic per workgroup round)
 // for expand_tasks.  The policy's visit_range(view, v, payload, beg, end, stride, L)
@@ -421,9 +440,10 @@ __device__ void expand_lanes(const FrontierArgs &fa, P &pol, int view, int L, co
     __shared__ int s_tbase;
     __shared__ int s_tex[BLOCK], s_tv[BLOCK], s_tbeg[BLOCK], s_tend[BLOCK];
     const int *off = fa.off[view];
-    for (int w0 = blockIdx.x * WPR; w0 < fa.nwords; w0 += gridDim.x * WPR) {
+    const int wpr = slice_words<BLOCK>(fa.nwords);
+    for (int w0 = blockIdx.x * wpr; w0 < fa.nwords; w0 += gridDim.x * wpr) {
         const int w = w0 + (int)threadIdx.x;
-        uint32_t word = (threadIdx.x < WPR && w < fa.nwords) ? fr[w] : 0u;
+        uint32_t word = ((int)threadIdx.x < wpr && w < fa.nwords) ? fr[w] : 0u;
         int total;
         int k = block_exclusive_scan<BLOCK>(__popc(word), s_wave2, &total);
         while (word) {

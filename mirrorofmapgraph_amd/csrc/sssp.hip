@@ -1082,7 +1082,7 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     a.fa = make_frontier_args(g, o.directed);
     a.dist = ws.vals;
     a.w = g->w;
-    a.G = o.level_grid > 0 ? o.level_grid : grid_blocks_cap(std::max<int64_t>(g->n / 4, g->m / 64), BLK, BIG_GRID);
+    a.G = o.level_grid > 0 ? o.level_grid : level_blocks(g->n, g->m, 64, BIG_GRID);
     a.delta = sssp_width(g, o);
     a.bucketed = sssp_bucketed_levels(o);
     a.bucket_edges = o.sssp_bucket_edges < 0 ? 0 : o.sssp_bucket_edges > 0 ? (long long)o.sssp_bucket_edges
