@@ -55,7 +55,8 @@ struct LevelPart {
 // advanced on the device; the host only reads `done` every few queued levels.
 struct Ctl {
     int level;          // level being processed
-    int done;           // 1 once the search has converged or hit iter_limit
+    int done;           // 1 once the search has converged or hit iter_limit; 2 while it waits
+                        // for a team (team.h): no step runs until the team kernel did
     int dir;            // DIR_TD or DIR_BU for the current level
     int steps;          // BFS / SSSP: steps whose first kernel found the search running
     int qsize[3];       // sizes of the three rotating frontier queues
@@ -83,7 +84,10 @@ struct Ctl {
     long long far_hi;         // bucketed SSSP: highest bucket holding a waiting distance
     int pair_end;             // batched SSSP: pair slots below this are valid this iteration
     long long fmin;           // SSSP: a lower bound on the distances of the current frontier
+    int team_step;            // BFS / SSSP: steps run when the first team took over (0: none did)
 };
+
+struct TeamCtl;
 
 // Pooled per-search device state, grown on demand and reused across searches.
 struct Workspace {
@@ -100,6 +104,8 @@ struct Workspace {
     uint32_t *bm[3] = {nullptr, nullptr, nullptr};
     ChunkRec *chunks = nullptr;
     LevelPart *part = nullptr;  // 3 * BIG_GRID slots
+    TeamCtl *team = nullptr;  // team of the narrow levels and its record queues (team.h)
+    uint64_t *team_rec = nullptr;
     Ctl *ctl = nullptr;
     Ctl *h_ctl = nullptr;     // pinned host mirror
     unsigned long long *h_reach = nullptr;  // pinned: TEPS count and reached vertices of a result
@@ -257,6 +263,7 @@ struct StepGraph {
     hipGraphExec_t part[STEPS_PER_GRAPH] = {};  // part[i]: i steps (1 <= i < STEPS_PER_GRAPH; captured on first use)
     uint64_t key = ~0ULL;
     int64_t last_steps = 0;  // steps the previous search with this key ran (0: not counted)
+    int64_t team_step = 0;   // how many of them before its first team (0: none)
 };
 
 // Returns MG_OK once the device sets ctl->done; a search still running after
@@ -268,9 +275,10 @@ struct NoTail {
 // tail (optional) queues the work that follows a finished search.  When the step count
 // is known from the previous search it is queued behind those steps, before the one
 // wait; *tail_queued then says whether the search finished there with the tail run.
-template <class Step, class Tail = NoTail>
+// team (optional) queues the team kernel, for searches whose steps may stop for one.
+template <class Step, class Tail = NoTail, class Team = NoTail>
 int drive(mg_graph *g, Step step, int64_t max_steps, int kind = -1, uint64_t key = 0, Ctl *ctl = nullptr,
-          Ctl *h_ctl = nullptr, Tail tail = Tail(), bool *tail_queued = nullptr);
+          Ctl *h_ctl = nullptr, Tail tail = Tail(), bool *tail_queued = nullptr, Team team = Team());
 inline int not_converged(int64_t max_steps) {
     return set_error(MG_ERR_DEVICE, "the search did not finish within %lld steps", (long long)max_steps);
 }
@@ -316,9 +324,9 @@ struct mg_graph_steps {
 // Queues steps until the device reports `done`.  Steps run from a captured HIP graph
 // (kind >= 0) or as direct launches; the host reads the control block only between
 // batches of steps (1, 2, 4, ... graphs), never once per level.
-template <class Step, class Tail>
+template <class Step, class Tail, class Team>
 int mg::drive(mg_graph *g, Step step, int64_t max_steps, int kind, uint64_t key, Ctl *ctl, Ctl *h_ctl, Tail tail,
-              bool *tail_queued) {
+              bool *tail_queued, Team team) {
     Workspace &ws = g->ws;
     if (tail_queued) *tail_queued = false;
     if (!ctl) {
@@ -353,31 +361,41 @@ int mg::drive(mg_graph *g, Step step, int64_t max_steps, int kind, uint64_t key,
                 x = nullptr;
             }
             sg.exec = nullptr;
-            sg.last_steps = 0;
+            sg.last_steps = sg.team_step = 0;
             int rc = capture(STEPS_PER_GRAPH, &sg.exec);
             if (rc) return rc;
             sg.key = key;
         }
         auto finish = [&]() {
             // kinds whose steps count themselves: the next search starts with this many
-            sg.last_steps = (kind == KIND_BFS || kind == KIND_SSSP) ? h_ctl->steps : 0;
+            const bool counts = kind == KIND_BFS || kind == KIND_SSSP;
+            sg.last_steps = counts ? h_ctl->steps : 0;
+            sg.team_step = counts ? h_ctl->team_step : 0;
         };
         int64_t queued = 0, k = 1;
-        // A search like the previous one (same graph, kind and options) ran last_steps
-        // steps: queue exactly that many (full graphs, then one graph of the rest) before
-        // the first look at the control block, so no empty steps trail the search.
-        if (sg.last_steps > 0) {
-            int64_t left = std::min<int64_t>(sg.last_steps, max_steps);
-            for (; left >= STEPS_PER_GRAPH; left -= STEPS_PER_GRAPH, queued += STEPS_PER_GRAPH)
-                MG_HIP(hipGraphLaunch(sg.exec, g->stream));
-            if (left > 0) {  // one graph of the remaining steps (each graph boundary costs ~10 us)
-                if (!sg.part[left]) {
-                    int rc = capture((int)left, &sg.part[left]);
+        // exactly `count` steps: full graphs, then one graph of the rest (each graph
+        // boundary costs ~10 us)
+        auto queue_steps = [&](int64_t count) -> int {
+            queued += count;
+            for (; count >= STEPS_PER_GRAPH; count -= STEPS_PER_GRAPH) MG_HIP(hipGraphLaunch(sg.exec, g->stream));
+            if (count > 0) {
+                if (!sg.part[count]) {
+                    int rc = capture((int)count, &sg.part[count]);
                     if (rc) return rc;
                 }
-                MG_HIP(hipGraphLaunch(sg.part[left], g->stream));
-                queued += left;
+                MG_HIP(hipGraphLaunch(sg.part[count], g->stream));
             }
+            return MG_OK;
+        };
+        // A search like the previous one (same graph, kind and options) ran last_steps
+        // steps: queue exactly that many before the first look at the control block (with
+        // the team where the previous one took it), so no empty steps trail the search.
+        if (sg.last_steps > 0) {
+            const int64_t all = std::min<int64_t>(sg.last_steps, max_steps);
+            const int64_t before = sg.team_step > 0 ? std::min(sg.team_step, all) : all;
+            int rc = queue_steps(before);
+            if (!rc && sg.team_step > 0 && !(rc = team())) rc = queue_steps(all - before);
+            if (rc) return rc;
             // the search most likely ends here: queue its tail before the wait (if not,
             // the caller queues it again after the remaining steps)
             if (tail_queued) {
@@ -386,10 +404,14 @@ int mg::drive(mg_graph *g, Step step, int64_t max_steps, int kind, uint64_t key,
             }
             MG_HIP(hipMemcpyAsync(h_ctl, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, g->stream));
             MG_HIP(hipStreamSynchronize(g->stream));
-            if (h_ctl->done) {
+            if (h_ctl->done == 1) {
                 finish();
                 if (tail_queued) *tail_queued = true;
                 return MG_OK;
+            }
+            if (h_ctl->done == 2) {
+                queued = h_ctl->steps;  // the steps behind the pause did nothing
+                if ((rc = team())) return rc;
             }
         }
         while (queued < max_steps) {
@@ -397,11 +419,18 @@ int mg::drive(mg_graph *g, Step step, int64_t max_steps, int kind, uint64_t key,
                 MG_HIP(hipGraphLaunch(sg.exec, g->stream));
             MG_HIP(hipMemcpyAsync(h_ctl, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, g->stream));
             MG_HIP(hipStreamSynchronize(g->stream));
-            if (h_ctl->done) {
+            if (h_ctl->done == 1) {
                 finish();
                 return MG_OK;
             }
-            if (k < 16) k *= 2;
+            if (h_ctl->done == 2) {
+                queued = h_ctl->steps;
+                const int rc = team();
+                if (rc) return rc;
+                k = 1;
+            } else if (k < 16) {
+                k *= 2;
+            }
         }
         return not_converged(max_steps);
     }
@@ -413,8 +442,15 @@ int mg::drive(mg_graph *g, Step step, int64_t max_steps, int kind, uint64_t key,
         }
         MG_HIP(hipMemcpyAsync(h_ctl, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, g->stream));
         MG_HIP(hipStreamSynchronize(g->stream));
-        if (h_ctl->done) return MG_OK;
-        if (k < 64) k *= 2;
+        if (h_ctl->done == 1) return MG_OK;
+        if (h_ctl->done == 2) {
+            queued = h_ctl->steps;
+            const int rc = team();
+            if (rc) return rc;
+            k = 2;
+        } else if (k < 64) {
+            k *= 2;
+        }
     }
     return not_converged(max_steps);
 }

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "engine.h"
+#include "team.h"
 
 namespace mg {
 
@@ -78,6 +79,8 @@ static void free_workspace(Workspace &ws) {
     for (auto &p : ws.bm) dfree(p);
     dfree(ws.chunks);
     dfree(ws.part);
+    dfree(ws.team);
+    dfree(ws.team_rec);
     dfree(ws.ctl);
     if (ws.h_ctl) (void)hipHostFree(ws.h_ctl);
     if (ws.h_reach) (void)hipHostFree(ws.h_reach);
@@ -115,7 +118,9 @@ int ensure_workspace(mg_graph *g) {
         (rc = dalloc(&ws.bm[0], ws.nwords)) || (rc = dalloc(&ws.bm[1], ws.nwords)) ||
         (rc = dalloc(&ws.bm[2], ws.nwords)) || (rc = dalloc(&ws.chunks, ws.chunk_cap)) ||
         (rc = dalloc(&ws.part, 3 * BIG_GRID)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2)) ||
-        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP))) {
+        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP)) ||
+        // search views serve graphs that are not thin, within a byte budget: no team there
+        (!g->arrays_borrowed && ((rc = dalloc(&ws.team, 1)) || (rc = dalloc(&ws.team_rec, TEAM_RECS))))) {
         free_workspace(ws);
         return rc;
     }
@@ -581,6 +586,7 @@ int mg_graph_device_bytes(const mg_graph *g, int64_t *bytes) {
     if (!g || !bytes) return set_error(MG_ERR_INVALID_ARG, "null argument");
     const Workspace &ws = g->ws;
     int64_t b = g->topo_bytes;
+    if (ws.team) b += (int64_t)sizeof(TeamCtl) + 8LL * (int64_t)TEAM_RECS;
     if (ws.ctl) b += 4LL * ws.n * 5 + 4LL * ws.nwords * 4 + (int64_t)sizeof(ChunkRec) * ws.chunk_cap;
     if (ws.rank) b += 12LL * ws.n;
     if (g->steps)

@@ -19,7 +19,7 @@
 // kernels per large level.
 #include <climits>
 
-#include "frontier.h"
+#include "team.h"
 
 namespace mg {
 
@@ -44,6 +44,8 @@ struct SsspArgs {
     int bucketed;
     long long bucket_edges;
     int wmin;  // smallest edge weight (>= 0)
+    TeamCtl *team;  // team of the narrow levels (nullptr: not used)
+    uint64_t *team_rec;
 };
 
 constexpr long long UNBUCKETED = LLONG_MAX / 4;  // a bucket bound no distance reaches
@@ -672,7 +674,7 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
     __shared__ int s_beg[2 * SMALL_Q];       // list starts
     __shared__ int s_d[SMALL_Q];             // frontier distances
     __shared__ int s_wave[SMALL_BLK / WAVE];
-    __shared__ int s_go, s_L, s_cnt, s_levels, s_limit, s_canpull, s_alpha, s_nfar, s_keep, s_qv, s_nq;
+    __shared__ int s_go, s_L, s_cnt, s_levels, s_limit, s_canpull, s_alpha, s_nfar, s_keep, s_qv, s_nq, s_narrow;
     __shared__ long long s_m, s_thr;
     if (c->pending) {
         const int L = c->level;
@@ -688,6 +690,7 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
     }
     if (threadIdx.x == 0) {
         const int L = c->level;
+        s_narrow = c->small_levels;
         s_go = !c->done && c->dir == DIR_PUSH && c->qsize[L % 3] <= SMALL_Q && c->mf_cur <= SSSP_SMALL_E;
         s_L = L;
         s_cnt = c->qsize[L % 3];
@@ -954,13 +957,15 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
             // close level L on the LDS copy of the direction state (as sssp_close)
             trace_level(fa, L, DIR_PUSH, nf, mf);
             s_levels++;
-            s_go = nf > 0 && nf <= SMALL_Q && !(s_canpull && mf * s_alpha > s_m) && mf <= SSSP_SMALL_E &&
-                   L + 1 < s_limit;
+            const bool go = nf > 0 && nf <= SMALL_Q && !(s_canpull && mf * s_alpha > s_m) && mf <= SSSP_SMALL_E &&
+                            L + 1 < s_limit;
+            // a search that stays narrow is handed to a team
+            s_go = go && a.team && s_narrow + s_levels >= TEAM_AFTER ? 2 : go;
             s_L = L + 1;
             s_keep = nf;
         }
         __syncthreads();
-        if (s_go) continue;
+        if (s_go == 1) continue;
         // hand over: the queue and the far list become the next bitmap (the whole-GPU
         // levels relax every frontier vertex), then the control block takes the state
         uint32_t *nx = fa.bm[(L + 1) % 3];
@@ -974,10 +979,12 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
             }
         }
         __syncthreads();
+        const bool to_team = s_go == 2;  // (the far bitmap is the team's far list)
+        if (to_team) team_open(a.team);
         long long nf_far = 0, mf_far = 0, mf_q = 0;
         if (nf > SMALL_Q)  // out-edges of the queued part (build() skipped)
             for (int i = threadIdx.x; i < SMALL_Q; i += SMALL_BLK) mf_q += view_degree(fa, s_q[i]);
-        const int nfar = s_nfar;
+        const int nfar = to_team ? 0 : s_nfar;
         for (int i = threadIdx.x; i < nfar; i += SMALL_BLK) {
             const int u = far[i];
             clear_bit_wg(farbm, u);
@@ -999,8 +1006,230 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
             c->thr = s_thr;
             advance_level(c, L, nft, mft);
             c->qvalid = 0;  // the queue stayed in LDS
+            if (to_team) {
+                c->done = 2;
+                if (c->team_step == 0) c->team_step = c->steps;
+            }
         }
         break;
+    }
+}
+
+// Narrow levels by a team (team.h), from the level sssp_small stopped at until the search
+// ends or outgrows the team's queues, with sssp_small's buckets.
+//
+// A wave takes TEAM_PIECE records of one member at a time, a lane per edge: neighbour and
+// weight with the vertex's distance, then the neighbour's distance and offsets, then for
+// a candidate the minimum and the claim together (a stale, larger distance only causes a
+// redundant relaxation).  Claims are test-and-sets: below the bucket bound in the next
+// level's frontier bitmap (the winner queues the vertex), else in the far bitmap, which
+// is the whole far list.  Whoever takes a vertex clears its frontier bit, so the bitmaps
+// rotate clean and always hold the frontier.  When no record is left the members move the
+// bound and sweep the far bitmap (n bits: about 1 us at 1M vertices, once per bucket).
+// Bound by the same chain as bfs_team with a distance load before the claim.  Grid
+// 1049 x 999, weights 1..16, about 2400 rounds: 38.0 -> 8.9 ms; 2048^2 127 -> 27 ms.
+__global__ __launch_bounds__(BLK) void sssp_team(SsspArgs a) {
+    Ctl *c = a.fa.ctl;
+    if (c->done != 2) return;
+    const FrontierArgs &fa = a.fa;
+    int rank, size;
+    if (!team_join(a.team, rank, size)) return;
+    const int lane = lane_id(), sub = lane % TEAM_EDGES;
+    const int *off = fa.off[0], *adj = fa.adj[0], *wts = a.w;
+    const int can_pull = c->can_bu, alpha = c->alpha, limit = c->iter_limit;
+    const long long m = c->m_unexplored, delta = a.delta;
+    long long thr = c->thr, ex = 0;
+    const int L0 = c->level;
+    int L = L0, it;
+    bool done = false, swept = false;  // swept: this meeting's records come from the far bitmap
+    {  // the first meeting: the frontier's records, from its bitmap
+        uint32_t *fr = fa.bm[L % 3];
+        TeamOut out(a.team_rec, 1, rank);
+        team_words(fr, fa.nwords, rank, size, [&](int i, uint32_t word) {
+            uint32_t todo = word, keep = 0;
+            while (wave_ballot(todo != 0)) {
+                const bool has = todo != 0;
+                const int b = has ? __ffs(todo) - 1 : 0, v = has ? i * 32 + b : 0;
+                todo &= todo - 1;
+                const IntPair o = ld_range(off, v);
+                const bool edges = has && o.b > o.a;  // one without has no record to clear its bit
+                if (edges) keep |= 1u << b;
+                const uint64_t takes = wave_ballot(edges);
+                if (takes) out.queue(edges, takes, v, o);
+            }
+            if (keep != word) __hip_atomic_store(&fr[i], keep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        });
+        team_post(a.team, 1, rank, out.word(1));
+    }
+    for (it = 1;; ++it) {
+        const uint64_t w = team_meet(a.team, it, size);
+        const TeamIn in = team_in(a.team_rec, it, w);
+        long long sweep_from = -1;  // >= 0: sweep, dropping waiting distances below this
+        // the same decisions in every wave
+        if (wave_ballot(team_over(w)) != 0) break;
+        const int mf = wave_total(team_mf(w));
+        if (it > 1 && !swept && rank == 0) {  // close level L - 1
+            const int nf = wave_total(team_nf(w));
+            if (lane == 0) trace_level(fa, L - 1, DIR_PUSH, nf, mf);
+        }
+        if (L >= limit) {
+            done = true;
+        } else if (in.pieces > 0) {
+            if (can_pull && (long long)mf * alpha > m) break;
+        } else if (thr >= UNBUCKETED) {
+            done = true;
+        } else if (!swept) {
+            sweep_from = thr;
+            thr += delta;
+        } else {
+            // nothing waits in that bucket: the one of the smallest waiting distance
+            int lo = lane < size ? ld_dev(&a.team->least[it & 1][lane]) : INT_MAX;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) lo = min(lo, __shfl_xor(lo, o));
+            if (lo == INT_MAX) {
+                done = true;
+            } else {
+                sweep_from = thr;
+                thr = ((long long)lo / delta + 1) * delta;
+            }
+        }
+        if (done) break;
+        TeamOut out(a.team_rec, it + 1, rank);
+        swept = sweep_from >= 0;
+        if (swept) {
+            // far vertices below the bound join frontier L (its bitmap is clear); those
+            // below the old bound were relaxed since and leave the far bitmap
+            uint32_t *fr = fa.bm[L % 3];
+            int least = INT_MAX;
+            team_words(a.farbm, fa.nwords, rank, size, [&](int i, uint32_t word) {
+                uint32_t todo = word, keep = 0, go = 0;
+                while (wave_ballot(todo != 0)) {
+                    const bool has = todo != 0;
+                    const int b = has ? __ffs(todo) - 1 : 0, u = has ? i * 32 + b : 0;
+                    todo &= todo - 1;
+                    const int d = ld_dev(&a.dist[u]);
+                    const IntPair o = ld_range(off, u);
+                    const bool take = has && d >= sweep_from && d < thr && o.b > o.a;
+                    if (has && d >= thr) {
+                        keep |= 1u << b;
+                        least = min(least, d);
+                    }
+                    if (take) go |= 1u << b;
+                    const uint64_t takes = wave_ballot(take);
+                    if (takes) out.queue(take, takes, u, o);
+                }
+                if (keep != word) __hip_atomic_store(&a.farbm[i], keep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (go) __hip_atomic_store(&fr[i], go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            });
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) least = min(least, __shfl_xor(least, o));
+            if (lane == 0)
+                __hip_atomic_store(&a.team->least[(it + 1) & 1][rank], least, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+            team_post(a.team, it + 1, rank, out.word(it + 1));
+            continue;
+        }
+        uint32_t *fr = fa.bm[L % 3], *nx = fa.bm[(L + 1) % 3];
+        auto relax = [&](auto kc, int p0) {
+            constexpr int K = decltype(kc)::value;
+            uint64_t rec[K];
+            int u[K], wt[K], dv[K], du[K];
+            bool on[K];
+            IntPair o[K];
+            uint32_t old[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                on[k] = true;
+                rec[k] = team_fetch(in, p0 + k * size, on[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                on[k] = on[k] && sub < rec_len(rec[k]);
+                const int e = rec_beg(rec[k]) + (on[k] ? sub : 0);
+                u[k] = adj[e];
+                wt[k] = wts[e];
+                dv[k] = ld_dev(&a.dist[rec_vertex(rec[k])]);
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                du[k] = ld_dev(&a.dist[u[k]]);
+                o[k] = ld_range(off, u[k]);
+                if (on[k] && sub == 0)
+                    __hip_atomic_store(&fr[rec_vertex(rec[k]) >> 5], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            bool cand[K], near[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const long long nd = (long long)dv[k] + wt[k];
+                ex += on[k];
+                cand[k] = on[k] && nd < du[k];
+                near[k] = nd < thr;
+                if (cand[k]) {
+                    __hip_atomic_fetch_min(&a.dist[u[k]], (int)nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    old[k] = __hip_atomic_fetch_or(&(near[k] ? nx : a.farbm)[u[k] >> 5], 1u << (u[k] & 31),
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                bool first = cand[k] && near[k] ? !((old[k] >> (u[k] & 31)) & 1u) : false;
+                // a vertex without out-edges has no record to clear its bit
+                if (first && o[k].a == o[k].b) {
+                    __hip_atomic_fetch_and(&nx[u[k] >> 5], ~(1u << (u[k] & 31)), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    first = false;
+                }
+                const uint64_t firsts = wave_ballot(first);
+                if (firsts) out.queue(first, firsts, u[k], o[k]);
+            }
+        };
+        int p = rank;
+        for (; p + size < in.pieces; p += 2 * size) relax(std::integral_constant<int, 2>(), p);
+        if (p < in.pieces) relax(std::integral_constant<int, 1>(), p);
+        ++L;
+        team_post(a.team, it + 1, rank, out.word(it + 1));
+    }
+    const bool lead = rank == 0 && lane == 0;
+    if (done) {
+        ex = wave_sum_ll(ex);
+        if (lane == 0) atomicAdd((unsigned long long *)&c->edges_examined, (unsigned long long)ex);
+        if (lead) {
+            c->small_levels += L - L0;
+            advance_level(c, L - 1, 0, 0);
+            c->qvalid = 0;
+            c->done = 1;
+        }
+        return;
+    }
+    // frontier L and the waiting vertices go to the whole-GPU levels as one frontier of a
+    // level that awaits its close
+    uint32_t *fr = fa.bm[L % 3];
+    long long nf = 0, mf = 0, mn = LLONG_MAX;
+    for (int i = rank * WAVE + lane; i < fa.nwords; i += size * WAVE) {
+        const uint32_t f = (uint32_t)ld_dev((const int *)a.farbm + i);
+        uint32_t word = (uint32_t)ld_dev((const int *)fr + i) | f;
+        if (!word) continue;
+        if (f) {
+            fr[i] = word;
+            a.farbm[i] = 0;
+        }
+        while (word) {
+            const int v = i * 32 + __ffs(word) - 1;
+            word &= word - 1;
+            const long long d = ld_dev(&a.dist[v]);
+            mn = d < mn ? d : mn;
+            ++nf;
+            mf += view_degree(fa, v);
+        }
+    }
+    write_part<BLK>(fa, nf, mf, ex, mn);
+    if (lead) {
+        c->small_levels += L - L0;
+        c->level = L - 1;
+        c->thr = thr;
+        c->pending = 1;
+        c->qvalid = 0;
+        c->done = 0;
     }
 }
 
@@ -1090,6 +1319,8 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     a.far = ws.hard;
     a.farbm = ws.visited;
     a.wmin = g->min_weight;
+    a.team = a.fa.nviews == 1 ? ws.team : nullptr;
+    a.team_rec = ws.team_rec;
     const int in_view = a.fa.off[2] != nullptr && a.fa.nviews == 1 && o.engine != MG_ENGINE_GAS;
     // pull levels relax every vertex from all its in-edges: unbucketed searches only
     const int can_pull = in_view && !a.bucketed;
@@ -1123,7 +1354,12 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     key = mix64(key ^ (uint64_t)a.G);
     bool tail_queued = false;
     auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, INT_MAX, ws.vals, 4 * (size_t)g->n); };
-    if ((rc = drive(g, step, max_steps, KIND_SSSP, key, nullptr, nullptr, tail, &tail_queued)))
+    auto team = [&]() -> int {
+        hipLaunchKernelGGL(sssp_team, dim3(TEAM_GRID), dim3(BLK), 0, g->stream, a);
+        MG_HIP(hipGetLastError());
+        return MG_OK;
+    };
+    if ((rc = drive(g, step, max_steps, KIND_SSSP, key, nullptr, nullptr, tail, &tail_queued, team)))
         return rc;
     rc = finish_search(g, stats, ws.vals, INT_MAX, dist_out, ws.vals, 4 * (size_t)g->n, o.out_on_device, timer,
                        tail_queued);

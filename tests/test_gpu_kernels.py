@@ -21,3 +21,95 @@ def test_frontier_slices_cover_ragged_graphs(mg, oracle, device, n):
             assert np.array_equal(got, oracle.bfs(g.row_offsets, g.col_idx, s))
         for got, s in zip(dg.sssp_batch(srcs), srcs):
             assert np.array_equal(got, oracle.sssp(g.row_offsets, g.col_idx, g.values, s))
+
+
+# ---------------------------------------------------------------- teams (narrow levels)
+def _chain(mg, lengths, hubs, seed, symmetric=True):
+    """Chains of the given lengths joined by stars: hubs[i] leaves around the end of chain i."""
+    src, dst, v = [], [], 0
+    for ln, hub in zip(lengths, hubs):
+        ids = np.arange(v, v + ln)
+        src.append(ids[:-1]), dst.append(ids[1:])
+        end = v + ln - 1
+        v += ln
+        if hub:
+            leaves = np.arange(v, v + hub)
+            src.append(np.full(hub, end)), dst.append(leaves)
+            v += hub
+            src.append(leaves[-1:]), dst.append([v])  # the next chain starts behind the last leaf
+    src, dst = np.concatenate(src).astype(np.int32), np.concatenate(dst).astype(np.int32)
+    keep = dst < v
+    flags = mg.MG_CSR_SORT_COLS | mg.MG_CSR_DEDUPE | (mg.MG_CSR_SYMMETRIZE if symmetric else 0)
+    g = mg.csr_from_edges(v, src[keep], dst[keep], flags)
+    g.values = mg.hash_weights(g, seed, 9)
+    return g
+
+
+def _team_graph(mg, which):
+    if which == "path":
+        return _chain(mg, [2500], [0], 3), True
+    if which == "hubs":  # stars around the record, member and vertex limits of a team
+        return _chain(mg, [40, 30, 30, 30, 20], [5, 1020, 1021, 9000, 0], 4), True
+    if which == "directed":  # sinks all along
+        return _chain(mg, [60, 200, 30], [33, 700, 0], 5, symmetric=False), False
+    if which == "zero":
+        g = mg.grid_graph(97, 61, seed=8, weight_max=3)
+        g.values = g.values - 1
+        return g, True
+    if which == "tails":  # chains into a dense graph and out of it
+        r = mg.rmat_graph(12, 16, seed=4)
+        k, n, hub = 60, r.n, int(np.argmax(r.degrees()))
+        a, b = np.arange(n, n + k), np.arange(n + k, n + 2 * k)
+        src = np.concatenate([np.repeat(np.arange(n), np.diff(r.row_offsets)), a[:-1], b[:-1], [a[-1], hub]])
+        dst = np.concatenate([r.col_idx, a[1:], b[1:], [hub, b[0]]])
+        g = mg.csr_from_edges(n + 2 * k, src.astype(np.int32), dst.astype(np.int32),
+                              mg.MG_CSR_SYMMETRIZE | mg.MG_CSR_DEDUPE | mg.MG_CSR_SORT_COLS)
+        g.values = mg.hash_weights(g, 3, 64)
+        return g, True
+    w, h = which
+    return mg.grid_graph(w, h, seed=w, weight_max=16), True
+
+
+@pytest.mark.parametrize("which", ["path", "hubs", "directed", "zero", "tails", (64, 64), (701, 13), (399, 403)])
+def test_teams_match_the_oracle(mg, oracle, device, which):
+    g, sym = _team_graph(mg, which)
+    with mg.Graph(g, symmetric=sym) as dg:
+        for src in {0, g.n // 2, g.n - 1}:
+            d, st = dg.bfs(src, stats=True)
+            exp = oracle.bfs(g.row_offsets, g.col_idx, src)
+            assert np.array_equal(d, exp)
+            assert st.edges_traversed == oracle.teps_edges(g.row_offsets, exp)
+            exp = oracle.sssp(g.row_offsets, g.col_idx, g.values, src)
+            for delta in (0, 1, 7, -1):
+                assert np.array_equal(dg.sssp(src, mg.options(sssp_delta=delta)), exp), (src, delta)
+
+
+@pytest.mark.parametrize("limit", [8, 9, 10, 11, 40])
+def test_team_stops_at_the_level_limit(mg, oracle, device, limit):
+    g = mg.grid_graph(90, 70, seed=2, weight_max=16)
+    with mg.Graph(g, symmetric=True) as dg:
+        d, st = dg.bfs(0, mg.options(iter_num=limit), stats=True)
+    exp = oracle.bfs(g.row_offsets, g.col_idx, 0)
+    assert st.iterations == limit
+    assert np.array_equal(d, np.where((exp >= 0) & (exp <= limit), exp, -1))
+
+
+def test_teams_of_several_graphs_at_once(mg, oracle, device):
+    """Teams on several streams share the GPU; none waits for a workgroup that is not running."""
+    import threading
+
+    hosts = [mg.grid_graph(150 + 31 * i, 120, seed=i, weight_max=16) for i in range(6)]
+    graphs = [mg.Graph(h, symmetric=True) for h in hosts]
+    got = [None] * len(hosts)
+
+    def work(i):
+        got[i] = [(graphs[i].bfs(s), graphs[i].sssp(s)) for s in (0, 77, 5000)]
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(len(hosts))]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    for h, rows in zip(hosts, got):
+        for s, (b, d) in zip((0, 77, 5000), rows):
+            assert np.array_equal(b, oracle.bfs(h.row_offsets, h.col_idx, s))
+            assert np.array_equal(d, oracle.sssp(h.row_offsets, h.col_idx, h.values, s))
+    [g.close() for g in graphs]
