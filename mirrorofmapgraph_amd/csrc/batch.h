@@ -143,6 +143,7 @@ struct BatchDev {
     int *D = nullptr;                            // SSSP distances, n x KS
     int *rows = nullptr;                         // S x n results
     int *rows_out = nullptr;                     // on a degree-ordered twin: rows in the caller's ids
+    bool deep = false;                           // BFS: a search outgrew the levels (batch_levels.hip)
     int2 *pairs = nullptr;                       // SSSP: (vertex, slot) pairs of sparse vertices
     int64_t pair_cap = 0;
     int nwords = 0;
@@ -198,6 +199,13 @@ int batch_live(BatchDev &b, hipStream_t st);
 int batch_row_stats(BatchDev &b, mg_graph *g, hipStream_t st, const SlotList &sl, int unreached);
 // Clears the assigned bits of `mask`.
 int batch_release_slots(BatchDev &b, hipStream_t st, const uint32_t mask[8]);
+
+int batch_alpha(const mg_options &o);
+int batch_beta(const mg_options &o);
+// Batched BFS by whole levels (batch_levels.hip).
+constexpr int LEVELS_ALPHA = 16;
+int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32_t *srcs, int32_t npairs, int32_t k,
+                   int32_t *depth_out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *deep);
 
 // ---- batched personalized PageRank (ppr.hip)
 constexpr int PPR_SLOTS = 64;  // slots per context: one per lane

@@ -727,6 +727,10 @@ int check_batch_sets(const char *fn, const mg_graph *g, const int32_t *slot_of, 
     return MG_OK;
 }
 
+// Graphs of at least this mean degree run by levels (batch_levels.hip) until a search turns
+// out deep; sparser ones (meshes: hundreds of levels) write rows as they go.
+constexpr int64_t LEVELS_DEGREE = 8;
+
 // Batched BFS with npairs (row, source) pairs; every row of [0, k) has a source.
 static int bfs_batch_run(mg_graph *g, const int32_t *slot_of, const int32_t *srcs, int32_t npairs, int32_t k,
                          int32_t *depth_out, const mg_options &o, mg_stats *stats, const CallTimer &timer) {
@@ -735,6 +739,12 @@ static int bfs_batch_run(mg_graph *g, const int32_t *slot_of, const int32_t *src
     if ((rc = graph_batch_dev(g, false, &b))) return rc;
     auto run = [&]() -> int {
         int rc;
+        if (!b->deep && g->m >= LEVELS_DEGREE * (int64_t)g->n) {
+            bool deep = false;
+            if ((rc = bfs_levels_run(g, *b, slot_of, srcs, npairs, k, depth_out, o, stats, timer, &deep)) || !deep)
+                return rc;
+            b->deep = true;
+        }
         MG_HIP(hipEventRecord(g->ev0, g->stream));
         if ((rc = bfs_batch_reset(*b, g, g->stream, o.iter_num, batch_alpha(o), batch_beta(o), 0))) return rc;
         if ((rc = bfs_batch_seed_pairs(*b, g, g->stream, slot_of, srcs, npairs))) return rc;

@@ -367,10 +367,9 @@ int mg::drive(mg_graph *g, Step step, int64_t max_steps, int kind, uint64_t key,
             sg.key = key;
         }
         auto finish = [&]() {
-            // kinds whose steps count themselves: the next search starts with this many
-            const bool counts = kind == KIND_BFS || kind == KIND_SSSP;
-            sg.last_steps = counts ? h_ctl->steps : 0;
-            sg.team_step = counts ? h_ctl->team_step : 0;
+            // steps that count themselves: the next search starts with this many
+            sg.last_steps = h_ctl->steps;
+            sg.team_step = h_ctl->team_step;
         };
         int64_t queued = 0, k = 1;
         // exactly `count` steps: full graphs, then one graph of the rest (each graph

@@ -113,3 +113,54 @@ def test_teams_of_several_graphs_at_once(mg, oracle, device):
             assert np.array_equal(b, oracle.bfs(h.row_offsets, h.col_idx, s))
             assert np.array_equal(d, oracle.sssp(h.row_offsets, h.col_idx, h.values, s))
     [g.close() for g in graphs]
+
+
+# ---------------------------------------------------------------- batched BFS by levels
+def _clique_chain(mg, cliques, size, symmetric=True):
+    """A chain of cliques: diameter about `cliques`, mean degree above 8."""
+    src, dst = [], []
+    for c in range(cliques):
+        ids = np.arange(c * size, (c + 1) * size)
+        a, b = np.meshgrid(ids, ids)
+        src.append(a.ravel()), dst.append(b.ravel())
+        if c + 1 < cliques:
+            src.append([ids[-1]]), dst.append([ids[-1] + 1])
+    flags = mg.MG_CSR_DROP_LOOPS | mg.MG_CSR_SORT_COLS | mg.MG_CSR_DEDUPE | (mg.MG_CSR_SYMMETRIZE if symmetric else 0)
+    return mg.csr_from_edges(cliques * size, np.concatenate(src).astype(np.int32), np.concatenate(dst).astype(np.int32),
+                             flags)
+
+
+@pytest.mark.parametrize("cliques", [3, 5, 9, 15, 16, 17, 40])
+@pytest.mark.parametrize("symmetric,k", [(True, 5), (False, 70)])
+def test_batch_levels_at_their_limits(mg, oracle, device, cliques, symmetric, k):
+    # two levels a clique: depths around the 8, 16 and 32 levels kept, and searches too deep for them
+    g = _clique_chain(mg, cliques, 40, symmetric)
+    srcs = np.random.default_rng(k).integers(0, g.n, k).astype(np.int32)
+    srcs[:2] = [0, g.n - 1]
+    exp = np.stack([oracle.bfs(g.row_offsets, g.col_idx, int(s)) for s in srcs])
+    for relabel in (False, True):
+        with mg.Graph(g, symmetric=symmetric, build_csc=not symmetric, relabel=relabel) as dg:
+            for alpha in (0, 1, 1 << 20):  # the default switch, push only, pull early
+                got, st = dg.bfs_batch(srcs, mg.options(batch_alpha=alpha), stats=True)
+                assert np.array_equal(got, exp)
+                assert st.edges_traversed == sum(oracle.teps_edges(g.row_offsets, r) for r in exp)
+                assert st.vertices_reached == int((exp >= 0).sum())
+            limit = 2 + cliques // 3
+            got = dg.bfs_batch(srcs, mg.options(iter_num=limit))
+            assert np.array_equal(got, np.where(exp <= limit, exp, -1))
+
+
+def test_batch_levels_long_in_lists(mg, oracle, device):
+    # hubs on both sides of the pieces a pull cuts long in-lists into
+    rng = np.random.default_rng(5)
+    n, hubs = 12000, [33, 1056, 1057, 2081, 9000]
+    src, dst = [rng.integers(0, n, 6 * n)], [rng.integers(0, n, 6 * n)]
+    for i, d in enumerate(hubs):
+        src.append(np.full(d, i)), dst.append(rng.choice(np.arange(10, n), d, replace=False))
+    g = mg.csr_from_edges(n, np.concatenate(src).astype(np.int32), np.concatenate(dst).astype(np.int32),
+                          mg.MG_CSR_SYMMETRIZE | mg.MG_CSR_DROP_LOOPS | mg.MG_CSR_DEDUPE | mg.MG_CSR_SORT_COLS)
+    srcs = rng.integers(0, n, 256).astype(np.int32)
+    with mg.Graph(g, symmetric=True) as dg:
+        rows = dg.bfs_batch(srcs, mg.options(batch_alpha=1 << 20))
+    for j in range(0, 256, 15):
+        assert np.array_equal(rows[j], oracle.bfs(g.row_offsets, g.col_idx, int(srcs[j])))
