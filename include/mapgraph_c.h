@@ -140,7 +140,8 @@ typedef struct mg_options {
                                single-workgroup levels at 4 x the largest weight and runs the
                                whole-GPU levels unbucketed (dense levels pull); -1 =
                                unbucketed.  Batched searches: the width of every level, 0 =
-                               about 4 x the mean weight, -1 = unbucketed                  */
+                               about 4 x the mean weight (4 x the largest on sparse graphs,
+                               whose rows run side by side), -1 = unbucketed               */
     int32_t ppr_iters;      /* personalized PageRank iterations (0 = 20)                   */
     int32_t sssp_bucket_edges; /* mg_sssp: once the pending vertices of a whole-GPU level
                                have fewer out-edges than this, the bucket bound is lifted

@@ -207,6 +207,12 @@ constexpr int LEVELS_ALPHA = 16;
 int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32_t *srcs, int32_t npairs, int32_t k,
                    int32_t *depth_out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *deep);
 
+// Batched searches by teams (batch_teams.hip), on graphs that teams_wanted() names: sparse
+// ones, until a search there turns out wide (then *wide is set and nothing delivered).
+bool teams_wanted(const mg_graph *g, bool sssp);
+int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
+                int32_t *out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *wide);
+
 // ---- batched personalized PageRank (ppr.hip)
 constexpr int PPR_SLOTS = 64;  // slots per context: one per lane
 

@@ -779,6 +779,10 @@ extern "C" int mg_bfs_batch(mg_graph *g, const int32_t *srcs, int32_t k, int32_t
         return set_error(MG_ERR_UNSUPPORTED, "mg_bfs_batch: directed=0 needs a symmetric graph");
     int32_t rows[MG_BATCH_MAX], tsrc[MG_BATCH_MAX];
     for (int s = 0; s < k; ++s) rows[s] = s;
+    if (teams_wanted(g, false)) {
+        bool wide = false;
+        if ((rc = teams_batch(g, false, rows, srcs, k, k, depth_out, o, stats, timer, &wide)) || !wide) return rc;
+    }
     mg_graph *sg = batch_graph(g, o, srcs, k, tsrc);  // the degree-ordered twin, when the graph keeps one
     if (sg != g && (rc = ensure_workspace(sg))) return rc;
     return bfs_batch_run(sg, rows, sg != g ? tsrc : srcs, k, k, depth_out, o, stats, timer);
@@ -794,6 +798,10 @@ extern "C" int mg_bfs_batch_sets(mg_graph *g, const int32_t *row_of, const int32
     if ((rc = check_batch_sets("mg_bfs_batch_sets", g, row_of, srcs, npairs, k))) return rc;
     if (o.directed == 0 && !(g->flags & MG_GRAPH_SYMMETRIC))
         return set_error(MG_ERR_UNSUPPORTED, "mg_bfs_batch_sets: directed=0 needs a symmetric graph");
+    if (teams_wanted(g, false)) {
+        bool wide = false;
+        if ((rc = teams_batch(g, false, row_of, srcs, npairs, k, depth_out, o, stats, timer, &wide)) || !wide) return rc;
+    }
     std::vector<int32_t> tsrc((size_t)npairs);
     mg_graph *sg = batch_graph(g, o, srcs, npairs, tsrc.data());
     if (sg != g && (rc = ensure_workspace(sg))) return rc;

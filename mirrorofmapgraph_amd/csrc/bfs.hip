@@ -19,7 +19,7 @@
 // when the frontier falls below n / beta.  Depths are unique, so any traversal
 // order yields the reference's labels (bfs.h:241-253: label = iteration + 1 on
 // first visit; bfs.cu:56-143 on the CPU).
-#include "team.h"
+#include "team_search.h"
 
 namespace mg {
 
@@ -32,8 +32,7 @@ struct BfsArgs {
     uint32_t *visited;
     int *hard;
     int G;               // workgroups of the level kernels
-    TeamCtl *team;       // team of the narrow levels (nullptr: not used)
-    uint64_t *team_rec;
+    int team;            // narrow searches pause for a team (bfs_team)
 };
 
 // Visit of edge (v, u) at level L: claim u through the visited bitmap, label it and
@@ -390,119 +389,62 @@ __global__ __launch_bounds__(SMALL_BLK) void bfs_small(BfsArgs a) {
         }
         __syncthreads();
         if (s_go == 1) continue;
-        if (s_go == 2) team_open(a.team);  // the frontier is in its bitmap
-        break;
+        break;  // (for a team: the frontier is in its bitmap)
     }
 }
 
-// Narrow top-down levels by a team (team.h), from the level bfs_small stopped at until
-// the search ends, turns bottom-up or outgrows the team's queues.
-//
-// A wave takes TEAM_PIECE records of one member at a time, a lane per edge: the neighbour
-// id, then its claim (test-and-set of the visited bit) and its offsets together, so a
-// claimed vertex joins the next frontier as records of its edge range and the next level
-// starts at the adjacency.  After the meeting every wave knows all members' counts and
-// finds its pieces by itself.  The frontier bitmaps stay empty: when the team hands a
-// frontier back, the members build its bitmap and counts from the depths, and leave a
-// level that awaits its close.
-// Bound by the chain record -> neighbour -> claim / offsets -> post -> meeting, about 3 us
-// at 1000 vertices a level.  2048^2 grid, 4095 levels: 72.1 -> 13.1 ms (17.6 -> 3.2 us a
-// level); with a lane per record (four edges each) and workgroup-wide queues 20.9 ms; 8
-// workgroups 22 ms; one / four pieces in step 16.6 / 15.6 ms against 15.6 ms.
-__global__ __launch_bounds__(BLK) void bfs_team(BfsArgs a) {
+// Narrow levels by a team (team_search.h), from the level bfs_small stopped at until the
+// search ends, turns bottom-up or outgrows the team's queues.  The frontier bitmaps stay
+// empty meanwhile: when the team hands a frontier back, the members build its bitmap and
+// counts from the depths, and leave a level that awaits its close.
+// 2048^2 grid, 4095 levels: 72.1 -> 13.1 ms (17.6 -> 3.2 us a level).
+__global__ __launch_bounds__(BLK) void bfs_team(BfsArgs a, TeamCtl *team, uint64_t *recs) {
     Ctl *c = a.fa.ctl;
     if (c->done != 2) return;
     const FrontierArgs &fa = a.fa;
-    int rank, size;
-    if (!team_join(a.team, rank, size)) return;
-    const int lane = lane_id(), sub = lane % TEAM_EDGES;
-    const int *off = fa.off[0], *adj = fa.adj[0];
-    const int can_bu = c->can_bu, alpha = c->alpha, limit = c->iter_limit;
-    int L = c->level, it;
+    TeamSeat t{team, recs, 0, 0};
+    if (!team_join(team, TEAM_WGS, t.rank, t.size)) return;
+    const int lane = lane_id();
+    const int can_bu = c->can_bu, alpha = c->alpha, limit = c->iter_limit, L0 = c->level;
     long long mu = c->m_unexplored;
     bool done = false;
     {  // the first meeting: the frontier's records, from its bitmap (which is cleared)
-        uint32_t *fr = fa.bm[L % 3];
-        TeamOut out(a.team_rec, 1, rank);
-        team_words(fr, fa.nwords, rank, size, [&](int i, uint32_t word) {
+        uint32_t *fr = fa.bm[L0 % 3];
+        TeamOut out(t.recs, 1, t.rank);
+        team_words(fr, fa.nwords, t.rank, t.size, [&](int i, uint32_t word) {
             if (word) __hip_atomic_store(&fr[i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             while (wave_ballot(word != 0)) {
                 const bool has = word != 0;
                 const int v = has ? i * 32 + __ffs(word) - 1 : 0;
                 word &= word - 1;
-                out.queue(has, wave_ballot(has), 0, ld_range(off, v));
+                out.queue(has, wave_ballot(has), 0, ld_range(fa.off[0], v));
             }
         });
-        team_post(a.team, 1, rank, out.word(1));
+        team_post(t.ctl, 1, t.rank, out.word(1));
     }
-    for (it = 1;; ++it) {
-        const uint64_t w = team_meet(a.team, it, size);
-        const TeamIn in = team_in(a.team_rec, it, w);
-        // the same decisions in every wave
+    int L = L0, it = 1;
+    team_bfs(t, fa.off[0], fa.adj[0], a.visited, a.depth, L, it, [&](uint64_t w) {
         const bool over = wave_ballot(team_over(w)) != 0;
-        if (it == 1) {
-            if (over) {
-                mu += c->mf_cur;  // level L - 1 is closed a second time
-                break;
-            }
-        } else {  // close level L - 1
-            const int mf = wave_total(team_mf(w));
-            done = !over && (wave_ballot(team_nf(w) != 0) == 0 || L >= limit);
-            if (over || (!done && can_bu && mf > (mu - mf) / alpha)) break;
-            mu -= mf;
-            if (rank == 0) {
-                const int nf = wave_total(team_nf(w));
-                if (lane == 0) trace_level(fa, L - 1, DIR_TD, nf, mf);
-            }
-            if (done) break;
+        if (L == L0) {
+            if (over) mu += c->mf_cur;  // level L0 - 1 is closed a second time
+            return over;
         }
-        TeamOut out(a.team_rec, it + 1, rank);
-        // K pieces in step, each stage's accesses in flight together
-        auto expand = [&](auto kc, int p0) {
-            constexpr int K = decltype(kc)::value;
-            uint64_t rec[K];
-            int u[K];
-            bool on[K];
-            uint32_t old[K];
-            IntPair o[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                on[k] = true;
-                rec[k] = team_fetch(in, p0 + k * size, on[k]);
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                on[k] = on[k] && sub < rec_len(rec[k]);
-                u[k] = adj[rec_beg(rec[k]) + (on[k] ? sub : 0)];
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-                if (on[k])
-                    old[k] = __hip_atomic_fetch_or(&a.visited[u[k] >> 5], 1u << (u[k] & 31), __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-            for (int k = 0; k < K; ++k) o[k] = ld_range(off, u[k]);
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const bool first = on[k] ? !((old[k] >> (u[k] & 31)) & 1u) : false;
-                const uint64_t firsts = wave_ballot(first);
-                if (!firsts) continue;
-                if (first) a.depth[u[k]] = L + 1;
-                out.queue(first, firsts, 0, o[k]);
-            }
-        };
-        int p = rank;
-        for (; p + size < in.pieces; p += 2 * size) expand(std::integral_constant<int, 2>(), p);
-        if (p < in.pieces) expand(std::integral_constant<int, 1>(), p);
-        ++L;
-        team_post(a.team, it + 1, rank, out.word(it + 1));
-    }
-    // it - 1 levels ran; frontier L awaits
-    const bool lead = rank == 0 && lane == 0;
+        // close level L - 1
+        const int mf = wave_total(team_mf(w));
+        done = !over && (wave_ballot(team_nf(w) != 0) == 0 || L >= limit);
+        if (over || (!done && can_bu && mf > (mu - mf) / alpha)) return true;
+        mu -= mf;
+        if (t.rank == 0) {
+            const int nf = wave_total(team_nf(w));
+            if (lane == 0) trace_level(fa, L - 1, DIR_TD, nf, mf);
+        }
+        return done;
+    });
+    const bool lead = t.rank == 0 && lane == 0;
     if (done) {
         if (lead) {
             c->m_unexplored = mu;
-            c->small_levels += it - 1;
+            c->small_levels += L - L0;
             advance_level(c, L - 1, 0, 0);
             c->qvalid = 0;
             c->done = 1;
@@ -511,7 +453,7 @@ __global__ __launch_bounds__(BLK) void bfs_team(BfsArgs a) {
     }
     uint32_t *fr = fa.bm[L % 3];
     long long nf = 0, mf = 0;
-    for (int v0 = rank * WAVE; v0 < fa.n; v0 += size * WAVE) {
+    for (int v0 = t.rank * WAVE; v0 < fa.n; v0 += t.size * WAVE) {
         const int v = v0 + lane;
         const bool in = v < fa.n && ld_dev(&a.depth[v]) == L;
         const uint64_t m = wave_ballot(in);
@@ -525,7 +467,7 @@ __global__ __launch_bounds__(BLK) void bfs_team(BfsArgs a) {
     write_part<BLK>(fa, nf, mf, 0);
     if (lead) {
         c->m_unexplored = mu;
-        c->small_levels += it - 1;
+        c->small_levels += L - L0;
         c->level = L - 1;
         c->pending = 1;
         c->qvalid = 0;
@@ -739,8 +681,8 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
     a.visited = ws.visited;
     a.hard = ws.hard;
     a.G = o.level_grid > 0 ? o.level_grid : level_blocks(g->n, g->m, 64, MAX_GRID);
-    a.team = a.fa.nviews == 1 ? ws.team : nullptr;
-    a.team_rec = ws.team_rec;
+    // (search views serve graphs that are not thin, within a byte budget: no team there)
+    a.team = a.fa.nviews == 1 && !g->arrays_borrowed;
     const long long m_views = g->m * a.fa.nviews;
 
     MG_HIP(hipEventRecord(g->ev0, g->stream));
@@ -759,7 +701,10 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
     bool tail_queued = false;
     auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, -1, ws.vals, 4 * (size_t)g->n); };
     auto team = [&]() -> int {
-        hipLaunchKernelGGL(bfs_team, dim3(TEAM_GRID), dim3(BLK), 0, g->stream, a);
+        const int trc = ensure_team(g);
+        if (trc) return trc;
+        hipLaunchKernelGGL(team_open<>, dim3(1), dim3(2 * TEAM_SIZE), 0, g->stream, ws.team);
+        hipLaunchKernelGGL(bfs_team, dim3(TEAM_GRID), dim3(BLK), 0, g->stream, a, ws.team, ws.team_rec);
         MG_HIP(hipGetLastError());
         return MG_OK;
     };

@@ -104,7 +104,7 @@ struct Workspace {
     uint32_t *bm[3] = {nullptr, nullptr, nullptr};
     ChunkRec *chunks = nullptr;
     LevelPart *part = nullptr;  // 3 * BIG_GRID slots
-    TeamCtl *team = nullptr;  // team of the narrow levels and its record queues (team.h)
+    TeamCtl *team = nullptr;  // team of the narrow levels and its queues (team.h; on first use)
     uint64_t *team_rec = nullptr;
     Ctl *ctl = nullptr;
     Ctl *h_ctl = nullptr;     // pinned host mirror
@@ -215,6 +215,7 @@ int grow_chunk_queue(mg_graph *g);
 // pointers; they are captured again on next use).
 void invalidate_steps(mg_graph *g);
 int ensure_pr_workspace(mg_graph *g);
+int ensure_team(mg_graph *g);
 int alloc_i32(int32_t **p, size_t n);
 int alloc_f32(float **p, size_t n);
 int alloc_chunks(ChunkRec **p, size_t n);
@@ -300,6 +301,7 @@ int graph_view_create(mg_graph *g, mg_graph **out);
 struct GasStateBase;
 struct BatchDev;
 struct PprDev;
+struct TeamsDev;
 int gas_bfs(mg_graph *g, int src, int *out, const mg_options &o, mg_stats *st, const CallTimer &t);
 int gas_sssp(mg_graph *g, int src, int *out, const mg_options &o, mg_stats *st, const CallTimer &t);
 int gas_cc(mg_graph *g, int *out, const mg_options &o, mg_stats *st, const CallTimer &t);
@@ -307,6 +309,8 @@ int gas_pagerank(mg_graph *g, float *out, const mg_options &o, mg_stats *st, con
 void gas_release(mg_graph *g);
 void batch_release(mg_graph *g);
 void ppr_release(mg_graph *g);
+void teams_release(mg_graph *g);
+int64_t teams_dev_size(const TeamsDev *t);
 int64_t batch_dev_size(const BatchDev *b);  // device bytes held by a batch context
 int64_t ppr_dev_size(const PprDev *p);
 // SSSP bucket width for options o on graph g (a huge value when unbucketed).
@@ -319,6 +323,7 @@ struct mg_graph_steps {
     mg::GasStateBase *gas[4] = {nullptr, nullptr, nullptr, nullptr};
     mg::BatchDev *bdev[2] = {nullptr, nullptr};  // batched BFS / SSSP contexts
     mg::PprDev *pdev = nullptr;                  // batched personalized PageRank context
+    mg::TeamsDev *teams = nullptr;               // batched searches by teams
 };
 
 // Queues steps until the device reports `done`.  Steps run from a captured HIP graph

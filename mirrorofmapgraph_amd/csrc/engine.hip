@@ -118,9 +118,7 @@ int ensure_workspace(mg_graph *g) {
         (rc = dalloc(&ws.bm[0], ws.nwords)) || (rc = dalloc(&ws.bm[1], ws.nwords)) ||
         (rc = dalloc(&ws.bm[2], ws.nwords)) || (rc = dalloc(&ws.chunks, ws.chunk_cap)) ||
         (rc = dalloc(&ws.part, 3 * BIG_GRID)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2)) ||
-        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP)) ||
-        // search views serve graphs that are not thin, within a byte budget: no team there
-        (!g->arrays_borrowed && ((rc = dalloc(&ws.team, 1)) || (rc = dalloc(&ws.team_rec, TEAM_RECS))))) {
+        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP))) {
         free_workspace(ws);
         return rc;
     }
@@ -131,6 +129,14 @@ int ensure_workspace(mg_graph *g) {
         return set_error(MG_ERR_OOM, "hipHostMalloc failed: %s", hipGetErrorString(e));
     }
     return MG_OK;
+}
+
+int ensure_team(mg_graph *g) {
+    Workspace &ws = g->ws;
+    if (ws.team) return MG_OK;
+    int rc = 0;
+    if ((rc = dalloc(&ws.team, 1)) || (rc = dalloc(&ws.team_rec, TEAM_RECS))) dfree(ws.team);
+    return rc;
 }
 
 int ensure_pr_workspace(mg_graph *g) {
@@ -544,6 +550,7 @@ int mg_graph_destroy(mg_graph *g) {
         gas_release(g);
         batch_release(g);
         ppr_release(g);
+        teams_release(g);
         for (auto &s : g->steps->sg) {
             if (s.exec) (void)hipGraphExecDestroy(s.exec);
             for (hipGraphExec_t x : s.part)
@@ -593,6 +600,7 @@ int mg_graph_device_bytes(const mg_graph *g, int64_t *bytes) {
         for (const BatchDev *p : g->steps->bdev)
             if (p) b += batch_dev_size(p);
     if (g->steps && g->steps->pdev) b += ppr_dev_size(g->steps->pdev);
+    if (g->steps && g->steps->teams) b += teams_dev_size(g->steps->teams);
     if (g->perm) b += 8LL * g->n;
     if (g->twin) {
         int64_t tb = 0;

@@ -19,7 +19,7 @@
 // kernels per large level.
 #include <climits>
 
-#include "team.h"
+#include "team_search.h"
 
 namespace mg {
 
@@ -44,8 +44,7 @@ struct SsspArgs {
     int bucketed;
     long long bucket_edges;
     int wmin;  // smallest edge weight (>= 0)
-    TeamCtl *team;  // team of the narrow levels (nullptr: not used)
-    uint64_t *team_rec;
+    int team;  // narrow searches pause for a team (sssp_team)
 };
 
 constexpr long long UNBUCKETED = LLONG_MAX / 4;  // a bucket bound no distance reaches
@@ -980,7 +979,6 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
         }
         __syncthreads();
         const bool to_team = s_go == 2;  // (the far bitmap is the team's far list)
-        if (to_team) team_open(a.team);
         long long nf_far = 0, mf_far = 0, mf_q = 0;
         if (nf > SMALL_Q)  // out-edges of the queued part (build() skipped)
             for (int i = threadIdx.x; i < SMALL_Q; i += SMALL_BLK) mf_q += view_degree(fa, s_q[i]);
@@ -1015,43 +1013,43 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
     }
 }
 
-// Narrow levels by a team (team.h), from the level sssp_small stopped at until the search
-// ends or outgrows the team's queues, with sssp_small's buckets.
-//
-// A wave takes TEAM_PIECE records of one member at a time, a lane per edge: neighbour and
-// weight with the vertex's distance, then the neighbour's distance and offsets, then for
-// a candidate the minimum and the claim together (a stale, larger distance only causes a
-// redundant relaxation).  Claims are test-and-sets: below the bucket bound in the next
-// level's frontier bitmap (the winner queues the vertex), else in the far bitmap, which
-// is the whole far list.  Whoever takes a vertex clears its frontier bit, so the bitmaps
-// rotate clean and always hold the frontier.  When no record is left the members move the
-// bound and sweep the far bitmap (n bits: about 1 us at 1M vertices, once per bucket).
-// Bound by the same chain as bfs_team with a distance load before the claim.  Grid
-// 1049 x 999, weights 1..16, about 2400 rounds: 38.0 -> 8.9 ms; 2048^2 127 -> 27 ms.
-__global__ __launch_bounds__(BLK) void sssp_team(SsspArgs a) {
+// Narrow levels by a team (team_search.h), from the level sssp_small stopped at until the
+// search ends or outgrows the team's queues, with sssp_small's buckets; the far bitmap is
+// the team's far list.  Grid 1049 x 999, weights 1..16, about 2400 rounds: 38.0 -> 8.9 ms;
+// 2048^2: 127 -> 27 ms.
+__global__ __launch_bounds__(BLK) void sssp_team(SsspArgs a, TeamCtl *team, uint64_t *recs) {
     Ctl *c = a.fa.ctl;
     if (c->done != 2) return;
     const FrontierArgs &fa = a.fa;
-    int rank, size;
-    if (!team_join(a.team, rank, size)) return;
-    const int lane = lane_id(), sub = lane % TEAM_EDGES;
-    const int *off = fa.off[0], *adj = fa.adj[0], *wts = a.w;
-    const int can_pull = c->can_bu, alpha = c->alpha, limit = c->iter_limit;
-    const long long m = c->m_unexplored, delta = a.delta;
-    long long thr = c->thr, ex = 0;
-    const int L0 = c->level;
-    int L = L0, it;
-    bool done = false, swept = false;  // swept: this meeting's records come from the far bitmap
+    TeamSeat t{team, recs, 0, 0};
+    if (!team_join(team, TEAM_WGS, t.rank, t.size)) return;
+    const int lane = lane_id();
+    const int can_pull = c->can_bu, alpha = c->alpha, L0 = c->level;
+    const long long m = c->m_unexplored;
+    TeamSssp s;
+    s.off = fa.off[0];
+    s.adj = fa.adj[0];
+    s.w = a.w;
+    s.dist = a.dist;
+    s.bm0 = fa.bm[0];
+    s.bm1 = fa.bm[1];
+    s.bm2 = fa.bm[2];
+    s.farbm = a.farbm;
+    s.nwords = fa.nwords;
+    s.limit = c->iter_limit;
+    s.delta = a.delta;
+    s.thr = c->thr;
+    s.unbucketed = UNBUCKETED;
     {  // the first meeting: the frontier's records, from its bitmap
-        uint32_t *fr = fa.bm[L % 3];
-        TeamOut out(a.team_rec, 1, rank);
-        team_words(fr, fa.nwords, rank, size, [&](int i, uint32_t word) {
+        uint32_t *fr = fa.bm[L0 % 3];
+        TeamOut out(t.recs, 1, t.rank);
+        team_words(fr, fa.nwords, t.rank, t.size, [&](int i, uint32_t word) {
             uint32_t todo = word, keep = 0;
             while (wave_ballot(todo != 0)) {
                 const bool has = todo != 0;
                 const int b = has ? __ffs(todo) - 1 : 0, v = has ? i * 32 + b : 0;
                 todo &= todo - 1;
-                const IntPair o = ld_range(off, v);
+                const IntPair o = ld_range(s.off, v);
                 const bool edges = has && o.b > o.a;  // one without has no record to clear its bit
                 if (edges) keep |= 1u << b;
                 const uint64_t takes = wave_ballot(edges);
@@ -1059,139 +1057,20 @@ __global__ __launch_bounds__(BLK) void sssp_team(SsspArgs a) {
             }
             if (keep != word) __hip_atomic_store(&fr[i], keep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         });
-        team_post(a.team, 1, rank, out.word(1));
+        team_post(t.ctl, 1, t.rank, out.word(1));
     }
-    for (it = 1;; ++it) {
-        const uint64_t w = team_meet(a.team, it, size);
-        const TeamIn in = team_in(a.team_rec, it, w);
-        long long sweep_from = -1;  // >= 0: sweep, dropping waiting distances below this
-        // the same decisions in every wave
-        if (wave_ballot(team_over(w)) != 0) break;
-        const int mf = wave_total(team_mf(w));
-        if (it > 1 && !swept && rank == 0) {  // close level L - 1
-            const int nf = wave_total(team_nf(w));
+    int L = L0, it = 1;
+    const bool done = team_sssp(
+        t, s, L, it,
+        [&](uint64_t w) {  // close level L - 1
+            if (L == L0 || t.rank != 0) return;
+            const int nf = wave_total(team_nf(w)), mf = wave_total(team_mf(w));
             if (lane == 0) trace_level(fa, L - 1, DIR_PUSH, nf, mf);
-        }
-        if (L >= limit) {
-            done = true;
-        } else if (in.pieces > 0) {
-            if (can_pull && (long long)mf * alpha > m) break;
-        } else if (thr >= UNBUCKETED) {
-            done = true;
-        } else if (!swept) {
-            sweep_from = thr;
-            thr += delta;
-        } else {
-            // nothing waits in that bucket: the one of the smallest waiting distance
-            int lo = lane < size ? ld_dev(&a.team->least[it & 1][lane]) : INT_MAX;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) lo = min(lo, __shfl_xor(lo, o));
-            if (lo == INT_MAX) {
-                done = true;
-            } else {
-                sweep_from = thr;
-                thr = ((long long)lo / delta + 1) * delta;
-            }
-        }
-        if (done) break;
-        TeamOut out(a.team_rec, it + 1, rank);
-        swept = sweep_from >= 0;
-        if (swept) {
-            // far vertices below the bound join frontier L (its bitmap is clear); those
-            // below the old bound were relaxed since and leave the far bitmap
-            uint32_t *fr = fa.bm[L % 3];
-            int least = INT_MAX;
-            team_words(a.farbm, fa.nwords, rank, size, [&](int i, uint32_t word) {
-                uint32_t todo = word, keep = 0, go = 0;
-                while (wave_ballot(todo != 0)) {
-                    const bool has = todo != 0;
-                    const int b = has ? __ffs(todo) - 1 : 0, u = has ? i * 32 + b : 0;
-                    todo &= todo - 1;
-                    const int d = ld_dev(&a.dist[u]);
-                    const IntPair o = ld_range(off, u);
-                    const bool take = has && d >= sweep_from && d < thr && o.b > o.a;
-                    if (has && d >= thr) {
-                        keep |= 1u << b;
-                        least = min(least, d);
-                    }
-                    if (take) go |= 1u << b;
-                    const uint64_t takes = wave_ballot(take);
-                    if (takes) out.queue(take, takes, u, o);
-                }
-                if (keep != word) __hip_atomic_store(&a.farbm[i], keep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (go) __hip_atomic_store(&fr[i], go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            });
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) least = min(least, __shfl_xor(least, o));
-            if (lane == 0)
-                __hip_atomic_store(&a.team->least[(it + 1) & 1][rank], least, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            team_post(a.team, it + 1, rank, out.word(it + 1));
-            continue;
-        }
-        uint32_t *fr = fa.bm[L % 3], *nx = fa.bm[(L + 1) % 3];
-        auto relax = [&](auto kc, int p0) {
-            constexpr int K = decltype(kc)::value;
-            uint64_t rec[K];
-            int u[K], wt[K], dv[K], du[K];
-            bool on[K];
-            IntPair o[K];
-            uint32_t old[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                on[k] = true;
-                rec[k] = team_fetch(in, p0 + k * size, on[k]);
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                on[k] = on[k] && sub < rec_len(rec[k]);
-                const int e = rec_beg(rec[k]) + (on[k] ? sub : 0);
-                u[k] = adj[e];
-                wt[k] = wts[e];
-                dv[k] = ld_dev(&a.dist[rec_vertex(rec[k])]);
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                du[k] = ld_dev(&a.dist[u[k]]);
-                o[k] = ld_range(off, u[k]);
-                if (on[k] && sub == 0)
-                    __hip_atomic_store(&fr[rec_vertex(rec[k]) >> 5], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            bool cand[K], near[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const long long nd = (long long)dv[k] + wt[k];
-                ex += on[k];
-                cand[k] = on[k] && nd < du[k];
-                near[k] = nd < thr;
-                if (cand[k]) {
-                    __hip_atomic_fetch_min(&a.dist[u[k]], (int)nd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    old[k] = __hip_atomic_fetch_or(&(near[k] ? nx : a.farbm)[u[k] >> 5], 1u << (u[k] & 31),
-                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                bool first = cand[k] && near[k] ? !((old[k] >> (u[k] & 31)) & 1u) : false;
-                // a vertex without out-edges has no record to clear its bit
-                if (first && o[k].a == o[k].b) {
-                    __hip_atomic_fetch_and(&nx[u[k] >> 5], ~(1u << (u[k] & 31)), __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-                    first = false;
-                }
-                const uint64_t firsts = wave_ballot(first);
-                if (firsts) out.queue(first, firsts, u[k], o[k]);
-            }
-        };
-        int p = rank;
-        for (; p + size < in.pieces; p += 2 * size) relax(std::integral_constant<int, 2>(), p);
-        if (p < in.pieces) relax(std::integral_constant<int, 1>(), p);
-        ++L;
-        team_post(a.team, it + 1, rank, out.word(it + 1));
-    }
-    const bool lead = rank == 0 && lane == 0;
+        },
+        [&](uint64_t w) { return can_pull && (long long)wave_total(team_mf(w)) * alpha > m; });
+    const bool lead = t.rank == 0 && lane == 0;
     if (done) {
-        ex = wave_sum_ll(ex);
+        const long long ex = wave_sum_ll(s.ex);
         if (lane == 0) atomicAdd((unsigned long long *)&c->edges_examined, (unsigned long long)ex);
         if (lead) {
             c->small_levels += L - L0;
@@ -1205,7 +1084,7 @@ __global__ __launch_bounds__(BLK) void sssp_team(SsspArgs a) {
     // level that awaits its close
     uint32_t *fr = fa.bm[L % 3];
     long long nf = 0, mf = 0, mn = LLONG_MAX;
-    for (int i = rank * WAVE + lane; i < fa.nwords; i += size * WAVE) {
+    for (int i = t.rank * WAVE + lane; i < fa.nwords; i += t.size * WAVE) {
         const uint32_t f = (uint32_t)ld_dev((const int *)a.farbm + i);
         uint32_t word = (uint32_t)ld_dev((const int *)fr + i) | f;
         if (!word) continue;
@@ -1222,11 +1101,11 @@ __global__ __launch_bounds__(BLK) void sssp_team(SsspArgs a) {
             mf += view_degree(fa, v);
         }
     }
-    write_part<BLK>(fa, nf, mf, ex, mn);
+    write_part<BLK>(fa, nf, mf, s.ex, mn);
     if (lead) {
         c->small_levels += L - L0;
         c->level = L - 1;
-        c->thr = thr;
+        c->thr = s.thr;
         c->pending = 1;
         c->qvalid = 0;
         c->done = 0;
@@ -1319,8 +1198,8 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     a.far = ws.hard;
     a.farbm = ws.visited;
     a.wmin = g->min_weight;
-    a.team = a.fa.nviews == 1 ? ws.team : nullptr;
-    a.team_rec = ws.team_rec;
+    // (search views serve graphs that are not thin, within a byte budget: no team there)
+    a.team = a.fa.nviews == 1 && !g->arrays_borrowed;
     const int in_view = a.fa.off[2] != nullptr && a.fa.nviews == 1 && o.engine != MG_ENGINE_GAS;
     // pull levels relax every vertex from all its in-edges: unbucketed searches only
     const int can_pull = in_view && !a.bucketed;
@@ -1355,7 +1234,10 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     bool tail_queued = false;
     auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, INT_MAX, ws.vals, 4 * (size_t)g->n); };
     auto team = [&]() -> int {
-        hipLaunchKernelGGL(sssp_team, dim3(TEAM_GRID), dim3(BLK), 0, g->stream, a);
+        const int trc = ensure_team(g);
+        if (trc) return trc;
+        hipLaunchKernelGGL(team_open<>, dim3(1), dim3(2 * TEAM_SIZE), 0, g->stream, ws.team);
+        hipLaunchKernelGGL(sssp_team, dim3(TEAM_GRID), dim3(BLK), 0, g->stream, a, ws.team, ws.team_rec);
         MG_HIP(hipGetLastError());
         return MG_OK;
     };

@@ -75,34 +75,35 @@ struct TeamCtl {
 // The XCD this wave runs on (hardware register XCC_ID).
 __device__ __forceinline__ int xcd_id() { return (int)__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15; }
 
-// Whole workgroup (at least 2 * TEAM_SIZE threads), before the launch that forms the
-// team: nobody has joined, nothing is posted (meetings are numbered from 1).
-__device__ __forceinline__ void team_open(TeamCtl *t) {
+// Before the launch that forms the team (one workgroup of at least 2 * TEAM_SIZE threads):
+// nobody has joined, nothing is posted (meetings are numbered from 1).
+template <int = 0>
+__global__ void team_open(TeamCtl *t) {
     if (threadIdx.x < 2 * TEAM_SIZE) (&t->word[0][0])[threadIdx.x] = 0;
     if (threadIdx.x == 0) t->leader = t->joined = t->size = 0;
 }
 
-// Whole workgroup: joins the team.  False for workgroups that take no part; else this
+// Whole workgroup: joins the team of up to `wgs` (<= TEAM_WGS) workgroups.  False for workgroups that take no part; else this
 // wave's number among the team's `size` waves (a workgroup's waves lie `size` /
 // (BLK / WAVE) apart, so the first few members are on different CUs).
-__device__ __forceinline__ bool team_join(TeamCtl *t, int &rank, int &size) {
+__device__ __forceinline__ bool team_join(TeamCtl *t, int wgs, int &rank, int &size) {
     __shared__ int s_rank, s_size;
     if (threadIdx.x == 0) {
         const int x = xcd_id() + 1;
-        int r = TEAM_WGS, n = 0;
+        int r = wgs, n = 0;
         int lead = ld_dev(&t->leader);
         if (lead == 0) {
             lead = atomicCAS(&t->leader, 0, x);
             if (lead == 0) lead = x;
         }
         // (the load spares late workgroups the atomic)
-        if (lead == x && ld_dev(&t->joined) < TEAM_WGS) r = atomicAdd(&t->joined, 1);
+        if (lead == x && ld_dev(&t->joined) < wgs) r = atomicAdd(&t->joined, 1);
         if (r == 0) {
             const long long t0 = wall_clock64();
-            while (ld_dev(&t->joined) < TEAM_WGS && wall_clock64() - t0 < TEAM_GATHER) __builtin_amdgcn_s_sleep(1);
-            n = min(atomicOr(&t->joined, TEAM_CLOSED), TEAM_WGS);
+            while (ld_dev(&t->joined) < wgs && wall_clock64() - t0 < TEAM_GATHER) __builtin_amdgcn_s_sleep(1);
+            n = min(atomicOr(&t->joined, TEAM_CLOSED), wgs);
             __hip_atomic_store(&t->size, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else if (r < TEAM_WGS) {
+        } else if (r < wgs) {
             // joined before the team closed: the first member is running and will close it
             while ((n = ld_dev(&t->size)) == 0) __builtin_amdgcn_s_sleep(1);
         }
@@ -203,6 +204,13 @@ __device__ __forceinline__ uint64_t team_fetch(const TeamIn &t, int p, bool &on)
     return __hip_atomic_load(&t.recs[(size_t)s * TEAM_SEG + min(r, have - 1)], __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// A wave's place in a team.
+struct TeamSeat {
+    TeamCtl *ctl;
+    uint64_t *recs;  // TEAM_RECS records
+    int rank, size;
+};
 
 // A member's part of the next frontier.
 struct TeamOut {

@@ -164,3 +164,54 @@ def test_batch_levels_long_in_lists(mg, oracle, device):
         rows = dg.bfs_batch(srcs, mg.options(batch_alpha=1 << 20))
     for j in range(0, 256, 15):
         assert np.array_equal(rows[j], oracle.bfs(g.row_offsets, g.col_idx, int(srcs[j])))
+
+
+# ---------------------------------------------------------------- batched searches by teams
+@pytest.mark.parametrize("which", ["path", "directed", "zero", (33, 31), (260, 19), "random"])
+@pytest.mark.parametrize("k", [1, 9, 256])
+def test_batch_teams_match_the_oracle(mg, oracle, device, which, k):
+    # sparse graphs; "random" outgrows the teams' queues and falls back to the shared batch
+    if which == "random":
+        g, sym = random_graph(mg, 120000, 350000, 3, wmax=20), True
+    elif which == "path":
+        g, sym = _chain(mg, [300], [0], 3), True
+    else:
+        g, sym = _team_graph(mg, which)
+    assert g.m < 8 * g.n
+    rng = np.random.default_rng(k)
+    srcs = rng.integers(0, g.n, k).astype(np.int32)
+    pick = sorted({0, k // 2, k - 1})
+    for relabel in (False, True):
+        with mg.Graph(g, symmetric=sym, relabel=relabel) as dg:
+            for _ in range(2):
+                rows, st = dg.bfs_batch(srcs, stats=True)
+                assert st.vertices_reached == int((rows >= 0).sum())
+                assert st.edges_traversed == sum(oracle.teps_edges(g.row_offsets, r) for r in rows)
+                srows = dg.sssp_batch(srcs)
+                for j in pick:
+                    assert np.array_equal(rows[j], oracle.bfs(g.row_offsets, g.col_idx, int(srcs[j])))
+                    exp = oracle.sssp(g.row_offsets, g.col_idx, g.values, int(srcs[j]))
+                    assert np.array_equal(srows[j], exp)
+            for delta in (1, 5, -1):
+                assert np.array_equal(dg.sssp_batch(srcs[:3], mg.options(sssp_delta=delta)), srows[:3])
+            # stopped short, then whole again: the teams' bitmaps are clean
+            cut = dg.bfs_batch(srcs, mg.options(iter_num=3))
+            assert np.array_equal(cut, np.where(rows <= 3, rows, -1))
+            dg.sssp_batch(srcs, mg.options(iter_num=3))
+            assert np.array_equal(dg.bfs_batch(srcs), rows) and np.array_equal(dg.sssp_batch(srcs), srows)
+
+
+def test_batch_teams_source_sets(mg, oracle, device):
+    g = mg.grid_graph(70, 45, seed=3, weight_max=9)
+    rng = np.random.default_rng(2)
+    row_of = np.concatenate([np.arange(5), rng.integers(0, 5, 200)]).astype(np.int32)
+    srcs = rng.integers(0, g.n, 205).astype(np.int32)
+    srcs[7] = srcs[8] = srcs[row_of.tolist().index(row_of[7])]  # repeated sources
+    with mg.Graph(g, symmetric=True) as dg:
+        rows, srows = dg.bfs_batch_sets(row_of, srcs, 5), dg.sssp_batch_sets(row_of, srcs, 5)
+    for r in range(5):
+        mine = [int(s) for s in srcs[row_of == r]]
+        b = np.stack([oracle.bfs(g.row_offsets, g.col_idx, s) for s in mine]).astype(np.int64)
+        assert np.array_equal(rows[r], np.where((b < 0).all(0), -1, np.where(b < 0, 1 << 40, b).min(0)))
+        d = np.stack([oracle.sssp(g.row_offsets, g.col_idx, g.values, s) for s in mine])
+        assert np.array_equal(srows[r], d.min(0))
