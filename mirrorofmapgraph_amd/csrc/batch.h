@@ -213,6 +213,13 @@ bool teams_wanted(const mg_graph *g, bool sssp);
 int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
                 int32_t *out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *wide);
 
+// Batched SSSP by pulling (batch_pull.hip), on graphs that pull_wanted() names: mean degree 8
+// and more with an in-edge view, until a search there takes too many rounds (then *deep is
+// set and nothing delivered).
+bool pull_wanted(const mg_graph *g);
+int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k, int32_t *out,
+               const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *deep);
+
 // ---- batched personalized PageRank (ppr.hip)
 constexpr int PPR_SLOTS = 64;  // slots per context: one per lane
 

@@ -646,6 +646,10 @@ static int sssp_batch_checks(const char *fn, const mg_graph *g, const mg_options
 static int sssp_batch_run(mg_graph *g, const int32_t *slot_of, const int32_t *srcs, int32_t npairs, int32_t k,
                           int32_t *dist_out, const mg_options &o, mg_stats *stats, const CallTimer &timer) {
     int rc;
+    if (pull_wanted(g)) {
+        bool deep = false;
+        if ((rc = pull_batch(g, slot_of, srcs, npairs, k, dist_out, o, stats, timer, &deep)) || !deep) return rc;
+    }
     BatchDev *b = nullptr;
     if ((rc = graph_batch_dev(g, true, &b))) return rc;
     const long long delta = sssp_delta(g, o);

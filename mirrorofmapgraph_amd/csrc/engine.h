@@ -302,6 +302,7 @@ struct GasStateBase;
 struct BatchDev;
 struct PprDev;
 struct TeamsDev;
+struct PullDev;
 int gas_bfs(mg_graph *g, int src, int *out, const mg_options &o, mg_stats *st, const CallTimer &t);
 int gas_sssp(mg_graph *g, int src, int *out, const mg_options &o, mg_stats *st, const CallTimer &t);
 int gas_cc(mg_graph *g, int *out, const mg_options &o, mg_stats *st, const CallTimer &t);
@@ -311,6 +312,8 @@ void batch_release(mg_graph *g);
 void ppr_release(mg_graph *g);
 void teams_release(mg_graph *g);
 int64_t teams_dev_size(const TeamsDev *t);
+void pull_release(mg_graph *g);
+int64_t pull_dev_size(const PullDev *p);
 int64_t batch_dev_size(const BatchDev *b);  // device bytes held by a batch context
 int64_t ppr_dev_size(const PprDev *p);
 // SSSP bucket width for options o on graph g (a huge value when unbucketed).
@@ -324,6 +327,7 @@ struct mg_graph_steps {
     mg::BatchDev *bdev[2] = {nullptr, nullptr};  // batched BFS / SSSP contexts
     mg::PprDev *pdev = nullptr;                  // batched personalized PageRank context
     mg::TeamsDev *teams = nullptr;               // batched searches by teams
+    mg::PullDev *pull = nullptr;                 // batched SSSP by pulling
 };
 
 // Queues steps until the device reports `done`.  Steps run from a captured HIP graph

@@ -551,6 +551,7 @@ int mg_graph_destroy(mg_graph *g) {
         batch_release(g);
         ppr_release(g);
         teams_release(g);
+        pull_release(g);
         for (auto &s : g->steps->sg) {
             if (s.exec) (void)hipGraphExecDestroy(s.exec);
             for (hipGraphExec_t x : s.part)
@@ -601,6 +602,7 @@ int mg_graph_device_bytes(const mg_graph *g, int64_t *bytes) {
             if (p) b += batch_dev_size(p);
     if (g->steps && g->steps->pdev) b += ppr_dev_size(g->steps->pdev);
     if (g->steps && g->steps->teams) b += teams_dev_size(g->steps->teams);
+    if (g->steps && g->steps->pull) b += pull_dev_size(g->steps->pull);
     if (g->perm) b += 8LL * g->n;
     if (g->twin) {
         int64_t tb = 0;

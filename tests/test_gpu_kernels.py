@@ -215,3 +215,54 @@ def test_batch_teams_source_sets(mg, oracle, device):
         assert np.array_equal(rows[r], np.where((b < 0).all(0), -1, np.where(b < 0, 1 << 40, b).min(0)))
         d = np.stack([oracle.sssp(g.row_offsets, g.col_idx, g.values, s) for s in mine])
         assert np.array_equal(srows[r], d.min(0))
+
+
+# ---------------------------------------------------------------- batched SSSP by pulling
+@pytest.mark.parametrize("k", [1, 3, 32, 33, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_batch_pull_row_widths(mg, oracle, device, k, symmetric):
+    # row widths around every group size; hubs around the piece length; a small component
+    rng = np.random.default_rng(k)
+    n, hubs = 3000, [511, 512, 513, 1024, 1025, 2500]
+    src, dst = [rng.integers(0, n - 20, 8 * n)], [rng.integers(0, n - 20, 8 * n)]
+    for i, d in enumerate(hubs):
+        a, b = np.full(d, i), rng.choice(np.arange(10, n - 20), d, replace=False)
+        src += [a, b]
+        dst += [b, a]
+    src.append(np.arange(n - 10, n - 1)), dst.append(np.arange(n - 9, n))
+    flags = mg.MG_CSR_DROP_LOOPS | mg.MG_CSR_DEDUPE | mg.MG_CSR_SORT_COLS | (mg.MG_CSR_SYMMETRIZE if symmetric else 0)
+    g = mg.csr_from_edges(n, np.concatenate(src).astype(np.int32), np.concatenate(dst).astype(np.int32), flags)
+    g.values = mg.hash_weights(g, k, 50) - 1
+    assert g.m >= 8 * g.n
+    srcs = rng.integers(0, n, k).astype(np.int32)
+    srcs[0] = n - 10  # in the small component
+    exp = np.stack([oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)) for s in srcs])
+    for relabel in (False, True):
+        with mg.Graph(g, symmetric=symmetric, build_csc=not symmetric, relabel=relabel) as dg:
+            for _ in range(2):
+                got, st = dg.sssp_batch(srcs, stats=True)
+                assert np.array_equal(got, exp)
+            assert st.vertices_reached == int((exp != 2**31 - 1).sum())
+            assert st.edges_traversed == sum(oracle.teps_edges(g.row_offsets, r, 2**31 - 1) for r in exp)
+            assert np.array_equal(dg.sssp_batch(srcs[:1])[0], exp[0])  # another width on the same state
+
+
+@pytest.mark.parametrize("cliques", [20, 47, 48, 60])
+def test_batch_pull_falls_back_when_deep(mg, oracle, device, cliques):
+    g = _clique_chain(mg, cliques, 20)
+    g.values = mg.hash_weights(g, 2, 30)
+    srcs = np.array([0, g.n // 2, g.n - 1], np.int32)
+    with mg.Graph(g, symmetric=True) as dg:
+        for _ in range(2):
+            for got, s in zip(dg.sssp_batch(srcs), srcs):
+                assert np.array_equal(got, oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)))
+
+
+def test_batch_pull_huge_weights(mg, oracle, device):
+    # distances at the top of the 32-bit range: sums past INT_MAX never improve anything
+    g = random_graph(mg, 400, 3000, 3, wmax=7)
+    g.values = (g.values * 150_000_000).astype(np.int32)
+    srcs = np.arange(5, dtype=np.int32)
+    with mg.Graph(g, symmetric=True) as dg:
+        for got, s in zip(dg.sssp_batch(srcs), srcs):
+            assert np.array_equal(got, dg.sssp(int(s)))
