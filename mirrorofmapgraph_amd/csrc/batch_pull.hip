@@ -140,12 +140,6 @@ struct PullLds {
     int off[WAVE + 1], top[WAVE], low[WAVE];
 };
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // cur becomes the minimum of itself and the rows of the kept edges [p, end) plus weight;
 // four rows a step (every lane of the wave calls it, each group with its own range).
 template <int LANES>

@@ -113,16 +113,16 @@ struct Workspace {
     // PageRank state (allocated on first use)
     float *rank = nullptr;
     float *contrib[2] = {nullptr, nullptr};
-    double *partials = nullptr;                       // per-workgroup L1 partial sums
-    int32_t *pr_mid = nullptr;                        // vertices of medium in-degree (a wave each)
-    ChunkRec *pr_chunks = nullptr;                    // in-edge chunks of high in-degree vertices
-    double *pr_partials = nullptr;                    // per-workgroup partials of the PageRank gather
-    LevelPart *pr_cpart = nullptr;
-    int pr_nslots = 0;
+    double *partials = nullptr;                       // per-workgroup L1 change and changed vertices
+    ChunkRec *pr_lists = nullptr;                     // in-edge chunks of high in-degree vertices, medium lists
     int32_t *pr_bigv = nullptr;                       // first chunk of each high in-degree vertex (+ end)
     float *pr_part = nullptr;                         // per-chunk partial sums
     int32_t *pr_pact = nullptr;                       // per-chunk "an in-neighbour changed" flags
-    int pr_nmid = 0, pr_nchunks = 0, pr_nbig = 0;
+    int32_t *pr_left = nullptr;                       // per high in-degree vertex: chunks summed
+    ChunkRec *pr_runs = nullptr;                      // runs of vertices of low in-degree
+    int pr_nruns = 0;
+    bool pr_hubs = false;                             // many edges come from the lowest ids
+    int pr_nlists = 0, pr_nbig = 0;
     const int32_t *pr_view = nullptr;                 // in-edge offsets the buckets were built for
     // Static pull tasks: PULL_TASK-edge pieces of the in-edge lists longer than LANE_T
     ChunkRec *pull_tasks = nullptr;
@@ -219,7 +219,6 @@ int ensure_team(mg_graph *g);
 int alloc_i32(int32_t **p, size_t n);
 int alloc_f32(float **p, size_t n);
 int alloc_chunks(ChunkRec **p, size_t n);
-int alloc_f64(double **p, size_t n);
 int alloc_parts(LevelPart **p, size_t n);
 void free_dev(void *p);
 int grid_blocks(int64_t work_items, int block);

@@ -89,10 +89,9 @@ static void free_workspace(Workspace &ws) {
     dfree(ws.contrib[0]);
     dfree(ws.contrib[1]);
     dfree(ws.partials);
-    dfree(ws.pr_mid);
-    dfree(ws.pr_chunks);
-    dfree(ws.pr_partials);
-    dfree(ws.pr_cpart);
+    dfree(ws.pr_lists);
+    dfree(ws.pr_left);
+    dfree(ws.pr_runs);
     dfree(ws.pr_part);
     dfree(ws.pr_pact);
     dfree(ws.pr_bigv);
@@ -201,7 +200,6 @@ int grow_chunk_queue(mg_graph *g) {
 int alloc_i32(int32_t **p, size_t n) { return dalloc(p, n); }
 int alloc_f32(float **p, size_t n) { return dalloc(p, n); }
 int alloc_chunks(ChunkRec **p, size_t n) { return dalloc(p, n); }
-int alloc_f64(double **p, size_t n) { return dalloc(p, n); }
 int alloc_parts(LevelPart **p, size_t n) { return dalloc(p, n); }
 void free_dev(void *p) {
     if (p) (void)hipFree(p);

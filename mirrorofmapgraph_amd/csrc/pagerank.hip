@@ -16,22 +16,55 @@
 // pass per iteration reads each in-edge once, sums precomputed contributions
 // contrib[u] = rank[u] / (float)outdeg[u] (the same float division as gather_edge),
 // and applies.  Summation order is fixed, so results are deterministic:
-//   in-degree <= PR_T1   one lane, sequentially in in-edge order;
-//   <= PR_T2             one wave: lane l sums edges l, l+64, ... in order, then an
+//   in-degree <= PR_T1   one lane, sequentially in in-edge order (the wave gathers the
+//                        edges of a run of such vertices together, into LDS);
+//   up to a piece        one wave: lane l sums edges l, l+64, ... in order, then an
 //                        xor-butterfly over offsets 32,16,8,4,2,1;
-//   >  PR_T2             chunks of PR_T2 edges summed as above, then the chunk
-//                        sums added in chunk order.
+//   longer               pieces summed as above, then their sums added in order.
 // MG_PR_ALL updates every vertex each iteration (all-vertex Jacobi) and can stop on
 // the L1 change, reduced in a fixed order as well.
+//
+// An iteration is one launch: the wave that finishes a high in-degree vertex's last chunk
+// adds its chunk sums, and the workgroup that finishes last closes the iteration
+// (counters in device memory, what they guard stored and loaded device-coherently).
+//
+// Bound: the gathers contrib[u], an L2 request for each distinct line of a wave's 64.  On
+// graphs whose hubs have the lowest ids (the degree-ordered twin; R-MAT as generated) every
+// workgroup copies the first PR_HUBS contributions into LDS, and a gather below PR_HUBS is
+// an LDS read: 50% of the edges of the directed R-MAT scale 21 (33.5M edges), 57% at scale
+// 20.  60 KB let two workgroups share a CU: 32768 contributions in 128 KB, one workgroup a
+// CU, took 136 us an iteration where 16384 and two took 130.  Gathering a low in-degree
+// vertex in a lane of its own made 64 lanes read 64 lists; a wave that gathers a run of them
+// in edge order reads adjacency lines once (130 -> 115).
+// Measured, us an iteration, directed R-MAT, edge factor 16, degree-ordered (as generated):
+//   scale 16   28 -> 15 (28 -> 14)
+//   scale 19   57 -> 33 (79 -> 45)
+//   scale 21   158 -> 112 (233 -> 179)
+// of which at scale 21 7.5 are the launch, the copy and the close, 55 with the adjacency read
+// and the sums made but no contribution loaded.  Without LDS hubs 147.
 #include <vector>
 
 #include "frontier.h"
 
 namespace mg {
 
-constexpr int PR_T1 = 64;
-constexpr int PR_T2 = 1024;
-constexpr int PR_MAX_GRID = 32768;  // workgroups of pr_k1 / pr_k2
+// In-degrees a lane sums alone: 32, 48, 64 and 128 took 129, 115, 115 and 120 us at scale 21,
+// 48 and 64 39 and 42 at scale 19.
+constexpr int PR_T1 = 48;
+constexpr int PR_BLK = 1024;        // threads of pr_iterate
+constexpr int PR_HUBS = 15360;      // contributions kept in LDS: 60 KB, two workgroups a CU
+constexpr int PR_BUF = 256;         // edges of a run in LDS at a time (per wave)
+// A wave's piece of work (a run of low in-degree vertices, or a part of a list) has
+// m / PR_PIECES edges, so that small graphs have pieces for all 8192 waves and large ones few
+// records: at 1024 edges whatever the size scales 16 and 19 took 20 and 34 us, now 15 and 33;
+// least pieces of 128 took 17 at scale 16.
+constexpr int PR_PIECES = 16384;
+constexpr int PR_PIECE_MIN = 256, PR_PIECE_MAX = 2048;
+constexpr int PR_GROUPS = 32;       // counters of finished workgroups, 16 ints apart
+constexpr int PR_LEFT = 16 + 16 * PR_GROUPS;
+// One edge in so many has to come from a hub for the copy to pay: it costs 1 us and the LDS
+// reads of every gather, a gather saved 1/230000 us.
+constexpr int PR_HUB_SHARE = 5;
 
 struct PrArgs {
     Ctl *ctl;
@@ -39,14 +72,14 @@ struct PrArgs {
     float *rank;
     float *contrib[2];
     uint32_t *chg[3];
-    const int *mid;
-    const ChunkRec *chunks;
+    const ChunkRec *runs;    // {first vertex, -, -, vertices}
+    const ChunkRec *lists;   // chunks (pad: the vertex's index in bigv), then medium lists (pad -1)
     const int *bigv;
     float *part;
     int *pact;
-    double *partials;    // per-workgroup L1 change
-    LevelPart *cpart;    // per-workgroup count of changed vertices (nf)
-    int n, nwords, nmid, nchunks, nbig, G1, G2, G3;  // G3: workgroups of pr_k3b (0: not run)
+    int *left;               // per high in-degree vertex: chunks summed; then workgroups finished
+    double *partials;        // per workgroup: L1 change, changed vertices
+    int n, nwords, nruns, nlists, nbig, G;
     int mode;
     float base, damp, eps;
     double tol_n;
@@ -70,34 +103,25 @@ __device__ __forceinline__ PrIter pr_iter(const PrArgs &a) {
     return s;
 }
 
-// Applies the gathered sum s to v; returns |new - old| (0 when inactive).
-__device__ __forceinline__ double pr_apply(const PrArgs &a, const PrIter &I, int v, float s, bool active,
-                                           int &nchanged) {
-    const int od = a.row_off[v + 1] - a.row_off[v];
+// Applies the gathered sum s to v; returns |new - old| (0 when inactive).  ranks: the rank
+// itself is read and stored (iterations whose ranks nothing looks at need only the
+// contributions).
+__device__ __forceinline__ double pr_apply(const PrArgs &a, const PrIter &I, int v, int od, float s, bool active,
+                                           bool ranks, int &nchanged) {
     if (!active) {
         I.c_new[v] = I.c_old[v];
         return 0.0;
     }
-    const float old = a.rank[v];
     const float nv = a.base + a.damp * s;
-    a.rank[v] = nv;
     I.c_new[v] = nv / (float)od;
+    if (!ranks) return 0.0;
+    const float old = a.rank[v];
+    a.rank[v] = nv;
     if (a.mode == MG_PR_GAS && !(fabsf(old - nv) < a.eps)) {
         atomicOr(&I.cur[v >> 5], 1u << (v & 31));
         if (od > 0) ++nchanged;  // only vertices with out-edges put anything in the next frontier
     }
     return fabs((double)nv - (double)old);
-}
-
-// Stores a workgroup's L1 change and changed-vertex count in slot `slot`.
-template <int BLOCK>
-__device__ __forceinline__ void pr_write_part(const PrArgs &a, int slot, double delta, long long nchanged) {
-    delta = block_sum<BLOCK>(delta);
-    nchanged = block_sum<BLOCK>(nchanged);
-    if (threadIdx.x == 0) {
-        a.partials[slot] = delta;
-        a.cpart[slot].nf = nchanged;
-    }
 }
 
 __global__ void pr_init(PrArgs a, int iter_limit) {
@@ -111,244 +135,291 @@ __global__ void pr_init(PrArgs a, int iter_limit) {
         a.chg[1][i] = 0;
         a.chg[2][i] = 0;
     }
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.nbig + PR_LEFT; i += gridDim.x * blockDim.x) a.left[i] = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl_reset(a.ctl, a.n, iter_limit, a.n);
 }
 
-// Low in-degree vertices, one lane each, in vertex order.
-__global__ __launch_bounds__(BLK) void pr_k1(PrArgs a) {
-    Ctl *c = a.ctl;
-    if (c->done) return;
-    const PrIter I = pr_iter(a);
-    const bool all = a.mode == MG_PR_ALL || I.it == 0;
-    // the bitmap filled at iteration it+1 is cleared now
-    uint32_t *clr = a.chg[(I.it + 1) % 3];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.nwords; i += gridDim.x * blockDim.x) clr[i] = 0;
-    double delta = 0;
-    int nchanged = 0;
-    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < a.n; v += gridDim.x * blockDim.x) {
-        const int beg = a.in_off[v], end = a.in_off[v + 1];
-        if (end - beg > PR_T1) continue;
-        float s = 0.0f;
-        bool act = all;
-        // four in-edges in flight (full groups load unconditionally), summed in order
-        int e = beg;
-        for (; e + 4 <= end; e += 4) {
-            int u[4];
-            float cv[4];
+// contrib[u]: from LDS below the hub count h, else from memory (lanes with a hub read one
+// shared entry there, so no branch waits between the loads of a batch).
+template <bool HUB>
+struct PrGather {
+    const float *c_old, *hubs;
+    int h, other;  // other: an entry of c_old for the lanes that have theirs in LDS
+    template <int K>
+    __device__ __forceinline__ void get(const int (&u)[K], float (&out)[K]) const {
+        if (!HUB) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) u[j] = a.in_adj[e + j];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) cv[j] = I.c_old[u[j]];
-            if (!all) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) act = act || test_bit(I.prev, u[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s = s + cv[j];
+            for (int j = 0; j < K; ++j) out[j] = c_old[u[j]];
+            return;
         }
-        for (; e < end; ++e) {
-            const int u = a.in_adj[e];
-            if (!all) act = act || test_bit(I.prev, u);
-            s = s + I.c_old[u];
+        float g[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) g[j] = c_old[u[j] < h ? other : u[j]];
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const float l = hubs[u[j] < h ? u[j] : 0];
+            out[j] = u[j] < h ? l : g[j];
         }
-        delta += pr_apply(a, I, v, s, act, nchanged);
     }
-    pr_write_part<BLK>(a, blockIdx.x, delta, nchanged);
-}
+};
 
 // Wave sum of edges [beg, end): lane-strided, then xor-butterfly.  `act` is OR-ed
 // over the wave as well.
-__device__ __forceinline__ float wave_gather(const PrArgs &a, const PrIter &I, int beg, int end, bool &act) {
+template <bool HUB>
+__device__ __forceinline__ float wave_gather(const PrArgs &a, const PrIter &I, const PrGather<HUB> &c, int beg, int end,
+                                             bool &act) {
     const int lane = lane_id();
     const bool all = act;  // activity already known: skip the bitmap
     float s = 0.0f;
     bool any = false;
-    // lane l sums edges l, l+64, ... in order, four in flight (full groups load
+    // lane l sums edges l, l+64, ... in order, eight then four in flight (full groups load
     // unconditionally), then the remainder one at a time
     int e = beg + lane;
-    for (; e + 3 * WAVE < end; e += 4 * WAVE) {
-        int u[4];
-        float cv[4];
+    auto batch = [&](auto kc) {
+        constexpr int K = decltype(kc)::value;
+        for (; e + (K - 1) * WAVE < end; e += K * WAVE) {
+            int u[K];
+            float cv[K];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) u[j] = a.in_adj[e + j * WAVE];
+            for (int j = 0; j < K; ++j) u[j] = a.in_adj[e + j * WAVE];
+            c.get(u, cv);
+            if (!all) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) cv[j] = I.c_old[u[j]];
-        if (!all) {
+                for (int j = 0; j < K; ++j) any = any || test_bit(I.prev, u[j]);
+            }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) any = any || test_bit(I.prev, u[j]);
+            for (int j = 0; j < K; ++j) s = s + cv[j];
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s = s + cv[j];
-    }
-    for (; e < end; e += WAVE) {
-        const int u = a.in_adj[e];
-        if (!all) any = any || test_bit(I.prev, u);
-        s = s + I.c_old[u];
-    }
+    };
+    batch(std::integral_constant<int, 8>());
+    batch(std::integral_constant<int, 4>());
+    batch(std::integral_constant<int, 1>());
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s = s + __shfl_xor(s, o);
     act = act || (wave_ballot(any) != 0);
     return s;
 }
 
-// Medium vertices (a wave each) and chunks of high in-degree vertices.
-__global__ __launch_bounds__(BLK) void pr_k2(PrArgs a) {
+// One iteration.
+template <bool HUB>
+__global__ __launch_bounds__(PR_BLK, 8) void pr_iterate(PrArgs a) {
     Ctl *c = a.ctl;
     if (c->done) return;
+    __shared__ float s_hubs[HUB ? PR_HUBS : 1];
+    __shared__ float s_buf[PR_BLK / WAVE][PR_BUF];
+    __shared__ int s_last;
     const PrIter I = pr_iter(a);
     const bool all = a.mode == MG_PR_ALL || I.it == 0;
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * BLK + threadIdx.x) / WAVE, nwaves = gridDim.x * BLK / WAVE;
+    const bool ranks = a.mode != MG_PR_ALL || a.tol_n > 0 || I.it + 1 >= c->iter_limit;
+    const int tid = blockIdx.x * PR_BLK + (int)threadIdx.x, nt = gridDim.x * PR_BLK;
+    PrGather<HUB> cg{I.c_old, s_hubs, 0, 0};
+    if (HUB) {
+        const int h = min(a.n, PR_HUBS);
+        const float4 *src = reinterpret_cast<const float4 *>(I.c_old);
+        for (int i = threadIdx.x; i < h / 4; i += PR_BLK) reinterpret_cast<float4 *>(s_hubs)[i] = src[i];
+        if ((int)threadIdx.x < h % 4) s_hubs[h / 4 * 4 + threadIdx.x] = I.c_old[h / 4 * 4 + threadIdx.x];
+        cg.h = h;
+        cg.other = min(h, a.n - 1);
+        __syncthreads();
+    }
+    // the bitmap filled at iteration it+1 is cleared now
+    uint32_t *clr = a.chg[(I.it + 1) % 3];
+    for (int i = tid; i < a.nwords; i += nt) clr[i] = 0;
     double delta = 0;
     int nchanged = 0;
-    for (int t = wave; t < a.nmid + a.nchunks; t += nwaves) {
+    // chunks of high in-degree vertices and medium vertices, a wave each; the next record is
+    // loaded, and the out-degree on its way, while a list is summed
+    const int lane = lane_id(), nw = nt / WAVE;
+    ChunkRec r{};
+    if (tid / WAVE < a.nlists) r = a.lists[tid / WAVE];
+    for (int t = tid / WAVE; t < a.nlists; t += nw) {
+        const ChunkRec next = a.lists[min(t + nw, a.nlists - 1)];
+        const int v = r.v, big = r.pad;
+        const int od = a.row_off[v + 1] - a.row_off[v];
         bool act = all;
-        if (t < a.nmid) {
-            const int v = a.mid[t];
-            const float s = wave_gather(a, I, a.in_off[v], a.in_off[v + 1], act);
-            if (lane == 0) delta += pr_apply(a, I, v, s, act, nchanged);
-        } else {
-            const int ci = t - a.nmid;
-            const ChunkRec r = a.chunks[ci];
-            const float s = wave_gather(a, I, r.beg, r.end, act);
-            if (lane == 0) {
-                a.part[ci] = s;
-                a.pact[ci] = act;
+        const float s = wave_gather<HUB>(a, I, cg, r.beg, r.end, act);
+        r = next;
+        if (big < 0) {
+            if (lane == 0) delta += pr_apply(a, I, v, od, s, act, ranks, nchanged);
+            continue;
+        }
+        const int c0 = a.bigv[big], c1 = a.bigv[big + 1];
+        int old = 0;
+        if (lane == 0) {
+            __hip_atomic_store(&a.part[t], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&a.pact[t], (int)act, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // stored before it is counted
+            old = atomicAdd(&a.left[big], 1);
+        }
+        if (__builtin_amdgcn_readfirstlane(old) != c1 - c0 - 1) continue;
+        // the vertex's last chunk: its sums in chunk order, 64 loaded together
+        float sum = 0.0f;
+        bool hot = all;
+        for (int ci = c0; ci < c1; ci += WAVE) {
+            const int i = min(ci + lane, c1 - 1);
+            const float p = __hip_atomic_load(&a.part[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int q = ld_dev(&a.pact[i]);
+            hot = hot || wave_ballot(ci + lane < c1 && q != 0) != 0;
+            const int m = min(WAVE, c1 - ci);
+            for (int j = 0; j < m; ++j) {
+                const float x = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j));
+                sum = ci == c0 && j == 0 ? x : sum + x;
             }
         }
+        if (lane == 0) {
+            a.left[big] = 0;
+            delta += pr_apply(a, I, v, od, sum, hot, ranks, nchanged);
+        }
     }
-    pr_write_part<BLK>(a, a.G1 + blockIdx.x, delta, nchanged);
-}
-
-// High in-degree vertices, a thread each: their chunk sums added in chunk order
-// (eight loads in flight), then applied.  Partials go to slots [G1 + G2, + G3).
-__global__ __launch_bounds__(BLK) void pr_k3b(PrArgs a) {
-    Ctl *c = a.ctl;
-    if (c->done) return;
-    const PrIter I = pr_iter(a);
-    const bool all = a.mode == MG_PR_ALL || I.it == 0;
-    double delta = 0;
-    int nchanged = 0;
-    for (int k = blockIdx.x * BLK + (int)threadIdx.x; k < a.nbig; k += gridDim.x * BLK) {
-        const int c0 = a.bigv[k], c1 = a.bigv[k + 1];
-        const int v = a.chunks[c0].v;
-        float s = a.part[c0];
-        bool act = a.pact[c0] != 0;
-        int ci = c0 + 1;
-        for (; ci + 8 <= c1; ci += 8) {
-            float p[8];
-            int q[8];
+    // low in-degree vertices: a wave gathers the edges of a run, each lane adds its vertex's
+    float *buf = s_buf[threadIdx.x / WAVE];
+    if (tid / WAVE < a.nruns) r = a.runs[tid / WAVE];
+    for (int t = tid / WAVE; t < a.nruns; t += nw) {
+        const ChunkRec next = a.runs[min(t + nw, a.nruns - 1)];
+        const bool mine = lane < r.pad;
+        const int w = mine ? r.v + lane : r.v;
+        const int od = a.row_off[w + 1] - a.row_off[w];
+        const int beg = a.in_off[r.v + min(lane, r.pad)], end = a.in_off[r.v + min(lane + 1, r.pad)];
+        const int e0 = __builtin_amdgcn_readfirstlane(beg), e1 = a.in_off[r.v + r.pad];
+        float s = 0.0f;
+        bool act = all;
+        for (int p0 = e0; p0 < e1; p0 += PR_BUF) {
+            constexpr int K = PR_BUF / WAVE;
+            int u[K];
+            float cv[K];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                p[j] = a.part[ci + j];
-                q[j] = a.pact[ci + j];
-            }
+            for (int j = 0; j < K; ++j) u[j] = a.in_adj[min(p0 + j * WAVE + lane, e1 - 1)];
+            cg.get(u, cv);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                s = s + p[j];
-                act = act || q[j] != 0;
+            for (int j = 0; j < K; ++j) buf[j * WAVE + lane] = cv[j];
+            if (!all) {
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    const uint64_t m = wave_ballot(test_bit(I.prev, u[j]));
+                    const int lo = max(beg - p0 - j * WAVE, 0), hi = min(end - p0 - j * WAVE, WAVE);
+                    if (hi > lo) act = act || ((m >> lo) & (~0ull >> (WAVE - (hi - lo)))) != 0;
+                }
             }
+            wave_sync();
+            for (int e = max(beg, p0); e < min(end, p0 + PR_BUF); ++e) s = s + buf[e - p0];
+            wave_sync();  // the next edges overwrite these
         }
-        for (; ci < c1; ++ci) {
-            s = s + a.part[ci];
-            act = act || a.pact[ci] != 0;
+        if (mine) delta += pr_apply(a, I, w, od, s, act, ranks, nchanged);
+        r = next;
+    }
+    // the last workgroup closes the iteration, adding the workgroups' sums in order; it is
+    // found by groups of counters (512 workgroups on one took 6 us)
+    if (ranks) {
+        delta = block_sum<PR_BLK>(delta);
+        const long long nch = block_sum<PR_BLK>((long long)nchanged);
+        if (threadIdx.x == 0) {
+            __hip_atomic_store(&a.partials[2 * blockIdx.x], delta, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&a.partials[2 * blockIdx.x + 1], (double)nch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        delta += pr_apply(a, I, v, s, act || all, nchanged);
     }
-    pr_write_part<BLK>(a, a.G1 + a.G2 + blockIdx.x, delta, nchanged);
-}
-
-// The iteration close in two stages, each in a fixed order (the same bits every run).
-// Tens of thousands of per-workgroup partials read by one workgroup took 22 us per
-// iteration at scale 22; first PR_RED workgroups sum fixed ranges of them into slots
-// np .. np + PR_RED - 1, then one workgroup sums those.
-constexpr int PR_RED = 64;
-__global__ __launch_bounds__(BLK) void pr_k3a(PrArgs a) {
-    if (a.ctl->done) return;
-    const int np = a.G1 + a.G2 + a.G3;
-    const int per = (np + PR_RED - 1) / PR_RED;
-    const int lo = blockIdx.x * per, hi = min(np, lo + per);
-    double delta = 0;
-    long long nch = 0;
-    for (int i = lo + (int)threadIdx.x; i < hi; i += BLK) {
-        delta += a.partials[i];
-        nch += a.cpart[i].nf;
-    }
-    delta = block_sum<BLK>(delta);
-    nch = block_sum<BLK>(nch);
+    __syncthreads();
     if (threadIdx.x == 0) {
-        a.partials[np + blockIdx.x] = delta;
-        a.cpart[np + blockIdx.x].nf = nch;
+        const int grp = blockIdx.x % PR_GROUPS, members = ((int)gridDim.x - grp + PR_GROUPS - 1) / PR_GROUPS;
+        int *cnt = a.left + a.nbig + 16 + 16 * grp;
+        s_last = 0;
+        if (atomicAdd(cnt, 1) == members - 1) {
+            *cnt = 0;
+            s_last = atomicAdd(&a.left[a.nbig], 1) == min((int)gridDim.x, PR_GROUPS) - 1;
+        }
     }
-}
-
-// One workgroup: closes the iteration from the PR_RED range sums.
-__global__ __launch_bounds__(SMALL_BLK) void pr_k3(PrArgs a) {
-    Ctl *c = a.ctl;
-    if (c->done) return;
-    const PrIter I = pr_iter(a);
-    double delta = 0;
-    long long nch = 0;
-    const int np = a.G1 + a.G2 + a.G3;
-    for (int i = threadIdx.x; i < PR_RED; i += SMALL_BLK) {
-        delta += a.partials[np + i];
-        nch += a.cpart[np + i].nf;
+    __syncthreads();
+    if (!s_last) return;
+    double l1 = 0, changed = 0;
+    if (ranks) {
+        for (int i = threadIdx.x; i < (int)gridDim.x; i += PR_BLK) {
+            l1 += __hip_atomic_load(&a.partials[2 * i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            changed += __hip_atomic_load(&a.partials[2 * i + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        l1 = block_sum<PR_BLK>(l1);
+        changed = block_sum<PR_BLK>(changed);
     }
-    const double l1 = block_sum<SMALL_BLK>(delta);
-    nch = block_sum<SMALL_BLK>(nch);
     if (threadIdx.x == 0) {
+        a.left[a.nbig] = 0;
         c->dsum = l1;
         c->level = I.it + 1;
-        c->changed = (int)nch;
+        c->changed = (int)changed;
         bool done = I.it + 1 >= c->iter_limit;
-        if (a.mode == MG_PR_GAS && nch == 0) done = true;
+        if (a.mode == MG_PR_GAS && changed == 0) done = true;
         if (a.mode == MG_PR_ALL && a.tol_n > 0 && l1 < a.tol_n) done = true;
         c->done = done;
     }
 }
 
-// Builds (once per graph and in-edge view) the medium-vertex list and the chunk
-// records of high in-degree vertices, on the host from the in-edge offsets.
-static int pr_buckets(mg_graph *g, const int *d_in_off) {
+// Edges whose source id is below `lim`.
+__global__ __launch_bounds__(BLK) void pr_count_below(const int *adj, int64_t m, int lim, unsigned long long *out) {
+    long long k = 0;
+    for (int64_t e = blockIdx.x * (int64_t)BLK + threadIdx.x; e < m; e += (int64_t)gridDim.x * BLK) k += adj[e] < lim;
+    k = block_sum<BLK>(k);
+    if (threadIdx.x == 0 && k) atomicAdd(out, (unsigned long long)k);
+}
+
+// Builds (once per graph and in-edge view) the records of the runs and lists, on the host from the in-edge offsets.
+static int pr_buckets(mg_graph *g, const int *d_in_off, const int *d_in_adj) {
     Workspace &ws = g->ws;
     if (ws.pr_view == d_in_off) return MG_OK;
     const int n = g->n;
     std::vector<int32_t> off((size_t)n + 1);
     MG_HIP(copy_on(g->stream, off.data(), d_in_off, 4 * ((size_t)n + 1), hipMemcpyDeviceToHost));
-    std::vector<int32_t> mid, bigv;
-    std::vector<ChunkRec> ch;
+    const int piece = (int)std::clamp<int64_t>(g->m / PR_PIECES / WAVE * WAVE, PR_PIECE_MIN, PR_PIECE_MAX);
+    std::vector<int32_t> bigv;
+    std::vector<ChunkRec> mid, ch, runs;
     for (int v = 0; v < n; ++v) {
         const int d = off[v + 1] - off[v];
-        if (d <= PR_T1) continue;
-        if (d <= PR_T2) {
-            mid.push_back(v);
+        if (d <= PR_T1) {
+            if (!runs.empty() && runs.back().v + runs.back().pad == v && runs.back().pad < WAVE &&
+                off[v + 1] - off[runs.back().v] <= piece)
+                runs.back().pad++;
+            else
+                runs.push_back(ChunkRec{v, 0, 0, 1});
+            continue;
+        }
+        if (d <= piece) {
+            mid.push_back(ChunkRec{v, off[v], off[v + 1], -1});
         } else {
             bigv.push_back((int)ch.size());
-            for (int b = off[v]; b < off[v + 1]; b += PR_T2) ch.push_back(ChunkRec{v, b, std::min(b + PR_T2, off[v + 1]), 0});
+            for (int b = off[v]; b < off[v + 1]; b += piece) ch.push_back(ChunkRec{v, b, std::min(b + piece, off[v + 1]), (int)bigv.size() - 1});
         }
     }
     bigv.push_back((int)ch.size());
-    free_dev(ws.pr_mid);
-    free_dev(ws.pr_chunks);
+    free_dev(ws.pr_lists);
     free_dev(ws.pr_bigv);
     free_dev(ws.pr_part);
     free_dev(ws.pr_pact);
-    ws.pr_mid = nullptr;
-    ws.pr_chunks = nullptr;
+    free_dev(ws.pr_left);
+    free_dev(ws.pr_runs);
+    ws.pr_left = nullptr;
+    ws.pr_runs = nullptr;
+    ws.pr_lists = nullptr;
     ws.pr_bigv = nullptr;
     ws.pr_part = nullptr;
     ws.pr_pact = nullptr;
     ws.pr_view = nullptr;
     int rc;
-    if ((rc = alloc_i32(&ws.pr_mid, mid.size())) || (rc = alloc_chunks(&ws.pr_chunks, ch.size())) ||
-        (rc = alloc_i32(&ws.pr_bigv, bigv.size())) || (rc = alloc_f32(&ws.pr_part, ch.size())) ||
-        (rc = alloc_i32(&ws.pr_pact, ch.size())))
+    const size_t nchunks = ch.size();
+    ch.insert(ch.end(), mid.begin(), mid.end());
+    if ((rc = alloc_chunks(&ws.pr_lists, ch.size())) || (rc = alloc_i32(&ws.pr_bigv, bigv.size())) ||
+        (rc = alloc_f32(&ws.pr_part, nchunks)) || (rc = alloc_i32(&ws.pr_pact, nchunks)) ||
+        (rc = alloc_i32(&ws.pr_left, bigv.size() + PR_LEFT)) || (rc = alloc_chunks(&ws.pr_runs, runs.size())))
         return rc;
-    if (!mid.empty()) MG_HIP(copy_on(g->stream, ws.pr_mid, mid.data(), 4 * mid.size(), hipMemcpyHostToDevice));
-    if (!ch.empty()) MG_HIP(copy_on(g->stream, ws.pr_chunks, ch.data(), sizeof(ChunkRec) * ch.size(), hipMemcpyHostToDevice));
+    // the share of the edges whose source is among the first PR_HUBS ids
+    MG_HIP(hipMemsetAsync(ws.d_reach, 0, 16, g->stream));
+    hipLaunchKernelGGL(pr_count_below, dim3(grid_blocks(g->m, BLK)), dim3(BLK), 0, g->stream, d_in_adj, g->m, PR_HUBS,
+                       ws.d_reach);
+    MG_HIP(hipGetLastError());
+    MG_HIP(copy_on(g->stream, ws.h_reach, ws.d_reach, 8, hipMemcpyDeviceToHost));
+    ws.pr_hubs = (int64_t)ws.h_reach[0] * PR_HUB_SHARE >= g->m;
+    if (!ch.empty()) MG_HIP(copy_on(g->stream, ws.pr_lists, ch.data(), sizeof(ChunkRec) * ch.size(), hipMemcpyHostToDevice));
     MG_HIP(copy_on(g->stream, ws.pr_bigv, bigv.data(), 4 * bigv.size(), hipMemcpyHostToDevice));
-    ws.pr_nmid = (int)mid.size();
-    ws.pr_nchunks = (int)ch.size();
+    if (!runs.empty())
+        MG_HIP(copy_on(g->stream, ws.pr_runs, runs.data(), sizeof(ChunkRec) * runs.size(), hipMemcpyHostToDevice));
+    ws.pr_nruns = (int)runs.size();
+    ws.pr_nlists = (int)ch.size();
     ws.pr_nbig = (int)bigv.size() - 1;
     ws.pr_view = d_in_off;
     return MG_OK;
@@ -381,7 +452,7 @@ extern "C" int mg_pagerank(mg_graph *g, float *rank_out, const mg_options *opt, 
     if ((rc = ensure_workspace(g)) || (rc = ensure_pr_workspace(g))) return rc;
     const int *in_off = sym ? g->row_off : g->col_off;
     const int *in_adj = sym ? g->col : g->row_idx;
-    if ((rc = pr_buckets(g, in_off))) return rc;
+    if ((rc = pr_buckets(g, in_off, in_adj))) return rc;
     Workspace &ws = g->ws;
     PrArgs a{};
     a.ctl = ws.ctl;
@@ -392,57 +463,33 @@ extern "C" int mg_pagerank(mg_graph *g, float *rank_out, const mg_options *opt, 
     a.contrib[0] = ws.contrib[0];
     a.contrib[1] = ws.contrib[1];
     for (int i = 0; i < 3; ++i) a.chg[i] = ws.bm[i];
-    a.mid = ws.pr_mid;
-    a.chunks = ws.pr_chunks;
+    a.lists = ws.pr_lists;
+    a.runs = ws.pr_runs;
+    a.nruns = ws.pr_nruns;
     a.bigv = ws.pr_bigv;
     a.part = ws.pr_part;
     a.pact = ws.pr_pact;
+    a.left = ws.pr_left;
     a.partials = ws.partials;
-    a.cpart = ws.part;
     a.n = g->n;
     a.nwords = ws.nwords;
-    a.nmid = ws.pr_nmid;
-    a.nchunks = ws.pr_nchunks;
+    a.nlists = ws.pr_nlists;
     a.nbig = ws.pr_nbig;
-    a.G1 = grid_blocks(g->n, BLK);
-    a.G2 = grid_blocks((int64_t)(a.nmid + a.nchunks) * WAVE, BLK);
     a.mode = o.pr_mode;
     a.base = o.pr_teleport;
     a.damp = 1.0f - o.pr_teleport;
     a.eps = o.pr_active_eps;
     a.tol_n = (double)o.pr_tol * (double)g->n;
-
-    // high in-degree vertices' chunk sums
-    a.G3 = a.nbig > 0 ? grid_blocks(a.nbig, BLK) : 0;
-    // The gather is latency-bound: with a grid-stride loop each thread walks several
-    // vertices (pr_k1) or each wave several lists (pr_k2) one after another.  Up to
-    // PR_MAX_GRID workgroups give every vertex / list its own thread / wave and let the
-    // hardware overlap them; the partial slots grow to match.
-    auto blocks = [](int64_t items) { return (int)std::max<int64_t>(1, std::min<int64_t>((items + BLK - 1) / BLK, PR_MAX_GRID)); };
-    a.G1 = blocks(g->n);
-    a.G2 = blocks((int64_t)(a.nmid + a.nchunks) * WAVE);
-    const int np = a.G1 + a.G2 + a.G3;
-    if (ws.pr_nslots < np + PR_RED) {  // the workgroups' slots, then the range sums
-        free_dev(ws.pr_partials);
-        free_dev(ws.pr_cpart);
-        ws.pr_partials = nullptr;
-        ws.pr_cpart = nullptr;
-        ws.pr_nslots = 0;
-        if ((rc = alloc_f64(&ws.pr_partials, np + PR_RED)) || (rc = alloc_parts(&ws.pr_cpart, np + PR_RED))) return rc;
-        ws.pr_nslots = np + PR_RED;
-    }
-    a.partials = ws.pr_partials;
-    a.cpart = ws.pr_cpart;
+    // two workgroups a CU; fewer on small graphs
+    const bool hubs = ws.pr_hubs;
+    a.G = grid_blocks_cap(std::max<int64_t>(a.nruns, a.nlists) * WAVE, PR_BLK, 512);
 
     MG_HIP(hipEventRecord(g->ev0, g->stream));
     hipLaunchKernelGGL(pr_init, dim3(grid_blocks(g->n, BLK)), dim3(BLK), 0, g->stream, a, o.iter_num);
     MG_HIP(hipGetLastError());
     auto step = [&]() -> int {
-        hipLaunchKernelGGL(pr_k1, dim3(a.G1), dim3(BLK), 0, g->stream, a);
-        hipLaunchKernelGGL(pr_k2, dim3(a.G2), dim3(BLK), 0, g->stream, a);
-        if (a.G3) hipLaunchKernelGGL(pr_k3b, dim3(a.G3), dim3(BLK), 0, g->stream, a);
-        hipLaunchKernelGGL(pr_k3a, dim3(PR_RED), dim3(BLK), 0, g->stream, a);
-        hipLaunchKernelGGL(pr_k3, dim3(1), dim3(SMALL_BLK), 0, g->stream, a);
+        if (hubs) hipLaunchKernelGGL(pr_iterate<true>, dim3(a.G), dim3(PR_BLK), 0, g->stream, a);
+        else hipLaunchKernelGGL(pr_iterate<false>, dim3(a.G), dim3(PR_BLK), 0, g->stream, a);
         MG_HIP(hipGetLastError());
         return MG_OK;
     };

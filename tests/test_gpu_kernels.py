@@ -266,3 +266,34 @@ def test_batch_pull_huge_weights(mg, oracle, device):
     with mg.Graph(g, symmetric=True) as dg:
         for got, s in zip(dg.sssp_batch(srcs), srcs):
             assert np.array_equal(got, dg.sssp(int(s)))
+
+
+# ---------------------------------------------------------------- PageRank
+@pytest.mark.parametrize("relabel", [False, True])
+@pytest.mark.parametrize("hubs", [True, False])
+@pytest.mark.parametrize("n", [3100, 15359, 15360, 15361, 40003])
+def test_pagerank_list_lengths(mg, oracle, device, n, hubs, relabel):
+    # in-degrees around a lane's, a wave's and a piece's edges, first, last and between low ones;
+    # sources all over the ids or, for a graph without hubs in LDS, past the ids kept there
+    rng = np.random.default_rng(n + hubs)
+    degs = [1, 2, 47, 48, 49, 63, 64, 65, 0, 255, 256, 257, 511, 512, 513, 1024, 1025, 3000]
+    at = [0, 1, 2, *sorted(rng.choice(np.arange(3, n - 3), len(degs) - 6, replace=False)), n - 3, n - 2, n - 1]
+    low = rng.integers(0, 5, n)
+    low[at] = rng.permutation(degs)
+    far = not hubs and n > 2 * 15360
+    src = np.concatenate([rng.choice(np.arange(15360 if far else 0, n), d, replace=False) for d in low])
+    g = mg.csr_from_edges(n, src.astype(np.int32), np.repeat(np.arange(n), low).astype(np.int32), mg.MG_CSR_SORT_COLS)
+    # all terms are positive: a list's sum errs by at most 48 (a lane), or 32 + 6 + 12 (pieces), roundings,
+    # the rank by 4 more, and 0.85 of an iteration's relative error goes into the next
+    rtol = (50 + 4) * 2.0**-24 / 0.15
+    with mg.Graph(g, build_csc=True, relabel=relabel) as dg:
+        for iters, tol in ((1, 0.0), (12, 0.0), (12, 1e-9)):
+            exp, _, _ = oracle.pr_jacobi_f64(g.row_offsets, g.col_idx, iters=iters)
+            for _ in range(2):
+                got, st = dg.pagerank(mg.options(pr_mode=mg.MG_PR_ALL, iter_num=iters, pr_tol=tol), stats=True)
+                assert st.iterations == iters
+                assert np.max(np.abs(got - exp) / exp) <= rtol
+        got, st = dg.pagerank(stats=True)
+    exp, it = oracle.pr_gas(g.row_offsets, g.col_idx)
+    assert abs(st.iterations - it) <= 1
+    assert np.max(np.abs(got.astype(np.float64) - exp)) / n <= 1e-6
