@@ -224,7 +224,7 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
 constexpr int PPR_SLOTS = 64;  // slots per context: one per lane
 
 struct PprDev {
-    int n = 0, ntasks = 0, nbig = 0, npart = 0;
+    int n = 0, ntasks = 0, npart = 0;
     int cur = 0;                          // X[cur] holds the current ranks
     int width = 8;                        // row width W: 8, 16, 32 or 64 columns
     uint64_t live = 0;                    // slots in use

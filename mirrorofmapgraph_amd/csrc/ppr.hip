@@ -7,12 +7,12 @@
 //   x_0 = e_s,   x_{i+1}[u] = (1 - t) * sum_{v -> u} x_i[v] / outdeg(v)  (+ t when u = s).
 // Ranks are vertex-major, X[v * W + slot], W = 8, 16, 32 or 64 floats per vertex: the
 // smallest width above every slot in use (slots are handed out lowest first; the rows
-// are repacked when it changes), so a wave gathers one in-edge's row for 64 / W edges
+// are repacked when it changes), so a wave gathers the rows of 256 / W in-edges
 // at a time and a row is one 32-byte sector while at most 8 slots are in use.
 // Vertices are covered by static tasks: runs of consecutive vertices with at most
-// PPR_T in-edges in total (one wave walks them), and PPR_T-edge pieces of longer
+// ppr_piece() in-edges in total (one wave walks them), and pieces of that size of longer
 // in-lists whose partial sums are added in piece order.  Every list is summed in one
-// order fixed by the list alone, whatever the width (see gather_sum), so a slot's
+// order fixed by the list alone, whatever the width (see team_list), so a slot's
 // arithmetic is fixed by the graph: a query gives the same bits alone or beside any
 // other queries.
 #include "batch.h"
@@ -21,20 +21,25 @@
 
 namespace mg {
 
-constexpr int PPR_T = 1024;    // in-edges per task
+// In-edges per task: m / PPR_PIECES within these limits, so that small graphs have tasks for
+// every wave (scale 16: 26 us an iteration with 1024 edges whatever the size, 17 so) and large
+// ones as few pieces as fill the GPU (scale 20: 512 edges 208 us, 1024 174, 2048 172).
+constexpr int PPR_PIECES = 16384, PPR_T_MIN = 256, PPR_T_MAX = 1024;
 constexpr int PPR_RUN = 64;    // vertices per run task
 
 struct PprArgs {
     const int *in_off, *in_adj;  // in-edges (CSR of a symmetric graph, or the CSC)
     const int *out_off;          // out-degrees
-    const float *X;              // current ranks, n x W
-    float *Xn;                   // next ranks
-    float *C;                    // contributions X / outdeg
+    const float *X;              // ranks, n x W (ppr_contrib)
+    const float *C;              // contributions rank / outdeg, n x W, and a row of zeros
+    float *D;                    // next contributions, or the ranks after the last iteration
     float *part;                 // piece partial sums, npart x W
-    const ChunkRec *tasks;       // runs: {v0, -, -, count}; pieces: {v, beg, end, -(part + 1)}
-    const int *big;              // per long list: vertex, first part, parts (3 ints)
+    const ChunkRec *tasks;       // pieces of long lists: {v, beg, end, list}; then runs: {v0, -, -, count}
+    int *big;                    // per long list: vertex, first part, parts, parts summed (4 ints)
     const int *src;              // per slot: source or -1
-    int n, ntasks, nbig;
+    int64_t m;
+    int n, npart, ntasks;
+    int last;                    // D takes ranks
     float t;                     // teleport
 };
 
@@ -42,159 +47,241 @@ struct PprArgs {
 // of 8, 16, 32, 64 above every slot in use (slots are handed out lowest first), so a
 // gathered row is W floats: 32 bytes (one sector) while at most 8 slots are in use,
 // and the contribution array of a 4M-vertex graph is 128 MB instead of 1 GB.
-__host__ __device__ constexpr int ppr_groups(int W) { return WAVE / W; }
 
-// C[v][c] = X[v][c] / outdeg(v) (0 for dangling v), over all n x W entries.
+// What bounds an iteration is reading rows that the L2 does not hold: at R-MAT scale 20 (31.4M
+// edges) and W = 8, 28M lines of 128 bytes go from L2 to L1 (92 us at 64 bytes a clock and CU)
+// and 7M from memory to the L2 (4.8 TB/s), at W = 64 4.5 GB (5.7 TB/s).  Below that the
+// address unit is: it takes a quad of lanes a clock whatever the lanes load, so a lane loads
+// four columns (16 bytes) at once, and four sources.  Four columns, a list per group and one
+// launch an iteration, against a column per lane, a list per wave and three launches, us an
+// iteration on the degree-ordered twin:
+//   scale    W = 8         16          64
+//   16     56 -> 17    76 -> 20    159 -> 53
+//   18     99 -> 44   136 -> 57    312 -> 164
+//   20    241 -> 174  378 -> 231  1070 -> 776
+// Rows of the highest degrees kept in LDS took 185 at W = 8; the next block's sources loaded
+// ahead of the gathers 185 (more registers, fewer waves).
+
+// A wave's lanes for rows of W columns: V columns a lane, L lanes a row, G rows side by side.
+// Eight partial sums make a list (see below): a team of T groups sums a list together, J
+// partial sums a lane, NT teams a wave.
 template <int W>
-__global__ __launch_bounds__(BLK) void ppr_contrib(PprArgs a) {
+struct PprLanes {
+    static constexpr int V = 4, L = W / V, G = WAVE / L, T = G < 8 ? G : 8, J = 8 / T, NT = G / T;
+    typedef float Vec __attribute__((ext_vector_type(V)));
+};
+
+// C[v][c] = X[v][c] / outdeg(v) (0 for dangling v), over all n x W entries; the rows of
+// zeros behind C and D.
+template <int W>
+__global__ __launch_bounds__(BLK) void ppr_contrib(PprArgs a, float *C) {
     const int64_t total = (int64_t)a.n * W;
     for (int64_t i = blockIdx.x * (int64_t)BLK + threadIdx.x; i < total; i += (int64_t)gridDim.x * BLK) {
         const int v = (int)(i / W);
         const int d = a.out_off[v + 1] - a.out_off[v];
-        a.C[i] = d > 0 ? a.X[i] / (float)d : 0.f;
+        C[i] = d > 0 ? a.X[i] / (float)d : 0.f;
+    }
+    if (blockIdx.x == 0 && threadIdx.x < W) {
+        C[total + threadIdx.x] = 0.f;
+        a.D[total + threadIdx.x] = 0.f;
     }
 }
 
-// Sum of the lane's column over in-edges [beg, end), in one order for every width:
-// the edge at offset k of the list goes to partial sum k mod 8 (each partial sum adds
-// its edges in list order), and the eight partial sums are combined as
-// ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)).  A wave holds G = 64 / W edge
-// groups of W lanes (lane = g * W + column): group g owns partial sums g + G j
-// (j < 8 / G), so a wave instruction gathers G rows; the combination steps over
-// partial sums on different groups are lane butterflies (xor W, 2W, 4W), the others
-// adds inside the lane, and addition is commutative, so every width and every lane of
-// a pair computes the same bits.  Eight gathers per lane are in flight per step
-// (G rounds of eight edges); the last step loads from clamped slots and adds only
-// the edges in range.
-template <int W>
-__device__ __forceinline__ float gather_sum(const PprArgs &a, int beg, int end, int g, int col) {
-    constexpr int G = ppr_groups(W), J = 8 / G;
-    float acc[J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) acc[j] = 0.f;
-    for (int e0 = beg; e0 < end; e0 += 8 * G) {
-        // round r of the step covers edges e0 + 8 r .. e0 + 8 r + 7; this lane's edge
-        // of partial sum g + G j in round r is e0 + 8 r + g + G j
-        int u[G][J];
-        bool ok[G][J];
-#pragma unroll
-        for (int r = 0; r < G; ++r)
-#pragma unroll
-            for (int j = 0; j < J; ++j) {
-                const int e = e0 + 8 * r + g + G * j;
-                ok[r][j] = e < end;
-                u[r][j] = a.in_adj[ok[r][j] ? e : beg];
-            }
-        float c[G][J];
-#pragma unroll
-        for (int r = 0; r < G; ++r)
-#pragma unroll
-            for (int j = 0; j < J; ++j) c[r][j] = a.C[(int64_t)u[r][j] * W + col];
-#pragma unroll
-        for (int r = 0; r < G; ++r)
-#pragma unroll
-            for (int j = 0; j < J; ++j)
-                if (ok[r][j]) acc[j] += c[r][j];
+// A block's sum in the lane's columns: the eight in-edges of the list (`len` long, at in_adj +
+// beg) from offset e on, past its end the row of zeros.  Two lanes load four sources each
+// (a.m bounds the array), quad permutes spread them, and the eight rows are gathered together.
+template <int W, bool WIDE>
+__device__ __forceinline__ typename PprLanes<W>::Vec ppr_block(const PprArgs &a, int beg, int len, int e) {
+    using P = PprLanes<W>;
+    typedef int Int4 __attribute__((ext_vector_type(4), aligned(4)));
+    e += 4 * (lane_id() & 1);
+    const int at = beg + (e < len ? e : 0);
+    Int4 x;
+    if (at + 4LL <= a.m) {
+        x = *(const Int4 *)(a.in_adj + at);
+    } else {
+        x = a.n;
+        for (int j = 0; j < 4; ++j)
+            if (at + j < a.m) x[j] = a.in_adj[at + j];
     }
-    // combine: level b pairs partial sums whose index differs in bit b
-    float s[J];
+    typename P::Vec c[8];
+    const uint32_t l = lane_id() % P::L * (4 * P::V);
 #pragma unroll
-    for (int j = 0; j < J; ++j) s[j] = acc[j];
-    int nj = J;
-#pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        if ((1 << b) < G) {  // partner on group g ^ (1 << b)
-#pragma unroll
-            for (int j = 0; j < J; ++j) s[j] += __shfl_xor(s[j], W << b);
-        } else {  // partner in this lane: j ^ (1 << (b - log2 G))
-            const int h = nj / 2;
-#pragma unroll
-            for (int j = 0; j < J / 2; ++j)
-                if (j < h) s[j] = s[2 * j] + s[2 * j + 1];
-            nj = h;
-        }
+    for (int k = 0; k < 8; ++k) {
+        const int y = e + k % 4 < len ? x[k % 4] : a.n;
+        const int u = P::L == 2 ? (k < 4 ? __builtin_amdgcn_mov_dpp(y, 0xA0, 0xF, 0xF, true)    // lanes 0, 0, 2, 2
+                                         : __builtin_amdgcn_mov_dpp(y, 0xF5, 0xF, 0xF, true))   // lanes 1, 1, 3, 3
+                                : (k < 4 ? __builtin_amdgcn_mov_dpp(y, 0x00, 0xF, 0xF, true)    // lane 0 of the quad
+                                         : __builtin_amdgcn_mov_dpp(y, 0x55, 0xF, 0xF, true));  // lane 1
+        const uint64_t off = WIDE ? (uint64_t)(uint32_t)u * (4 * W) + l : (uint64_t)((uint32_t)u * (4 * W) + l);
+        c[k] = *(const typename P::Vec *)((const char *)a.C + off);
     }
-    return s[0];
-}
-
-// The same sum for a list of at most 8 edges, by one group alone: edge k is partial
-// sum k (the others are 0), combined in the same tree inside the lane.  Slots past
-// the end load from beg, which is in range only for a non-empty list (an empty list
-// at the end of the array has beg = m): an empty list loads nothing and sums to 0,
-// as the tree of eight zero partial sums does.
-template <int W>
-__device__ __forceinline__ float short_sum(const PprArgs &a, int beg, int end, int col) {
-    if (end <= beg) return 0.f;
-    int u[8];
-    float c[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) u[k] = a.in_adj[beg + k < end ? beg + k : beg];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) c[k] = a.C[(int64_t)u[k] * W + col];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) c[k] = beg + k < end ? 0.f + c[k] : 0.f;
     return ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
 }
 
-__device__ __forceinline__ float ppr_apply(float s, float t, bool is_src) {
-    const float v = (1.0f - t) * s;
-    return is_src ? t + v : v;
+// Sum of the lane's columns over a list of `len` in-edges, in one order for every width: the
+// list is cut into blocks of eight edges, a block is summed as in ppr_block, block i is added
+// to partial sum i mod 8 (each adds its blocks in order), and the partial sums are combined
+// as ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)).  Here a team sums one list: group g of
+// its T sums blocks T i + g; the combination steps over partial sums on different groups are
+// lane butterflies, the others adds inside the lane, and addition is commutative, so every
+// width and every lane computes the same bits.
+template <int W, bool WIDE>
+__device__ __forceinline__ typename PprLanes<W>::Vec team_list(const PprArgs &a, int beg, int len, int steps) {
+    using P = PprLanes<W>;
+    const int g = lane_id() / P::L % P::T;
+    typename P::Vec acc[P::J];
+#pragma unroll
+    for (int j = 0; j < P::J; ++j) acc[j] = 0.f;
+    for (int i = 0; i < steps; i += P::J)
+#pragma unroll
+        for (int j = 0; j < P::J; ++j) {
+            if (i + j >= steps) continue;
+            acc[j] += ppr_block<W, WIDE>(a, beg, len, 8 * (P::T * (i + j) + g));
+        }
+    // partial sum g + T j is acc[j] of group g
+    static_assert(P::T * P::J == 8, "eight partial sums");
+#pragma unroll
+    for (int b = 1; b < P::T; b *= 2)
+#pragma unroll
+        for (int j = 0; j < P::J; ++j)
+#pragma unroll
+            for (int i = 0; i < P::V; ++i) acc[j][i] += __shfl_xor(acc[j][i], P::L * b);
+#pragma unroll
+    for (int b = 1; b < P::J; b *= 2)
+#pragma unroll
+        for (int j = 0; j + b < P::J; j += 2 * b) acc[j] += acc[j + b];
+    return acc[0];
 }
 
+// The same sums with a list per group, in `steps` blocks (the longest list's).
+template <int W, bool WIDE>
+__device__ __forceinline__ typename PprLanes<W>::Vec group_list(const PprArgs &a, int beg, int len, int steps) {
+    typename PprLanes<W>::Vec acc[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[k] = 0.f;
+    for (int i = 0; i < steps; i += 8)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (i + j >= steps) continue;
+            acc[j] += ppr_block<W, WIDE>(a, beg, len, 8 * (i + j));
+        }
+    return ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+}
+
+// The lane's columns of u from their sums, as ranks after the last iteration, as the
+// contributions that the next one gathers before.  Idle columns are set too, to nothing that
+// is looked at.
 template <int W>
+__device__ __forceinline__ void ppr_apply(const PprArgs &a, int u, typename PprLanes<W>::Vec s,
+                                          const int (&src)[PprLanes<W>::V]) {
+    using P = PprLanes<W>;
+    const int d = a.out_off[u + 1] - a.out_off[u];
+    typename P::Vec x;
+#pragma unroll
+    for (int i = 0; i < P::V; ++i) {
+        const float v = (1.0f - a.t) * s[i];
+        x[i] = u == src[i] ? a.t + v : v;
+        if (!a.last) x[i] = d > 0 ? x[i] / (float)d : 0.f;
+    }
+    *(typename P::Vec *)(a.D + (int64_t)u * W + lane_id() % P::L * P::V) = x;
+}
+
+// One iteration.  WIDE: rows past 4 GiB.
+template <int W, bool WIDE>
 __global__ __launch_bounds__(BLK) void ppr_gather(PprArgs a) {
-    constexpr int G = ppr_groups(W);
-    const int lane = lane_id(), g = lane / W, col = lane % W;
+    using P = PprLanes<W>;
+    const int lane = lane_id(), g = lane / P::L, l = lane % P::L, team = g / P::T;
     const int wave = (blockIdx.x * BLK + (int)threadIdx.x) / WAVE, nwaves = gridDim.x * BLK / WAVE;
-    const int src = a.src[col];
-    const bool on = src >= 0;
-    if (!__any(on)) return;
-    for (int t = wave; t < a.ntasks; t += nwaves) {
-        const ChunkRec r = a.tasks[t];
-        if (r.pad > 0) {
-            // G vertices of the run at a time: lists of at most 8 edges are summed by
-            // their group alone, longer ones by the whole wave, one after another
-            // (idle columns unused)
-            for (int u0 = r.v; u0 < r.v + r.pad; u0 += G) {
-                const int u = u0 + g;
-                const bool has = u < r.v + r.pad;
-                const int b = has ? a.in_off[u] : 0, e = has ? a.in_off[u + 1] : 0;
-                const bool shortl = has && e - b <= 8;
-                if (__any(shortl) && shortl) {
-                    const float s = short_sum<W>(a, b, e, col);
-                    if (on) a.Xn[(int64_t)u * W + col] = ppr_apply(s, a.t, u == src);
+    int src[P::V];
+#pragma unroll
+    for (int i = 0; i < P::V; ++i) src[i] = a.src[l * P::V + i];
+    // pieces of long lists, one a team; the team that sums a list's last adds them all in
+    // order, T loaded together
+    for (int t0 = wave * P::NT; t0 < a.npart; t0 += nwaves * P::NT) {
+        const int t = t0 + team;
+        const ChunkRec r = a.tasks[min(t, a.npart - 1)];
+        const int len = t < a.npart ? r.end - r.beg : 0;
+        int steps = (len + 8 * P::T - 1) / (8 * P::T);
+#pragma unroll
+        for (int o = P::T * P::L; o < WAVE; o *= 2) steps = max(steps, __shfl_xor(steps, o));
+        const auto s = team_list<W, WIDE>(a, r.beg, len, __builtin_amdgcn_readfirstlane(steps));
+        if (len == 0) continue;
+        int *big = a.big + 4 * r.pad;
+        const int p0 = big[1], np = big[2];
+        if (g % P::T == 0)
+#pragma unroll
+            for (int i = 0; i < P::V; ++i)
+                __hip_atomic_store(&a.part[(int64_t)t * W + l * P::V + i], s[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // stored before it is counted
+        const int first = team * P::T * P::L;
+        int old = 0;
+        if (lane == first) old = atomicAdd(&big[3], 1);
+        if (__shfl(old, first) != np - 1) continue;
+        typename P::Vec sum = 0.f;
+        for (int p = 0; p < np; p += P::T) {
+            const int64_t at = (int64_t)(p0 + min(p + g % P::T, np - 1)) * W + l * P::V;
+            typename P::Vec x;
+#pragma unroll
+            for (int i = 0; i < P::V; ++i) x[i] = __hip_atomic_load(&a.part[at + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int j = 0; j < P::T; ++j)
+#pragma unroll
+                for (int i = 0; i < P::V; ++i) {
+                    const float y = __shfl(x[i], first + j * P::L + l);
+                    if (p + j < np) sum[i] += y;
                 }
-                uint64_t longs = wave_ballot(has && !shortl && col == 0);  // bit g * W per long list
-                while (longs) {
-                    const int gl = (__ffsll((unsigned long long)longs) - 1) / W;
-                    longs &= longs - 1;
-                    const int ul = u0 + gl;
-                    const float s = gather_sum<W>(a, a.in_off[ul], a.in_off[ul + 1], g, col);
-                    if (on && g == 0) a.Xn[(int64_t)ul * W + col] = ppr_apply(s, a.t, ul == src);
+        }
+        if (lane == first) big[3] = 0;
+        if (g % P::T == 0) ppr_apply<W>(a, r.v, sum, src);
+    }
+    // runs, G vertices at a time: a list per group, or, where that takes more steps, a list
+    // per team, one after another
+    for (int t = a.npart + wave; t < a.ntasks; t += nwaves) {
+        const ChunkRec r = a.tasks[t];
+        for (int u0 = r.v; u0 < r.v + r.pad; u0 += P::G) {
+            const int u = u0 + g;
+            const bool has = u < r.v + r.pad;
+            const int b = has ? a.in_off[u] : 0, len = has ? a.in_off[u + 1] - b : 0;
+            int longest = (len + 7) / 8, one = (len + 8 * P::T - 1) / (8 * P::T);
+#pragma unroll
+            for (int o = P::L; o < WAVE; o *= 2) {
+                longest = max(longest, __shfl_xor(longest, o));
+                one += __shfl_xor(one, o);
+            }
+            longest = __builtin_amdgcn_readfirstlane(longest);
+            one = __builtin_amdgcn_readfirstlane(one);
+            typename P::Vec s = 0.f;
+            if (longest * P::NT <= one) {
+                s = group_list<W, WIDE>(a, b, len, longest);
+            } else {
+                uint64_t some = wave_ballot(len > 0 && l == 0);  // bit g * L per list
+                while (some) {
+                    int at[P::NT];
+#pragma unroll
+                    for (int i = 0; i < P::NT; ++i) {
+                        at[i] = some ? __ffsll((unsigned long long)some) - 1 : -1;
+                        some &= some - 1;
+                    }
+                    const int mine = at[team], from = max(mine, 0);
+                    int tb = __shfl(b, from), tl = __shfl(len, from);
+                    if (mine < 0) tb = tl = 0;
+                    int steps = 0;
+#pragma unroll
+                    for (int i = 0; i < P::NT; ++i)
+                        steps = max(steps, at[i] < 0 ? 0 : (__builtin_amdgcn_readlane(len, at[i]) + 8 * P::T - 1) / (8 * P::T));
+                    const auto sl = team_list<W, WIDE>(a, tb, tl, steps);
+#pragma unroll
+                    for (int i = 0; i < P::NT; ++i)
+#pragma unroll
+                        for (int c = 0; c < P::V; ++c) {
+                            const float y = __shfl(sl[c], i * P::T * P::L + l);
+                            if (at[i] / P::L == g && at[i] >= 0) s[c] = y;
+                        }
                 }
             }
-        } else {
-            const float s = gather_sum<W>(a, r.beg, r.end, g, col);
-            if (on && g == 0) a.part[(int64_t)(-r.pad - 1) * W + col] = s;
+            if (has) ppr_apply<W>(a, u, s, src);
         }
-    }
-}
-
-// Long in-lists: the pieces' partial sums added in piece order (G lists per wave).
-template <int W>
-__global__ __launch_bounds__(BLK) void ppr_combine(PprArgs a) {
-    constexpr int G = ppr_groups(W);
-    const int lane = lane_id(), g = lane / W, col = lane % W;
-    const int wave = (blockIdx.x * BLK + (int)threadIdx.x) / WAVE, nwaves = gridDim.x * BLK / WAVE;
-    const int src = a.src[col];
-    const bool on = src >= 0;
-    for (int b0 = wave * G; b0 < a.nbig; b0 += nwaves * G) {
-        const int b = b0 + g;
-        if (b >= a.nbig) continue;
-        const int u = a.big[3 * b], p0 = a.big[3 * b + 1], np = a.big[3 * b + 2];
-        float s = 0.f;
-        for (int p = p0; p < p0 + np; ++p) s += on ? a.part[(int64_t)p * W + col] : 0.f;
-        if (on) a.Xn[(int64_t)u * W + col] = ppr_apply(s, a.t, u == src);
     }
 }
 
@@ -270,11 +357,16 @@ static bool ppr_view(const mg_graph *g, const int **off, const int **adj) {
     return false;
 }
 
+static int ppr_piece(const mg_graph *g) {
+    return (int)std::clamp<int64_t>(g->m / PPR_PIECES / WAVE * WAVE, PPR_T_MIN, PPR_T_MAX);
+}
+
 int64_t ppr_dev_bytes(const mg_graph *g) {
     const int64_t n = g->n;
-    const int64_t tasks = g->m / PPR_T + n / PPR_RUN + 2 * (g->m / PPR_T) + 64;
-    return 3 * 4LL * PPR_SLOTS * n + 4LL * PPR_SLOTS * (g->m / PPR_T + 64) + (int64_t)sizeof(ChunkRec) * tasks +
-           12LL * (g->m / PPR_T + 64) + 4LL * PPR_SLOTS + 4LL * PPR_SLOTS * n;
+    const int T = ppr_piece(g);
+    const int64_t tasks = g->m / T + n / PPR_RUN + 2 * (g->m / T) + 64;
+    return 3 * 4LL * PPR_SLOTS * (n + 1) + 4LL * PPR_SLOTS * (g->m / T + 64) + (int64_t)sizeof(ChunkRec) * tasks +
+           16LL * (g->m / T + 64) + 4LL * PPR_SLOTS + 4LL * PPR_SLOTS * n;
 }
 
 int ppr_dev_alloc(PprDev &p, mg_graph *g, hipStream_t st) {
@@ -285,44 +377,36 @@ int ppr_dev_alloc(PprDev &p, mg_graph *g, hipStream_t st) {
     const int n = g->n;
     std::vector<int> h_off((size_t)n + 1);
     MG_HIP(copy_on(st, h_off.data(), off, 4 * ((size_t)n + 1), hipMemcpyDeviceToHost));
-    std::vector<ChunkRec> tasks;
+    const int T = ppr_piece(g);
+    std::vector<ChunkRec> tasks, runs;
     std::vector<int> big;
-    int npart = 0;
     for (int v = 0; v < n;) {
         const int d = h_off[v + 1] - h_off[v];
-        if (d > PPR_T) {
-            const int np = (d + PPR_T - 1) / PPR_T;
-            big.push_back(v);
-            big.push_back(npart);
-            big.push_back(np);
-            for (int k = 0; k < np; ++k) {
-                const int b = h_off[v] + k * PPR_T;
-                tasks.push_back(ChunkRec{v, b, std::min(b + PPR_T, h_off[v + 1]), -(npart + k + 1)});
-            }
-            npart += np;
+        if (d > T) {
+            big.insert(big.end(), {v, (int)tasks.size(), (d + T - 1) / T, 0});
+            for (int b = h_off[v]; b < h_off[v + 1]; b += std::min(T, h_off[v + 1] - b))
+                tasks.push_back(ChunkRec{v, b, b + std::min(T, h_off[v + 1] - b), (int)(big.size() / 4) - 1});
             ++v;
             continue;
         }
         int u = v, e = 0;
-        while (u < n && u - v < PPR_RUN && h_off[u + 1] - h_off[u] <= PPR_T && e + (h_off[u + 1] - h_off[u]) <= PPR_T) {
+        while (u < n && u - v < PPR_RUN && h_off[u + 1] - h_off[u] <= T && e + (h_off[u + 1] - h_off[u]) <= T) {
             e += h_off[u + 1] - h_off[u];
             ++u;
         }
-        if (u == v) ++u;  // cannot happen (d <= PPR_T), kept for termination
-        tasks.push_back(ChunkRec{v, 0, 0, u - v});
+        runs.push_back(ChunkRec{v, 0, 0, u - v});
         v = u;
     }
+    const int npart = (int)tasks.size();
+    tasks.insert(tasks.end(), runs.begin(), runs.end());
     p.n = n;
     p.ntasks = (int)tasks.size();
-    p.nbig = (int)(big.size() / 3);
     p.npart = npart;
     hipError_t e = hipSuccess;
     auto A = [&](void **q, size_t bytes) {
         if (e == hipSuccess) e = alloc_refused() ? hipErrorOutOfMemory : hipMalloc(q, bytes ? bytes : 16);
     };
-    A((void **)&p.X[0], 4 * (size_t)PPR_SLOTS * n);
-    A((void **)&p.X[1], 4 * (size_t)PPR_SLOTS * n);
-    A((void **)&p.C, 4 * (size_t)PPR_SLOTS * n);
+    for (float **q : {&p.X[0], &p.X[1], &p.C}) A((void **)q, 4 * (size_t)PPR_SLOTS * (n + 1));
     A((void **)&p.part, 4 * (size_t)PPR_SLOTS * npart);
     A((void **)&p.tasks, sizeof(ChunkRec) * tasks.size());
     A((void **)&p.big, 4 * big.size());
@@ -334,8 +418,8 @@ int ppr_dev_alloc(PprDev &p, mg_graph *g, hipStream_t st) {
         std::vector<int> none(PPR_SLOTS, -1);
         e = copy_on(st, p.src, none.data(), 4 * PPR_SLOTS, hipMemcpyHostToDevice);
     }
-    if (e == hipSuccess) e = hipMemsetAsync(p.X[0], 0, 4 * (size_t)PPR_SLOTS * n, st);
-    if (e == hipSuccess) e = hipMemsetAsync(p.X[1], 0, 4 * (size_t)PPR_SLOTS * n, st);
+    if (e == hipSuccess) e = hipMemsetAsync(p.X[0], 0, 4 * (size_t)PPR_SLOTS * (n + 1), st);
+    if (e == hipSuccess) e = hipMemsetAsync(p.X[1], 0, 4 * (size_t)PPR_SLOTS * (n + 1), st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
         ppr_dev_free(p);
@@ -356,15 +440,14 @@ static PprArgs ppr_args(PprDev &p, mg_graph *g, float t) {
     ppr_view(g, &a.in_off, &a.in_adj);
     a.out_off = g->row_off;
     a.X = p.X[p.cur];
-    a.Xn = p.X[p.cur ^ 1];
-    a.C = p.C;
     a.part = p.part;
     a.tasks = p.tasks;
     a.big = p.big;
     a.src = p.src;
+    a.m = g->m;
     a.n = p.n;
+    a.npart = p.npart;
     a.ntasks = p.ntasks;
-    a.nbig = p.nbig;
     a.t = t;
     return a;
 }
@@ -388,20 +471,28 @@ int ppr_seed(PprDev &p, hipStream_t st, const SeedList &sl, const SlotList &reti
     return MG_OK;
 }
 
+// A launch per iteration, contributions to contributions, the last one to ranks: through C
+// and the spare rank buffer, and over the current ranks (needed by then for nothing) when the
+// last contributions are in the spare one.
 template <int W>
 static int ppr_iterate_w(PprDev &p, mg_graph *g, hipStream_t st, float t, int iters) {
+    if (iters <= 0 || p.live == 0) return MG_OK;
+    PprArgs a = ppr_args(p, g, t);
+    float *spare = p.X[p.cur ^ 1], *from = p.C;
+    a.D = spare;
+    hipLaunchKernelGGL(ppr_contrib<W>, dim3(grid_blocks_cap((int64_t)p.n * W, BLK, 4 * MAX_GRID)), dim3(BLK), 0, st, a, p.C);
+    const int G = grid_blocks_cap((int64_t)p.ntasks * WAVE, BLK, 1 << 20);  // hardware hands them out as waves end
+    const bool wide = ((uint64_t)p.n + 1) * W * 4 > UINT32_MAX;
     for (int i = 0; i < iters; ++i) {
-        PprArgs a = ppr_args(p, g, t);
-        const int G = grid_blocks(std::max<int64_t>((int64_t)p.ntasks * WAVE, (int64_t)p.n * 4), BLK);
-        hipLaunchKernelGGL(ppr_contrib<W>, dim3(grid_blocks_cap((int64_t)p.n * W, BLK, 4 * MAX_GRID)), dim3(BLK), 0,
-                           st, a);
-        hipLaunchKernelGGL(ppr_gather<W>, dim3(G), dim3(BLK), 0, st, a);
-        if (p.nbig)
-            hipLaunchKernelGGL(ppr_combine<W>, dim3(grid_blocks((int64_t)p.nbig * WAVE / ppr_groups(W), BLK) + 1),
-                               dim3(BLK), 0, st, a);
-        MG_HIP(hipGetLastError());
-        p.cur ^= 1;
+        a.last = i == iters - 1;
+        a.C = from;
+        a.D = from == p.C ? spare : a.last ? p.X[p.cur] : p.C;
+        if (wide) hipLaunchKernelGGL((ppr_gather<W, true>), dim3(G), dim3(BLK), 0, st, a);
+        else hipLaunchKernelGGL((ppr_gather<W, false>), dim3(G), dim3(BLK), 0, st, a);
+        from = a.D;
     }
+    MG_HIP(hipGetLastError());
+    if (from == spare) p.cur ^= 1;
     return MG_OK;
 }
 

@@ -297,3 +297,40 @@ def test_pagerank_list_lengths(mg, oracle, device, n, hubs, relabel):
     exp, it = oracle.pr_gas(g.row_offsets, g.col_idx)
     assert abs(st.iterations - it) <= 1
     assert np.max(np.abs(got.astype(np.float64) - exp)) / n <= 1e-6
+
+
+# ---------------------------------------------------------------- personalized PageRank
+@pytest.mark.parametrize("relabel", [False, True])
+@pytest.mark.parametrize("n", [1500, 1537, 4096])
+def test_ppr_list_lengths(mg, oracle, device, n, relabel):
+    # in-degrees around a block's, a team's and a piece's edges; empty lists first and last
+    rng = np.random.default_rng(n)
+    low = rng.integers(0, 12, n)
+    degs = [7, 8, 9, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1400]
+    low[rng.choice(np.arange(2, n - 2), len(degs), replace=False)] = degs
+    low[[0, 1, n - 2, n - 1]] = [0, 1, 3, 0]
+    src = np.concatenate([rng.choice(n, d, replace=False) for d in low])
+    g = mg.csr_from_edges(n, src.astype(np.int32), np.repeat(np.arange(n), low).astype(np.int32), mg.MG_CSR_SORT_COLS)
+    srcs = rng.integers(0, n, 64).astype(np.int32)
+    # all terms are positive: a list's sum errs by at most 3 + 4 + 3 + 6 roundings (block, partial sum, their
+    # tree, pieces), the rank by 4 more, and 0.85 of an iteration's relative error goes into the next
+    rtol = 20 * 2.0**-24 / 0.15
+    with mg.Graph(g, build_csc=True, relabel=relabel) as dg:
+        for iters in (1, 2, 3, 20):
+            o = mg.options(ppr_iters=iters)
+            full = dg.ppr_batch(srcs, o)
+            for j in (0, 40, 63):
+                exp = oracle.ppr(g.row_offsets, g.col_idx, int(srcs[j]), iters=iters)
+                assert np.all(np.abs(full[j] - exp) <= rtol * exp + 1e-37)
+            for k in (1, 8, 9, 16, 17, 32, 33):  # the other row widths
+                assert np.array_equal(dg.ppr_batch(srcs[:k], o).view(np.int32), full[:k].view(np.int32))
+
+
+@pytest.mark.parametrize("edges", [0, 1, 2, 3, 4, 5, 9])
+def test_ppr_tiny_adjacency(mg, oracle, device, edges):
+    # fewer edges than the loads of a block are wide
+    src, dst = np.arange(edges, dtype=np.int32), np.arange(1, edges + 1, dtype=np.int32)
+    g = mg.csr_from_edges(edges + 2, src, dst, 0)
+    with mg.Graph(g, build_csc=True) as dg:
+        for s, got in enumerate(dg.ppr_batch(np.arange(min(edges + 2, 8), dtype=np.int32))):
+            assert np.max(np.abs(got - oracle.ppr(g.row_offsets, g.col_idx, s))) <= 1e-6
