@@ -699,7 +699,8 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
     };
     const int64_t max_steps = std::min<int64_t>((int64_t)o.iter_num, (int64_t)g->n) + 3;
     bool tail_queued = false;
-    auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, -1, ws.vals, 4 * (size_t)g->n); };
+    const Delivery to = plan_delivery(g, depth_out, 4 * (size_t)g->n, o.out_on_device);
+    auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, -1, ws.vals, 4 * (size_t)g->n, to); };
     auto team = [&]() -> int {
         const int trc = ensure_team(g);
         if (trc) return trc;
@@ -711,8 +712,7 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
     if ((rc = drive(g, step, max_steps, KIND_BFS, mix64((uint64_t)o.directed + 2 * (uint64_t)a.G), nullptr, nullptr,
                     tail, &tail_queued, team)))
         return rc;
-    rc = finish_search(g, stats, ws.vals, -1, depth_out, ws.vals, 4 * (size_t)g->n, o.out_on_device, timer,
-                       tail_queued);
+    rc = finish_search(g, stats, ws.vals, -1, ws.vals, 4 * (size_t)g->n, to, timer, tail_queued);
     if (rc == MG_OK && o.verbose) rc = print_trace(g, "bfs", "top-down", "bottom-up");
     return rc;
 }

@@ -264,5 +264,6 @@ extern "C" int mg_cc(mg_graph *g, int32_t *label_out, const mg_options *opt, mg_
     hipLaunchKernelGGL(cc_compress, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
     hipLaunchKernelGGL(cc_done, dim3(1), dim3(1), 0, g->stream, ws.ctl);
     MG_HIP(hipGetLastError());
-    return finish_search(g, stats, ws.vals, -1, label_out, ws.vals, 4 * (size_t)g->n, o.out_on_device, timer);
+    return finish_search(g, stats, ws.vals, -1, ws.vals, 4 * (size_t)g->n,
+                         plan_delivery(g, label_out, 4 * (size_t)g->n, o.out_on_device), timer);
 }

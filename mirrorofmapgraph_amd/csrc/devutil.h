@@ -76,6 +76,27 @@ __device__ __forceinline__ int block_exclusive_scan(int x, int *s_wave, int *tot
     return wave_off + incl - x;
 }
 
+// True in every thread of the workgroup that comes here last of the launch's (each comes
+// once, its thread 0 having waited for what it stored for that one).  cnt: LAST_WG_INTS
+// zeros, which it leaves zero; counted in groups, as 512 workgroups on one counter take 6 us.
+constexpr int LAST_WG_GROUPS = 32, LAST_WG_INTS = 16 + 16 * LAST_WG_GROUPS;
+__device__ __forceinline__ bool last_workgroup(int *cnt) {
+    __shared__ int s_last;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int grp = blockIdx.x % LAST_WG_GROUPS, members = ((int)gridDim.x - grp + LAST_WG_GROUPS - 1) / LAST_WG_GROUPS;
+        int *c = cnt + 16 + 16 * grp;
+        s_last = 0;
+        if (atomicAdd(c, 1) == members - 1) {
+            *c = 0;
+            s_last = atomicAdd(cnt, 1) == min((int)gridDim.x, LAST_WG_GROUPS) - 1;
+            if (s_last) *cnt = 0;
+        }
+    }
+    __syncthreads();
+    return s_last;
+}
+
 // p[i] when ok, else dflt, with the load made unconditional (from p[safe] when !ok;
 // safe must be in bounds).  A conditional load compiles to a branch that waits for
 // the load before the next one; loads written this way issue back to back, so a

@@ -36,6 +36,7 @@ constexpr int SMALL_BIG = SMALL_E / (LANE_T + 1) + 1;  // lists > LANE_T in a fr
 
 enum { DIR_TD = 0, DIR_BU = 1 };
 
+constexpr int TAIL_WGS = 256;     // workgroups of what follows a search, at most
 constexpr int MAX_GRID = 2048;    // workgroups of a multi-workgroup launch (256 CUs x 8)
 constexpr int BIG_GRID = 8192;    // SSSP level and CC kernels: more workgroups hide their gather latency
 
@@ -109,7 +110,10 @@ struct Workspace {
     Ctl *ctl = nullptr;
     Ctl *h_ctl = nullptr;     // pinned host mirror
     unsigned long long *h_reach = nullptr;  // pinned: TEPS count and reached vertices of a result
-    unsigned long long *d_reach = nullptr;  // their device accumulators
+    unsigned long long *d_reach = nullptr;  // their device partial sums, two a workgroup
+    int *tail_cnt = nullptr;                // counters of the workgroups that added theirs
+    Ctl *h_ctl_dev = nullptr;               // h_ctl and h_reach as the device addresses them
+    unsigned long long *h_reach_dev = nullptr;
     // PageRank state (allocated on first use)
     float *rank = nullptr;
     float *contrib[2] = {nullptr, nullptr};
@@ -406,10 +410,11 @@ int mg::drive(mg_graph *g, Step step, int64_t max_steps, int kind, uint64_t key,
             // the search most likely ends here: queue its tail before the wait (if not,
             // the caller queues it again after the remaining steps)
             if (tail_queued) {
-                const int trc = tail();
+                const int trc = tail();  // brings the control block along
                 if (trc) return trc;
+            } else {
+                MG_HIP(hipMemcpyAsync(h_ctl, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, g->stream));
             }
-            MG_HIP(hipMemcpyAsync(h_ctl, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, g->stream));
             MG_HIP(hipStreamSynchronize(g->stream));
             if (h_ctl->done == 1) {
                 finish();

@@ -85,6 +85,7 @@ static void free_workspace(Workspace &ws) {
     if (ws.h_ctl) (void)hipHostFree(ws.h_ctl);
     if (ws.h_reach) (void)hipHostFree(ws.h_reach);
     dfree(ws.d_reach);
+    dfree(ws.tail_cnt);
     dfree(ws.rank);
     dfree(ws.contrib[0]);
     dfree(ws.contrib[1]);
@@ -116,13 +117,17 @@ int ensure_workspace(mg_graph *g) {
         (rc = dalloc(&ws.q[2], n)) || (rc = dalloc(&ws.hard, n)) || (rc = dalloc(&ws.visited, ws.nwords)) ||
         (rc = dalloc(&ws.bm[0], ws.nwords)) || (rc = dalloc(&ws.bm[1], ws.nwords)) ||
         (rc = dalloc(&ws.bm[2], ws.nwords)) || (rc = dalloc(&ws.chunks, ws.chunk_cap)) ||
-        (rc = dalloc(&ws.part, 3 * BIG_GRID)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2)) ||
+        (rc = dalloc(&ws.part, 3 * BIG_GRID)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2 * TAIL_WGS)) ||
+        (rc = dalloc(&ws.tail_cnt, LAST_WG_INTS)) ||
         (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP))) {
         free_workspace(ws);
         return rc;
     }
     hipError_t e = hipHostMalloc((void **)&ws.h_ctl, sizeof(Ctl), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void **)&ws.h_reach, 2 * sizeof(unsigned long long), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&ws.h_ctl_dev, ws.h_ctl, 0);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&ws.h_reach_dev, ws.h_reach, 0);
+    if (e == hipSuccess) e = hipMemsetAsync(ws.tail_cnt, 0, 4 * LAST_WG_INTS, g->stream);
     if (e != hipSuccess) {
         free_workspace(ws);
         return set_error(MG_ERR_OOM, "hipHostMalloc failed: %s", hipGetErrorString(e));

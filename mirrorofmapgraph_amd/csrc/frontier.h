@@ -653,10 +653,24 @@ int ensure_dense_tasks(mg_graph *g, const int *d_in_off);
 // Prints the per-level trace of the search that just finished to stderr (the
 // reference's verbose per-iteration frontier sizes).
 int print_trace(mg_graph *g, const char *what, const char *dir0, const char *dir1);
+// Where a result goes.  by_kernel: device memory of the graph's own device, written by the
+// kernels that end the search; early: host memory, copied ahead of the wait that the search
+// ends with, up to EARLY_BYTES (that wait may come before the search is over, and the copy is
+// then made again).  Otherwise it is copied after the wait.
+constexpr size_t EARLY_BYTES = 1 << 20;
+struct Delivery {
+    void *out = nullptr;
+    bool on_device = false, by_kernel = false, early = false;
+};
+Delivery plan_delivery(const mg_graph *g, void *out, size_t bytes, bool out_on_device);
 // Queues what follows a finished search: the result back to the caller's ids (a twin's
-// search), the closing event and, with_stats, the TEPS count over vals.
-int queue_finish(mg_graph *g, bool with_stats, const int *vals, int unreached, const void *result, size_t bytes);
-int finish_search(mg_graph *g, mg_stats *stats, const int *vals, int unreached, void *out, const void *result,
-                  size_t bytes, bool out_on_device, const CallTimer &timer, bool tail_queued = false);
+// search), the closing event, the control block and, with_stats, the TEPS count over vals
+// into their pinned copies, and the result to where `to` has it now.
+int queue_finish(mg_graph *g, bool with_stats, const int *vals, int unreached, const void *result, size_t bytes,
+                 const Delivery &to);
+// Does that unless the search's steps were followed by it (tail_queued), waits, and fills
+// *stats; vals (nullable) is the int result that the TEPS count reads.
+int finish_search(mg_graph *g, mg_stats *stats, const int *vals, int unreached, const void *result, size_t bytes,
+                  const Delivery &to, const CallTimer &timer, bool tail_queued = false);
 
 }  // namespace mg

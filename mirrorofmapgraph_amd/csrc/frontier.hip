@@ -146,34 +146,68 @@ int ensure_dense_tasks(mg_graph *g, const int *d_in_off) {
     return MG_OK;
 }
 
-// Reference TEPS count (bfs.cu:483-493) and reached-vertex count over a result
-// array: sum of CSR out-degrees of vertices whose value differs from `unreached`.
-__global__ __launch_bounds__(1024) void reached_stats(const int *vals, int unreached, const int *row_off, int n,
-                                                      unsigned long long *out) {
+// What follows a search, in one launch: the control block to its pinned copy, the result
+// `vals` copied to `out` (nullable), and, with `off`, the reference TEPS count
+// (bfs.cu:483-493) and the reached vertices: the sum of CSR out-degrees of vertices whose
+// value differs from `unreached`, and their number, to the pinned h_reach.
+// Bound: launches and the wait.  With a fill, the count, copies of both, a wait and a copy of
+// the result one after another a call took, us: CC of 4.2M vertices 216, BFS of 2.1M 229, of
+// 65 thousand to the host 167; in one launch ahead of the wait 190, 204 and 157.
+struct TailArgs {
+    const Ctl *ctl;
+    Ctl *h_ctl;
+    const int *vals, *off;
+    int *out;
+    unsigned long long *part, *h_reach;
+    int *cnt;
+    int n, unreached;
+};
+
+__global__ __launch_bounds__(1024) void search_tail(TailArgs a) {
+    static_assert(sizeof(Ctl) % 4 == 0, "copied by words");
+    if (blockIdx.x == 0 && threadIdx.x < sizeof(Ctl) / 4)
+        reinterpret_cast<int *>(a.h_ctl)[threadIdx.x] = reinterpret_cast<const int *>(a.ctl)[threadIdx.x];
+    if (!a.out && !a.off) return;
+    constexpr int K = 4;  // vertices in flight
+    const int nt = gridDim.x * blockDim.x;
     long long te = 0, nr = 0;
-    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
-        if (vals[v] != unreached) {
-            te += row_off[v + 1] - row_off[v];
-            nr++;
+    for (int64_t base = blockIdx.x * blockDim.x + threadIdx.x; base < a.n; base += (int64_t)K * nt) {
+        int x[K], d[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int64_t v = min(base + (int64_t)k * nt, (int64_t)a.n - 1);
+            x[k] = a.vals[v];
+            d[k] = a.off ? a.off[v + 1] - a.off[v] : 0;
         }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int64_t v = base + (int64_t)k * nt;
+            if (v >= a.n) continue;
+            if (a.out) a.out[v] = x[k];
+            te += x[k] != a.unreached ? d[k] : 0;
+            nr += x[k] != a.unreached;
+        }
+    }
+    if (!a.off) return;
     te = block_sum<1024>(te);
     nr = block_sum<1024>(nr);
-    if (threadIdx.x == 0) {  // one atomic per workgroup (at most 256 workgroups)
-        if (te) atomicAdd(&out[0], (unsigned long long)te);
-        if (nr) atomicAdd(&out[1], (unsigned long long)nr);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&a.part[2 * blockIdx.x], (unsigned long long)te, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&a.part[2 * blockIdx.x + 1], (unsigned long long)nr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-}
-
-// Queues the TEPS count over `vals` on the graph's stream; the two counts land in the
-// pinned ws.h_reach once the stream has drained.
-static int queue_reached_stats(mg_graph *g, const int *vals, int unreached) {
-    unsigned long long *d = g->ws.d_reach;
-    MG_HIP(hipMemsetAsync(d, 0, 16, g->stream));
-    const int blocks = std::min(256, std::max(1, (g->n + 1023) / 1024));
-    hipLaunchKernelGGL(reached_stats, dim3(blocks), dim3(1024), 0, g->stream, vals, unreached, g->row_off, g->n, d);
-    MG_HIP(hipGetLastError());
-    MG_HIP(hipMemcpyAsync(g->ws.h_reach, d, 16, hipMemcpyDeviceToHost, g->stream));
-    return MG_OK;
+    if (!last_workgroup(a.cnt)) return;
+    te = nr = 0;
+    if (threadIdx.x < gridDim.x) {
+        te = (long long)__hip_atomic_load(&a.part[2 * threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        nr = (long long)__hip_atomic_load(&a.part[2 * threadIdx.x + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    te = block_sum<1024>(te);
+    nr = block_sum<1024>(nr);
+    if (threadIdx.x == 0) {
+        a.h_reach[0] = (unsigned long long)te;
+        a.h_reach[1] = (unsigned long long)nr;
+    }
 }
 
 int print_trace(mg_graph *g, const char *what, const char *dir0, const char *dir1) {
@@ -193,9 +227,6 @@ int print_trace(mg_graph *g, const char *what, const char *dir0, const char *dir
     return MG_OK;
 }
 
-// Records the closing event, fills *stats from the control block and copies
-// `bytes` of the device result `result` to `out`.  `vals` (nullable) is the int
-// result the TEPS count reads.
 // out[v] = vals[perm[v]]: a result of the degree-ordered twin in the caller's numbering
 __global__ void unpermute_vals(const int *perm, const int *vals, int n, int *out) {
     for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) out[v] = vals[perm[v]];
@@ -208,27 +239,65 @@ int launch_unpermute(const int *perm, const void *vals, int n, void *out, hipStr
     return MG_OK;
 }
 
-int queue_finish(mg_graph *g, bool with_stats, const int *vals, int unreached, const void *result, size_t bytes) {
-    if (g->perm && result && bytes == 4 * (size_t)g->n) {
+Delivery plan_delivery(const mg_graph *g, void *out, size_t bytes, bool out_on_device) {
+    Delivery d;
+    d.out = out;
+    d.on_device = out_on_device;
+    if (!out) return d;
+    if (!out_on_device) {
+        d.early = bytes <= EARLY_BYTES;
+        return d;
+    }
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, out) != hipSuccess) {
+        (void)hipGetLastError();  // not memory the runtime knows
+        return d;
+    }
+    d.by_kernel = at.type == hipMemoryTypeDevice && at.device == g->device && (uintptr_t)out % 4 == 0;
+    return d;
+}
+
+int queue_finish(mg_graph *g, bool with_stats, const int *vals, int unreached, const void *result, size_t bytes,
+                 const Delivery &to) {
+    Workspace &ws = g->ws;
+    const bool twin = g->perm && result && bytes == 4 * (size_t)g->n;
+    if (twin) {
         // a search on a twin: its per-vertex result (int32 or float) goes back to the caller's ids
-        hipLaunchKernelGGL(unpermute_vals, dim3(grid_blocks_cap(g->n, BLK, 4 * MAX_GRID)), dim3(BLK), 0, g->stream,
-                           g->perm, (const int *)result, g->n, g->unperm);
-        MG_HIP(hipGetLastError());
+        const int rc = launch_unpermute(g->perm, result, g->n, to.by_kernel ? to.out : g->unperm, g->stream);
+        if (rc) return rc;
+        result = g->unperm;
     }
     MG_HIP(hipEventRecord(g->ev1, g->stream));  // the end of the timed search
-    if (with_stats && vals) return queue_reached_stats(g, vals, unreached);
+    TailArgs a{};
+    a.ctl = ws.ctl;
+    a.h_ctl = ws.h_ctl_dev;
+    a.n = g->n;
+    if (with_stats && vals) {
+        a.vals = vals;
+        a.off = g->row_off;
+        a.unreached = unreached;
+        a.part = ws.d_reach;
+        a.h_reach = ws.h_reach_dev;
+        a.cnt = ws.tail_cnt;
+    }
+    if (!twin && to.by_kernel) {
+        a.vals = (const int *)result;
+        a.out = (int *)to.out;
+    }
+    const int blocks = a.out || a.off ? std::min(TAIL_WGS, std::max(1, (g->n + 1023) / 1024)) : 1;
+    hipLaunchKernelGGL(search_tail, dim3(blocks), dim3(1024), 0, g->stream, a);
+    MG_HIP(hipGetLastError());
+    if (to.early) MG_HIP(hipMemcpyAsync(to.out, result, bytes, hipMemcpyDeviceToHost, g->stream));
     return MG_OK;
 }
 
-int finish_search(mg_graph *g, mg_stats *stats, const int *vals, int unreached, void *out, const void *result,
-                  size_t bytes, bool out_on_device, const CallTimer &timer, bool tail_queued) {
+int finish_search(mg_graph *g, mg_stats *stats, const int *vals, int unreached, const void *result, size_t bytes,
+                  const Delivery &to, const CallTimer &timer, bool tail_queued) {
     Workspace &ws = g->ws;
     const bool reach = stats && vals;
     if (!tail_queued) {
-        // the closing event, then the control block and the TEPS count behind it: one wait
-        int rc = queue_finish(g, stats != nullptr, vals, unreached, result, bytes);
+        int rc = queue_finish(g, stats != nullptr, vals, unreached, result, bytes, to);
         if (rc) return rc;
-        MG_HIP(hipMemcpyAsync(ws.h_ctl, ws.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, g->stream));
         MG_HIP(hipStreamSynchronize(g->stream));
     }  // else drive queued the same work and waited for it
     if (g->perm && result && bytes == 4 * (size_t)g->n) result = g->unperm;
@@ -247,8 +316,10 @@ int finish_search(mg_graph *g, mg_stats *stats, const int *vals, int unreached, 
             stats->vertices_reached = (int64_t)ws.h_reach[1];
         }
     }
-    int rc = deliver(g, out, result, bytes, out_on_device);
-    if (rc) return rc;
+    if (!to.by_kernel && !to.early) {
+        const int rc = deliver(g, to.out, result, bytes, to.on_device);
+        if (rc) return rc;
+    }
     if (stats) stats->host_ms = timer.ms();
     return MG_OK;
 }

@@ -60,8 +60,6 @@ constexpr int PR_BUF = 256;         // edges of a run in LDS at a time (per wave
 // least pieces of 128 took 17 at scale 16.
 constexpr int PR_PIECES = 16384;
 constexpr int PR_PIECE_MIN = 256, PR_PIECE_MAX = 2048;
-constexpr int PR_GROUPS = 32;       // counters of finished workgroups, 16 ints apart
-constexpr int PR_LEFT = 16 + 16 * PR_GROUPS;
 // One edge in so many has to come from a hub for the copy to pay: it costs 1 us and the LDS
 // reads of every gather, a gather saved 1/230000 us.
 constexpr int PR_HUB_SHARE = 5;
@@ -135,7 +133,7 @@ __global__ void pr_init(PrArgs a, int iter_limit) {
         a.chg[1][i] = 0;
         a.chg[2][i] = 0;
     }
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.nbig + PR_LEFT; i += gridDim.x * blockDim.x) a.left[i] = 0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.nbig + LAST_WG_INTS; i += gridDim.x * blockDim.x) a.left[i] = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl_reset(a.ctl, a.n, iter_limit, a.n);
 }
 
@@ -207,7 +205,6 @@ __global__ __launch_bounds__(PR_BLK, 8) void pr_iterate(PrArgs a) {
     if (c->done) return;
     __shared__ float s_hubs[HUB ? PR_HUBS : 1];
     __shared__ float s_buf[PR_BLK / WAVE][PR_BUF];
-    __shared__ int s_last;
     const PrIter I = pr_iter(a);
     const bool all = a.mode == MG_PR_ALL || I.it == 0;
     const bool ranks = a.mode != MG_PR_ALL || a.tol_n > 0 || I.it + 1 >= c->iter_limit;
@@ -307,8 +304,7 @@ __global__ __launch_bounds__(PR_BLK, 8) void pr_iterate(PrArgs a) {
         if (mine) delta += pr_apply(a, I, w, od, s, act, ranks, nchanged);
         r = next;
     }
-    // the last workgroup closes the iteration, adding the workgroups' sums in order; it is
-    // found by groups of counters (512 workgroups on one took 6 us)
+    // the last workgroup closes the iteration, adding the workgroups' sums in order
     if (ranks) {
         delta = block_sum<PR_BLK>(delta);
         const long long nch = block_sum<PR_BLK>((long long)nchanged);
@@ -318,18 +314,7 @@ __global__ __launch_bounds__(PR_BLK, 8) void pr_iterate(PrArgs a) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int grp = blockIdx.x % PR_GROUPS, members = ((int)gridDim.x - grp + PR_GROUPS - 1) / PR_GROUPS;
-        int *cnt = a.left + a.nbig + 16 + 16 * grp;
-        s_last = 0;
-        if (atomicAdd(cnt, 1) == members - 1) {
-            *cnt = 0;
-            s_last = atomicAdd(&a.left[a.nbig], 1) == min((int)gridDim.x, PR_GROUPS) - 1;
-        }
-    }
-    __syncthreads();
-    if (!s_last) return;
+    if (!last_workgroup(a.left + a.nbig)) return;
     double l1 = 0, changed = 0;
     if (ranks) {
         for (int i = threadIdx.x; i < (int)gridDim.x; i += PR_BLK) {
@@ -340,7 +325,6 @@ __global__ __launch_bounds__(PR_BLK, 8) void pr_iterate(PrArgs a) {
         changed = block_sum<PR_BLK>(changed);
     }
     if (threadIdx.x == 0) {
-        a.left[a.nbig] = 0;
         c->dsum = l1;
         c->level = I.it + 1;
         c->changed = (int)changed;
@@ -405,7 +389,7 @@ static int pr_buckets(mg_graph *g, const int *d_in_off, const int *d_in_adj) {
     ch.insert(ch.end(), mid.begin(), mid.end());
     if ((rc = alloc_chunks(&ws.pr_lists, ch.size())) || (rc = alloc_i32(&ws.pr_bigv, bigv.size())) ||
         (rc = alloc_f32(&ws.pr_part, nchunks)) || (rc = alloc_i32(&ws.pr_pact, nchunks)) ||
-        (rc = alloc_i32(&ws.pr_left, bigv.size() + PR_LEFT)) || (rc = alloc_chunks(&ws.pr_runs, runs.size())))
+        (rc = alloc_i32(&ws.pr_left, bigv.size() + LAST_WG_INTS)) || (rc = alloc_chunks(&ws.pr_runs, runs.size())))
         return rc;
     // the share of the edges whose source is among the first PR_HUBS ids
     MG_HIP(hipMemsetAsync(ws.d_reach, 0, 16, g->stream));
@@ -499,7 +483,8 @@ extern "C" int mg_pagerank(mg_graph *g, float *rank_out, const mg_options *opt, 
                        (uint64_t)__builtin_bit_cast(uint64_t, a.tol_n), (uint64_t)(uintptr_t)in_off})
         key = mix64(key ^ x);
     if ((rc = drive(g, step, (int64_t)std::max(o.iter_num, 0) + 1, KIND_PR, key))) return rc;
-    rc = finish_search(g, stats, nullptr, 0, rank_out, ws.rank, 4 * (size_t)g->n, o.out_on_device, timer);
+    rc = finish_search(g, stats, nullptr, 0, ws.rank, 4 * (size_t)g->n,
+                       plan_delivery(g, rank_out, 4 * (size_t)g->n, o.out_on_device), timer);
     if (rc) return rc;
     if (stats) {
         stats->edges_traversed = g->m * (int64_t)stats->iterations;

@@ -1232,7 +1232,8 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     key = mix64(key ^ (uint64_t)a.bucket_edges);
     key = mix64(key ^ (uint64_t)a.G);
     bool tail_queued = false;
-    auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, INT_MAX, ws.vals, 4 * (size_t)g->n); };
+    const Delivery to = plan_delivery(g, dist_out, 4 * (size_t)g->n, o.out_on_device);
+    auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, INT_MAX, ws.vals, 4 * (size_t)g->n, to); };
     auto team = [&]() -> int {
         const int trc = ensure_team(g);
         if (trc) return trc;
@@ -1243,8 +1244,7 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     };
     if ((rc = drive(g, step, max_steps, KIND_SSSP, key, nullptr, nullptr, tail, &tail_queued, team)))
         return rc;
-    rc = finish_search(g, stats, ws.vals, INT_MAX, dist_out, ws.vals, 4 * (size_t)g->n, o.out_on_device, timer,
-                       tail_queued);
+    rc = finish_search(g, stats, ws.vals, INT_MAX, ws.vals, 4 * (size_t)g->n, to, timer, tail_queued);
     if (rc == MG_OK && o.verbose) rc = print_trace(g, "sssp", "push", "pull");
     return rc;
 }

@@ -334,3 +334,56 @@ def test_ppr_tiny_adjacency(mg, oracle, device, edges):
     with mg.Graph(g, build_csc=True) as dg:
         for s, got in enumerate(dg.ppr_batch(np.arange(min(edges + 2, 8), dtype=np.int32))):
             assert np.max(np.abs(got - oracle.ppr(g.row_offsets, g.col_idx, s))) <= 1e-6
+
+
+# ---------------------------------------------------------------- what follows a search
+@pytest.mark.parametrize("relabel", [False, True])
+@pytest.mark.parametrize("n", [1, 3, 1023, 1025, 262144, 262145, 1100003])
+def test_results_reach_every_kind_of_output(mg, oracle, device, n, relabel):
+    # vertex counts around the workgroups of the closing kernel and the host copies made ahead
+    import ctypes as C
+
+    hip = C.CDLL("libamdhip64.so")
+    dev, pin = C.c_void_p(), C.c_void_p()
+    assert hip.hipMalloc(C.byref(dev), C.c_size_t(4 * n + 8)) == 0
+    assert hip.hipHostMalloc(C.byref(pin), C.c_size_t(4 * n), 0) == 0
+    g = random_graph(mg, n, 3 * n, seed=n, symmetric=True, wmax=9)
+    srcs = [int(np.argmax(g.degrees())), 0, n - 1]  # searches of other lengths than the last one's
+    with mg.Graph(g, symmetric=True, relabel=relabel) as dg:
+        def outputs(name, *args):
+            fn, st = getattr(mg.lib(), name), mg.Stats()
+
+            def call(ptr, on_device, stats):
+                o = mg.options(out_on_device=on_device, pr_mode=mg.MG_PR_ALL, iter_num=5 if name == "mg_pagerank" else 100000)
+                mg.check(fn(dg.handle, *args, C.c_void_p(ptr), C.byref(o), C.byref(st) if stats else None))
+
+            host, bare, raw = np.empty(n, np.int32), np.empty(n, np.int32), np.empty(4 * n + 8, np.uint8)
+            call(host.ctypes.data, 0, True)
+            call(bare.ctypes.data, 0, False)
+            call(pin.value, 0, True)
+            assert np.array_equal(bare, host)
+            assert np.array_equal(np.ctypeslib.as_array(C.cast(pin, C.POINTER(C.c_int32)), (n,)), host)
+            for at, stats in ((4, True), (4, False), (1, True)):  # (odd addresses too)
+                raw[:] = 0xA5
+                assert hip.hipMemcpy(dev, raw.ctypes.data_as(C.c_void_p), C.c_size_t(raw.nbytes), 1) == 0
+                call(dev.value + at, 1, stats)
+                assert hip.hipMemcpy(raw.ctypes.data_as(C.c_void_p), dev, C.c_size_t(raw.nbytes), 2) == 0
+                assert np.array_equal(raw[at:at + 4 * n].copy().view(np.int32), host)
+                assert np.all(raw[:at] == 0xA5) and np.all(raw[at + 4 * n:] == 0xA5)
+            call(None, 0, True)
+            return host, st
+
+        for src in srcs:
+            d, st = outputs("mg_bfs", src)
+            assert np.array_equal(d, oracle.bfs(g.row_offsets, g.col_idx, src))
+            assert st.vertices_reached == int((d >= 0).sum())
+            assert st.edges_traversed == oracle.teps_edges(g.row_offsets, d)
+            d, st = outputs("mg_sssp", src)
+            assert np.array_equal(d, oracle.sssp(g.row_offsets, g.col_idx, g.values, src))
+            assert st.edges_traversed == oracle.teps_edges(g.row_offsets, d, 2**31 - 1)
+        d, st = outputs("mg_cc")
+        assert np.array_equal(d, oracle.cc(g.row_offsets, g.col_idx))
+        assert (st.vertices_reached, st.edges_traversed) == (n, g.m)
+        outputs("mg_pagerank")
+    hip.hipFree(dev)
+    hip.hipHostFree(pin)
