@@ -21,6 +21,12 @@
 //      vertex outside C is seen from the outside end, adjacency being symmetric);
 //   4. compress: label[v] = root(v).
 // Other graphs unite every CSR edge, which gives the weak components.
+//
+// Bound, R-MAT scale 22 (4.2M vertices, 128M edges): the lines that hold the first two
+// neighbours, which one pass reads and leaves to the other in 4 bytes a vertex (29 + 53 us
+// where each read them, 35 + 31 so); then walks to the roots (17, 11 and 8 us).  Sampling in a
+// launch of its own took 5 us, tiles without an edge to unite 6, a launch to end the search 4;
+// a call took 216 us, now 154.
 #include "frontier.h"
 
 namespace mg {
@@ -90,27 +96,32 @@ __global__ void cc_init(FrontierArgs fa, int *p) {
 // min(v, first neighbour of v).  Only the thread of v writes parent[v] here, and every
 // parent points to a smaller id or to itself, so the pointers form a forest whose
 // roots are minima without any compare-and-swap.  A first neighbour larger than v
-// is united in the second pass.
-__global__ void cc_link_first(FrontierArgs fa, int *p) {
+// is united in the second pass.  next[v] keeps what that pass unites v with: its second
+// neighbour, -1 for none, -2 for the first neighbour as well (looked up again).
+__global__ void cc_link_first(FrontierArgs fa, int *p, int *next) {
     const int *off = fa.off[0], *adj = fa.adj[0];
     for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < fa.n; v += gridDim.x * blockDim.x) {
-        const int e = off[v];
-        p[v] = e < off[v + 1] ? min(v, adj[e]) : v;
+        const int e = off[v], d = off[v + 1] - e;
+        const int u0 = d > 0 ? adj[e] : v, u1 = d > 1 ? adj[e + 1] : -1;
+        p[v] = min(v, u0);
+        next[v] = u0 > v ? -2 : u1;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl_reset(fa.ctl, fa.n, 1, fa.n);
 }
 
 // Afforest step 1, second pass: the first neighbour where it is larger than v, and
 // the second neighbour, by union-find.
-__global__ void cc_link_second(FrontierArgs fa, int *p) {
+__global__ void cc_link_second(FrontierArgs fa, int *p, const int *next) {
     const int *off = fa.off[0], *adj = fa.adj[0];
     for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < fa.n; v += gridDim.x * blockDim.x) {
-        const int e = off[v], end = off[v + 1];
-        if (e < end) {
-            const int u0 = adj[e];
-            if (u0 > v) uf_unite(p, v, u0);
-            if (e + 1 < end) uf_unite(p, v, adj[e + 1]);
+        int u = next[v];
+        if (u == -1) continue;
+        if (u == -2) {
+            const int e = off[v];
+            uf_unite(p, v, adj[e]);
+            u = e + 1 < off[v + 1] ? adj[e + 1] : v;
         }
+        if (ld_parent(p, v) != ld_parent(p, u)) uf_unite(p, v, u);
     }
 }
 
@@ -123,46 +134,45 @@ __global__ void cc_link_round(FrontierArgs fa, int *p, int r) {
     }
 }
 
-__global__ void cc_compress(FrontierArgs fa, int *p) {
-    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < fa.n; v += gridDim.x * blockDim.x) {
-        int r = v;
-        for (int pr = p[r]; pr != r; pr = p[r]) r = pr;
-        p[v] = r;
-    }
-}
-
 // Afforest step 2: most frequent root among CC_SAMPLES hashed vertices (one
 // workgroup; roots counted in an LDS hash table, then the largest count, ties to the
 // smaller root).  Which component is skipped only decides the work of step 3, not the
 // labels.
-__global__ __launch_bounds__(CC_SAMPLES) void cc_sample(FrontierArgs fa, const int *p, uint64_t seed) {
+__device__ __forceinline__ int cc_root(const int *p, int r) {
+    for (int pr = p[r]; pr != r; pr = p[r]) r = pr;
+    return r;
+}
+
+__device__ __forceinline__ void cc_sample(Ctl *ctl, int n, const int *p, uint64_t seed) {
     constexpr int H = 2 * CC_SAMPLES;
     __shared__ int s_key[H];
     __shared__ int s_cnt[H];
-    __shared__ unsigned long long s_best[CC_SAMPLES / WAVE];
+    __shared__ unsigned long long s_best[BLK / WAVE];
     const int t = threadIdx.x;
-    for (int i = t; i < H; i += CC_SAMPLES) {
+    for (int i = t; i < H; i += BLK) {
         s_key[i] = -1;
         s_cnt[i] = 0;
     }
-    uint64_t h = (seed + (uint64_t)t * 0x9e3779b97f4a7c15ULL);
-    h = (h ^ (h >> 30)) * 0xbf58476d1ce4e5b9ULL;
-    h = (h ^ (h >> 27)) * 0x94d049bb133111ebULL;
-    h ^= h >> 31;
-    const int r = p[(int)(h % (uint64_t)fa.n)];
     __syncthreads();
-    // insert r (linear probing; at most CC_SAMPLES distinct keys in 2 * CC_SAMPLES slots)
-    uint32_t slot = ((uint32_t)r * 2654435761u) % H;
-    for (;;) {
-        const int old = atomicCAS(&s_key[slot], -1, r);
-        if (old == -1 || old == r) break;
-        slot = (slot + 1) % H;
+    for (int i = t; i < CC_SAMPLES; i += BLK) {
+        uint64_t h = (seed + (uint64_t)i * 0x9e3779b97f4a7c15ULL);
+        h = (h ^ (h >> 30)) * 0xbf58476d1ce4e5b9ULL;
+        h = (h ^ (h >> 27)) * 0x94d049bb133111ebULL;
+        h ^= h >> 31;
+        const int r = cc_root(p, (int)(h % (uint64_t)n));
+        // insert r (linear probing; at most CC_SAMPLES distinct keys in 2 * CC_SAMPLES slots)
+        uint32_t slot = ((uint32_t)r * 2654435761u) % H;
+        for (;;) {
+            const int old = atomicCAS(&s_key[slot], -1, r);
+            if (old == -1 || old == r) break;
+            slot = (slot + 1) % H;
+        }
+        atomicAdd(&s_cnt[slot], 1);
     }
-    atomicAdd(&s_cnt[slot], 1);
     __syncthreads();
     // the largest (count, -root) over the slots
     unsigned long long best = 0;
-    for (int i = t; i < H; i += CC_SAMPLES)
+    for (int i = t; i < H; i += BLK)
         if (s_cnt[i] > 0) {
             const unsigned long long k = ((unsigned long long)s_cnt[i] << 32) | (0xFFFFFFFFu - (uint32_t)s_key[i]);
             best = k > best ? k : best;
@@ -175,9 +185,26 @@ __global__ __launch_bounds__(CC_SAMPLES) void cc_sample(FrontierArgs fa, const i
     if ((t & (WAVE - 1)) == 0) s_best[t / WAVE] = best;
     __syncthreads();
     if (t == 0) {
-        for (int w = 1; w < CC_SAMPLES / WAVE; ++w) best = s_best[w] > best ? s_best[w] : best;
-        fa.ctl->aux = (int)(0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFu));  // the skipped component's root
-        fa.ctl->nf_prev = (int)(best >> 32);
+        for (int w = 1; w < BLK / WAVE; ++w) best = s_best[w] > best ? s_best[w] : best;
+        ctl->aux = (int)(0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFu));  // the skipped component's root
+        ctl->nf_prev = (int)(best >> 32);
+    }
+}
+
+// label[v] = root(v) for every v; p itself, or another array.  The workgroup that samples
+// does so beside the others: pointers move to ancestors while it walks them, and roots stay.
+template <bool SAMPLE>
+__global__ __launch_bounds__(BLK) void cc_compress(FrontierArgs fa, const int *p, int *label) {
+    if (SAMPLE && blockIdx.x == 0) cc_sample(fa.ctl, fa.n, p, 0x5eed);
+    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < fa.n; v += gridDim.x * blockDim.x) label[v] = cc_root(p, v);
+}
+
+// The last compress, which ends the search too.
+__global__ __launch_bounds__(BLK) void cc_labels(FrontierArgs fa, const int *p, int *label) {
+    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < fa.n; v += gridDim.x * blockDim.x) label[v] = cc_root(p, v);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        fa.ctl->level = 1;
+        fa.ctl->done = 1;
     }
 }
 
@@ -194,7 +221,7 @@ __global__ __launch_bounds__(BLK) void cc_finish(FrontierArgs fa, int *p) {
             beg = off[v] + CC_SAMPLE_ROUNDS;
             deg = max(0, off[v + 1] - beg);
         }
-        expand_tile_range<BLK, true>(fa, pol, 0, 0, v < fa.n ? v : -1, beg, deg, no_emit);
+        if (__syncthreads_or(deg > 0)) expand_tile_range<BLK, true>(fa, pol, 0, 0, v < fa.n ? v : -1, beg, deg, no_emit);
     }
 }
 
@@ -211,11 +238,6 @@ __global__ __launch_bounds__(BLK) void cc_hook(FrontierArgs fa, int *p) {
 __global__ __launch_bounds__(BLK) void cc_hook_chunks(FrontierArgs fa, int *p) {
     CcPolicy pol{p, false};
     expand_chunks<BLK>(fa, pol, 0);
-}
-
-__global__ void cc_done(Ctl *c) {
-    c->level = 1;
-    c->done = 1;
 }
 
 }  // namespace mg
@@ -239,31 +261,35 @@ extern "C" int mg_cc(mg_graph *g, int32_t *label_out, const mg_options *opt, mg_
     int *p = ws.vals;
     const int G = grid_blocks_cap(std::max<int64_t>(g->n / 4, g->m / 64), BLK, BIG_GRID);
     const int Gn = grid_blocks_cap(g->n, BLK, BIG_GRID);
+    const Delivery to = plan_delivery(g, label_out, 4 * (size_t)g->n, o.out_on_device);
     MG_HIP(hipEventRecord(g->ev0, g->stream));
     if ((g->flags & MG_GRAPH_SYMMETRIC) && o.engine != MG_ENGINE_GAS && g->n > 0) {
         if (g->m >= (int64_t)CC_PLAIN_FIRST_DEGREE * g->n) {
-            hipLaunchKernelGGL(cc_link_first, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
-            hipLaunchKernelGGL(cc_compress, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
-            hipLaunchKernelGGL(cc_link_second, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
-            hipLaunchKernelGGL(cc_compress, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
+            int *next = ws.q[0];
+            hipLaunchKernelGGL(cc_link_first, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, next);
+            hipLaunchKernelGGL(cc_compress<false>, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, p);
+            hipLaunchKernelGGL(cc_link_second, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, next);
         } else {
             hipLaunchKernelGGL(cc_init, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
-            for (int r = 0; r < CC_SAMPLE_ROUNDS; ++r) {
-                hipLaunchKernelGGL(cc_link_round, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, r);
-                hipLaunchKernelGGL(cc_compress, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
-            }
+            hipLaunchKernelGGL(cc_link_round, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, 0);
+            hipLaunchKernelGGL(cc_compress<false>, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, p);
+            hipLaunchKernelGGL(cc_link_round, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, 1);
         }
-        hipLaunchKernelGGL(cc_sample, dim3(1), dim3(CC_SAMPLES), 0, g->stream, fa, (const int *)p,
-                           (uint64_t)0x5eed);
+        hipLaunchKernelGGL(cc_compress<true>, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, p);
         hipLaunchKernelGGL(cc_finish, dim3(G), dim3(BLK), 0, g->stream, fa, p);
     } else {
         hipLaunchKernelGGL(cc_init, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
         hipLaunchKernelGGL(cc_hook, dim3(G), dim3(BLK), 0, g->stream, fa, p);
     }
-    hipLaunchKernelGGL(cc_hook_chunks, dim3(G), dim3(BLK), 0, g->stream, fa, p);
-    hipLaunchKernelGGL(cc_compress, dim3(Gn), dim3(BLK), 0, g->stream, fa, p);
-    hipLaunchKernelGGL(cc_done, dim3(1), dim3(1), 0, g->stream, ws.ctl);
+    hipLaunchKernelGGL(cc_hook_chunks, dim3(std::min(G, MAX_GRID)), dim3(BLK), 0, g->stream, fa, p);
+    int *label = to.by_kernel ? (int *)to.out : p;
+    hipLaunchKernelGGL(cc_labels, dim3(Gn), dim3(BLK), 0, g->stream, fa, p, label);
     MG_HIP(hipGetLastError());
-    return finish_search(g, stats, ws.vals, -1, ws.vals, 4 * (size_t)g->n,
-                         plan_delivery(g, label_out, 4 * (size_t)g->n, o.out_on_device), timer);
+    rc = finish_search(g, stats, nullptr, 0, label, 4 * (size_t)g->n, to, timer);
+    if (rc) return rc;
+    if (stats) {  // every vertex has a label
+        stats->edges_traversed = g->m;
+        stats->vertices_reached = g->n;
+    }
+    return MG_OK;
 }

@@ -280,7 +280,7 @@ int queue_finish(mg_graph *g, bool with_stats, const int *vals, int unreached, c
         a.h_reach = ws.h_reach_dev;
         a.cnt = ws.tail_cnt;
     }
-    if (!twin && to.by_kernel) {
+    if (!twin && to.by_kernel && result != to.out) {
         a.vals = (const int *)result;
         a.out = (int *)to.out;
     }

@@ -387,3 +387,27 @@ def test_results_reach_every_kind_of_output(mg, oracle, device, n, relabel):
         outputs("mg_pagerank")
     hip.hipFree(dev)
     hip.hipHostFree(pin)
+
+
+# ---------------------------------------------------------------- connected components
+@pytest.mark.parametrize("sort", [False, True])
+@pytest.mark.parametrize("n,parts", [(40, 1), (257, 3), (5000, 7), (70001, 2), (300007, 40)])
+def test_cc_dense_components(mg, oracle, device, n, parts, sort):
+    # mean degree above 8; first neighbours above and below their vertex, lists of any order, hubs
+    # and isolated vertices outside the sampled component
+    rng = np.random.default_rng(n + sort)
+    part = rng.integers(0, parts, n)
+    ids = [np.flatnonzero(part == k) for k in range(parts)]
+    src = np.concatenate([rng.choice(i[: max(1, len(i) * 3 // 4)], 8 * len(i)) for i in ids if len(i)])
+    dst = np.concatenate([rng.choice(i[: max(1, len(i) * 3 // 4)], 8 * len(i)) for i in ids if len(i)])
+    small = min(ids, key=len)
+    src, dst = np.concatenate([src, np.full(len(small), small[0])]), np.concatenate([dst, small])  # a hub
+    flags = mg.MG_CSR_SYMMETRIZE | mg.MG_CSR_DROP_LOOPS | (mg.MG_CSR_SORT_COLS | mg.MG_CSR_DEDUPE if sort else 0)
+    g = mg.csr_from_edges(n, src.astype(np.int32), dst.astype(np.int32), flags)
+    assert g.m >= 8 * n
+    exp = oracle.cc(g.row_offsets, g.col_idx)
+    with mg.Graph(g, symmetric=True) as dg:
+        for _ in range(2):
+            got, st = dg.cc(stats=True)
+            assert np.array_equal(got, exp)
+            assert (st.vertices_reached, st.edges_traversed, st.iterations) == (n, g.m, 1)
