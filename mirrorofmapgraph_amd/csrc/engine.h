@@ -133,7 +133,7 @@ struct Workspace {
     int pull_ntasks = 0;
     const int32_t *pull_view = nullptr;
     ChunkRec *dense_tasks = nullptr;  // dense SSSP pull tasks (pieces and vertex ranges)
-    int dense_ntasks = 0;
+    int dense_ntasks = 0, dense_big = 0;
     const int32_t *dense_view = nullptr;
 };
 
@@ -252,14 +252,19 @@ int deliver(mg_graph *g, void *dst, const void *src, size_t bytes, bool out_on_d
 constexpr int STEPS_PER_GRAPH = 8;
 constexpr int TRACE_CAP = 16384;  // levels recorded in the per-level trace (verbose)
 constexpr int PULL_TASK = 512;   // static pull tasks: in-edges per wave (8 per lane in flight)
-// Dense SSSP pull tasks: in-lists longer than DENSE_BIG are cut into DENSE_T-slot
-// pieces; the other vertices are grouped into ranges of whole bitmap words (at most
-// DENSE_V vertices) holding about DENSE_T in-edges.  A range holds at most DENSE_T
-// in-edges, or a single word's (32 vertices of up to DENSE_BIG each): DENSE_RANGE_MAX.
-constexpr int DENSE_BIG = 512;
-constexpr int DENSE_T = 2048;
+// Dense SSSP pull tasks: in-lists longer than T / 4 (dense_big) are cut into pieces of T
+// slots; the other vertices are grouped into ranges of whole bitmap words (at most
+// DENSE_V vertices) holding about T in-edges, T = m / DENSE_TASKS from DENSE_T_MIN to DENSE_T.
+// A range holds at most T in-edges, or a single word's (32 vertices of up to T / 4 each):
+// DENSE_RANGE_MAX.
+// A wave walks a task in windows of two loads, so with T fixed at 2048 a level of a small
+// graph was a few waves' chains of them.  Search times, us, T = 2048 / this rule: R-MAT scale
+// 16 symmetric 306 / 267, directed 362 / 298, scale 18 414 / 388, 501 / 446; least T of 256
+// 281 and 302 at scale 16, 128 293 and 318; from scale 20 on (31M edges) T is 2048 by either.
+constexpr int DENSE_T = 2048, DENSE_T_MIN = 512;
+constexpr int DENSE_TASKS = 8192;
 constexpr int DENSE_V = 256;
-constexpr int DENSE_RANGE_MAX = DENSE_T > 32 * DENSE_BIG ? DENSE_T : 32 * DENSE_BIG;
+constexpr int DENSE_RANGE_MAX = 8 * DENSE_T;
 enum { KIND_BFS = 0, KIND_SSSP = 1, KIND_PR = 2, KIND_GAS = 3, KIND_BATCH = 4, KIND_BATCH_SSSP = 5, NKINDS = 8 };
 
 struct StepGraph {

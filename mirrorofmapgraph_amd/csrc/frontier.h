@@ -646,9 +646,9 @@ int launch_fill(mg_graph *g, int *p, int v, int64_t n);
 int launch_fill(mg_graph *g, uint32_t *p, uint32_t v, int64_t n);
 int ensure_pull_tasks(mg_graph *g, const int *d_in_off);
 // Tasks of the dense SSSP pull levels: {v, beg, end} = slots [beg, end) of the
-// in-list of a vertex v with more than DENSE_BIG in-edges (DENSE_T per piece), or
+// in-list of a vertex v with more than dense_big in-edges, or
 // {-1, va, vb} = the vertices [va, vb) (va a multiple of 32, vb too or n, at most
-// DENSE_V of them) whose in-lists are at most DENSE_BIG long, about DENSE_T edges in all.
+// DENSE_V of them) whose in-lists are at most dense_big long.
 int ensure_dense_tasks(mg_graph *g, const int *d_in_off);
 // Prints the per-level trace of the search that just finished to stderr (the
 // reference's verbose per-iteration frontier sizes).

@@ -110,12 +110,13 @@ int ensure_dense_tasks(mg_graph *g, const int *d_in_off) {
     const int n = g->n;
     std::vector<int32_t> off((size_t)n + 1);
     MG_HIP(copy_on(g->stream, off.data(), d_in_off, 4 * ((size_t)n + 1), hipMemcpyDeviceToHost));
+    const int T = (int)std::clamp<int64_t>(g->m / DENSE_TASKS / WAVE * WAVE, DENSE_T_MIN, DENSE_T), big = T / 4;
     std::vector<ChunkRec> t;
     // pieces of the long lists
     for (int v = 0; v < n; ++v)
-        if (off[v + 1] - off[v] > DENSE_BIG)
-            for (int b = off[v]; b < off[v + 1]; b += DENSE_T)
-                t.push_back(ChunkRec{v, b, std::min(b + DENSE_T, off[v + 1]), 0});
+        if (off[v + 1] - off[v] > big)
+            for (int b = off[v]; b < off[v + 1]; b += T)
+                t.push_back(ChunkRec{v, b, std::min(b + T, off[v + 1]), 0});
     // ranges of whole words over the other vertices (ranges without in-edges are dropped)
     int va = 0;
     int64_t edges = 0;
@@ -124,9 +125,9 @@ int ensure_dense_tasks(mg_graph *g, const int *d_in_off) {
         int64_t we = 0;
         for (int v = w0; v < w1; ++v) {
             const int d = off[v + 1] - off[v];
-            if (d <= DENSE_BIG) we += d;
+            if (d <= big) we += d;
         }
-        if (w0 > va && (edges + we > DENSE_T || w0 - va >= DENSE_V)) {
+        if (w0 > va && (edges + we > T || w0 - va >= DENSE_V)) {
             if (edges) t.push_back(ChunkRec{-1, va, w0, 0});
             va = w0;
             edges = 0;
@@ -142,6 +143,7 @@ int ensure_dense_tasks(mg_graph *g, const int *d_in_off) {
     if (rc) return rc;
     if (!t.empty()) MG_HIP(copy_on(g->stream, ws.dense_tasks, t.data(), sizeof(ChunkRec) * t.size(), hipMemcpyHostToDevice));
     ws.dense_ntasks = (int)t.size();
+    ws.dense_big = big;
     ws.dense_view = d_in_off;
     return MG_OK;
 }

@@ -32,7 +32,7 @@ struct SsspArgs {
     int G;                 // workgroups of the whole-GPU level kernels
     // pull levels: the dense tasks, all in one launch
     const ChunkRec *dpull;
-    int ndpull;
+    int ndpull, dense_big;
     int push_range;  // symmetric graph with dense tasks: wide push levels use range_push
     // buckets: width, far list of the small-frontier loop (n entries) and its bitmap
     long long delta;
@@ -329,7 +329,7 @@ __device__ __forceinline__ void dense_range(const SsspArgs &a, int L, int va, in
         cur[j] = a.dist[vv];
         beg[j] = o0;
         // a vertex at or below fmin + (smallest weight) cannot improve: its list is skipped
-        len[j] = in && o1 - o0 <= DENSE_BIG && fmin + a.wmin < cur[j] ? o1 - o0 : 0;
+        len[j] = in && o1 - o0 <= a.dense_big && fmin + a.wmin < cur[j] ? o1 - o0 : 0;
     }
     const int total = range_index(lds, wv, lane, beg, len, cur, rank);
     if (lane == 0) ex += total;  // the wave's edges, counted once
@@ -539,7 +539,7 @@ __device__ __forceinline__ void range_push(const SsspArgs &a, int L, DenseLds &l
             const int vv = v < vb ? v : va;
             const int o0 = off[vv], o1 = off[vv + 1];
             beg[j] = o0;
-            len[j] = v < vb && o1 - o0 <= DENSE_BIG && test_bit(fr, v) ? o1 - o0 : 0;
+            len[j] = v < vb && o1 - o0 <= a.dense_big && test_bit(fr, v) ? o1 - o0 : 0;
             dvs[j] = a.dist[vv];
         }
 #pragma unroll
@@ -1207,6 +1207,7 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
         if ((rc = ensure_dense_tasks(g, a.fa.off[2]))) return rc;
         a.dpull = ws.dense_tasks;
         a.ndpull = ws.dense_ntasks;
+        a.dense_big = ws.dense_big;
         // the tasks cut the in-lists; on a symmetric graph those are the out-lists too
         a.push_range = a.fa.off[2] == a.fa.off[0] && a.fa.nviews == 1 && a.fa.eid[0] == nullptr;
     }

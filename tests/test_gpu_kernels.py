@@ -411,3 +411,30 @@ def test_cc_dense_components(mg, oracle, device, n, parts, sort):
             got, st = dg.cc(stats=True)
             assert np.array_equal(got, exp)
             assert (st.vertices_reached, st.edges_traversed, st.iterations) == (n, g.m, 1)
+
+
+# ---------------------------------------------------------------- SSSP pull and wide push tasks
+@pytest.mark.parametrize("symmetric", [False, True])
+@pytest.mark.parametrize("n", [2000, 2049, 300001])
+def test_sssp_dense_task_sizes(mg, oracle, device, n, symmetric):
+    # in-lists around the pieces and ranges of the smallest tasks; at the last size (over 5M edges)
+    # around those of larger ones
+    rng = np.random.default_rng(n)
+    big = n > 10**5
+    low = rng.integers(0, 40 if big else 16, n)
+    t = 704 if big else 512  # edges a task (directed)
+    degs = [t // 4 - 1, t // 4, t // 4 + 1, t - 1, t, t + 1, 2 * t, 2 * t + 1]
+    low[[0, 1, n - 1, *rng.choice(np.arange(40, n - 40), 5, replace=False)]] = degs
+    low[64:96] = t // 4  # a word of the longest lists that are not cut
+    dst = np.repeat(np.arange(n), low).astype(np.int32)
+    src = rng.integers(0, n, len(dst)).astype(np.int32)
+    flags = mg.MG_CSR_SORT_COLS | (mg.MG_CSR_SYMMETRIZE if symmetric else 0)
+    g = mg.csr_from_edges(n, src, dst, flags)
+    g.values = mg.hash_weights(g, 5, 64) - 1
+    with mg.Graph(g, symmetric=symmetric, build_csc=not symmetric) as dg:
+        pulls = 0
+        for s in (int(np.argmax(g.degrees())), 70, n - 1):
+            got, st = dg.sssp(s, stats=True)
+            assert np.array_equal(got, oracle.sssp(g.row_offsets, g.col_idx, g.values, s))
+            pulls += st.bottom_up_levels
+        assert pulls or not big
