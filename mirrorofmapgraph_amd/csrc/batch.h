@@ -229,8 +229,8 @@ struct PprDev {
     int width = 8;                        // row width W: 8, 16, 32 or 64 columns
     uint64_t live = 0;                    // slots in use
     int64_t bytes = 0;
-    float *X[2] = {nullptr, nullptr};     // ranks, n x W (room for n x PPR_SLOTS)
-    float *C = nullptr;                   // contributions
+    float *X[2] = {nullptr, nullptr};     // ranks, n x W, then a row of zeros (room for (n + 1) x PPR_SLOTS)
+    float *C = nullptr;                   // contributions, the same
     float *part = nullptr;                // partial sums of long in-lists
     float *rows = nullptr;                // PPR_SLOTS x n results
     ChunkRec *tasks = nullptr;

@@ -326,6 +326,24 @@ def test_ppr_list_lengths(mg, oracle, device, n, relabel):
                 assert np.array_equal(dg.ppr_batch(srcs[:k], o).view(np.int32), full[:k].view(np.int32))
 
 
+def test_ppr_rows_past_4_gib(mg, oracle, device):
+    # 64 columns of 2^24 + 3 vertices: the widest rows' offsets need more than 32 bits
+    n = (1 << 24) + 3
+    rng = np.random.default_rng(4)
+    src, dst = rng.integers(0, n, 2 * n, dtype=np.int32), rng.integers(0, n, 2 * n, dtype=np.int32)
+    hub = rng.integers(n - 50, n, 4000, dtype=np.int32)
+    src, dst = np.concatenate([src, hub]), np.concatenate([dst, np.full(4000, n - 1, np.int32)])
+    g = mg.csr_from_edges(n, src, dst, mg.MG_CSR_SORT_COLS)
+    srcs = np.concatenate([np.arange(n - 30, n), rng.integers(0, n, 3)]).astype(np.int32)
+    o = mg.options(ppr_iters=2)
+    with mg.Graph(g, build_csc=True) as dg:
+        few = dg.ppr_batch(srcs[:8], o)  # rows of 8 columns: below 4 GiB
+        full = dg.ppr_batch(srcs, o)
+    assert np.array_equal(full[:8].view(np.int32), few.view(np.int32))
+    for j in (0, 29, 32):
+        assert np.max(np.abs(full[j] - oracle.ppr(g.row_offsets, g.col_idx, int(srcs[j]), iters=2))) <= 1e-6
+
+
 @pytest.mark.parametrize("edges", [0, 1, 2, 3, 4, 5, 9])
 def test_ppr_tiny_adjacency(mg, oracle, device, edges):
     # fewer edges than the loads of a block are wide
