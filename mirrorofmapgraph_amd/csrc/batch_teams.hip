@@ -15,6 +15,8 @@
 // 64 SSSP sources on a 512^2 grid 76 -> 6.0 ms (93 before the shared batches' slices fitted
 // the grid); with 1024 workgroups 6.4 ms.  256 sources: SSSP 13.8 ms with 256 teams of two
 // workgroups, 17.8 with 128 of eight, 24 with 64 of 16; BFS 11.3 / 12.2 / 13.8 ms.
+#include <cmath>
+
 #include "batch.h"
 #include "team_search.h"
 
@@ -26,6 +28,12 @@ constexpr int XCDS = 8;
 // Sparse: fewer edges than this per vertex.  The same line as mg_bfs_batch's levels: a
 // search of a denser graph has a wide level soon, and would only be started for nothing.
 constexpr int64_t TEAMS_DEGREE = 8;
+// A level of a mesh has up to a few times sqrt(n) vertices (buckets: twice that): teams are
+// given room for TEAMS_FRONT (SSSP 2 x) sqrt(n) records, which many small ones lack on a
+// large graph, and twice the workgroups, down to 32 teams of 16, when a row outgrows one all
+// the same.  2048^2 grid, 256 rows (two workgroups a team outgrown, the call run again in
+// general / so): BFS 410 / 159 ms, SSSP 884 / 284; on the 512^2 grid two workgroups do.
+constexpr int TEAMS_FRONT = 4;
 
 struct TeamsCtl {
     int arrived[16];             // workgroups that came, by XCD
@@ -44,7 +52,8 @@ struct TeamsDev {
     int64_t rows_cap = 0;
     int *pairs = nullptr;      // row starts (MG_BATCH_MAX + 1), then the sources by row
     int64_t pairs_cap = 0;
-    bool wide[2] = {false, false};  // a BFS / SSSP row was too wide for a team
+    bool wide[2] = {false, false};  // a BFS / SSSP row was too wide for the largest team
+    int wgs[2] = {0, 0};            // least workgroups of a team, since smaller ones were outgrown (0: none yet)
     int64_t bytes = 0;
 };
 
@@ -266,7 +275,10 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
     if (!tp && !(tp = new (std::nothrow) TeamsDev())) return set_error(MG_ERR_OOM, "host allocation failed");
     TeamsDev &t = *tp;
     const int nwords = ((g->n + 63) / 64) * 2;
-    const int per_xcd = std::min((k + XCDS - 1) / XCDS, TEAMS_MAX / XCDS), teams = per_xcd * XCDS;
+    const int room = TEAM_SEG * (BLK / WAVE);  // records a workgroup queues
+    const int front = (int)std::min(1e6, (sssp ? 2 : 1) * TEAMS_FRONT * std::sqrt((double)g->n));
+    const int least = std::min(TEAM_WGS, std::max(t.wgs[sssp], (front + room - 1) / room));
+    const int per_xcd = std::min({(k + XCDS - 1) / XCDS, TEAMS_MAX / XCDS, TEAMS_GRID / XCDS / least}), teams = per_xcd * XCDS;
     if (!t.ctl && (rc = teams_buf(t, &t.ctl, 0, sizeof(TeamsCtl)))) return rc;
     if (!t.h_ctl && hipHostMalloc((void **)&t.h_ctl, sizeof(TeamsCtl), hipHostMallocDefault) != hipSuccess)
         return set_error(MG_ERR_OOM, "hipHostMalloc failed");
@@ -337,6 +349,10 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
     MG_HIP(hipEventRecord(g->ev1, g->stream));
     MG_HIP(hipMemcpyAsync(t.h_ctl, t.ctl, sizeof(TeamsCtl), hipMemcpyDeviceToHost, g->stream));
     MG_HIP(hipStreamSynchronize(g->stream));
+    if (t.h_ctl->wide && a.wgs < TEAM_WGS) {
+        t.wgs[sssp] = 2 * a.wgs;
+        return teams_batch(g, sssp, row_of, srcs, npairs, k, out, o, stats, timer, wide);
+    }
     if (t.h_ctl->wide) {
         t.wide[sssp] = *wide = true;
         return MG_OK;

@@ -456,3 +456,26 @@ def test_sssp_dense_task_sizes(mg, oracle, device, n, symmetric):
             assert np.array_equal(got, oracle.sssp(g.row_offsets, g.col_idx, g.values, s))
             pulls += st.bottom_up_levels
         assert pulls or not big
+
+
+@pytest.mark.parametrize("k", [100, 256])
+@pytest.mark.parametrize("depth", [10, 12, 13, 15])
+def test_batch_teams_grow(mg, oracle, device, depth, k):
+    # binary trees whose levels outgrow teams of 2, 4 and 8 workgroups, and the largest
+    n = 2 ** (depth + 1) - 1
+    v = np.arange(1, n)
+    g = mg.csr_from_edges(n, ((v - 1) // 2).astype(np.int32), v.astype(np.int32), mg.MG_CSR_SYMMETRIZE | mg.MG_CSR_SORT_COLS)
+    g.values = mg.hash_weights(g, depth, 9)
+    srcs = np.random.default_rng(depth).integers(0, n, k).astype(np.int32)
+    srcs[:3] = [0, n - 1, n // 2]
+    bfs = np.stack([oracle.bfs(g.row_offsets, g.col_idx, int(s)) for s in srcs])
+    sssp = np.stack([oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)) for s in srcs])
+    with mg.Graph(g, symmetric=True) as dg:
+        for _ in range(2):
+            got, st = dg.bfs_batch(srcs, stats=True)
+            assert np.array_equal(got, bfs)
+            assert st.vertices_reached == k * n and st.edges_traversed == k * g.m
+            got, st = dg.sssp_batch(srcs, stats=True)
+            assert np.array_equal(got, sssp)
+            assert st.vertices_reached == k * n
+        assert np.array_equal(dg.bfs_batch(srcs[:5]), bfs[:5])
