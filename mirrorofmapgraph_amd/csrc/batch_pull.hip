@@ -520,7 +520,8 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
         return MG_OK;
     };
     // the captured rounds read k and the row width from their arguments
-    if ((rc = drive(g, step, PULL_ROUNDS + 2, KIND_BATCH_SSSP, mix64(0x9011 + (uint64_t)k), p.ctl, p.h_ctl))) return rc;
+    const StepKey sk = batch_pull_steps(k);
+    if ((rc = drive(g, step, PULL_ROUNDS + 2, sk.kind, sk.key, p.ctl, p.h_ctl))) return rc;
     if (p.h_ctl->changed & PULL_DEEP) {
         p.deep = *deep = true;
         return MG_OK;

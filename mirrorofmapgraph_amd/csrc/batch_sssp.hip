@@ -670,8 +670,8 @@ static int sssp_batch_run(mg_graph *g, const int32_t *slot_of, const int32_t *sr
             if ((rc = sssp_batch_seed(*b, g, g->stream, sl, delta, true, false))) return rc;
         }
         auto step = [&]() -> int { return sssp_batch_step(*b, g, g->stream, delta); };
-        if ((rc = drive(g, step, (int64_t)o.iter_num + 3, KIND_BATCH_SSSP, mix64((uint64_t)delta), b->ctl, b->h_ctl)))
-            return rc;
+        const StepKey sk = batch_sssp_steps(delta);
+        if ((rc = drive(g, step, (int64_t)o.iter_num + 3, sk.kind, sk.key, b->ctl, b->h_ctl))) return rc;
         if ((rc = sssp_batch_extract(*b, g, g->stream, all))) return rc;
         if ((rc = batch_row_stats(*b, g, g->stream, all, INT_MAX))) return rc;
         hipLaunchKernelGGL(sb_sum_stats, dim3(1), dim3(SMALL_BLK), 0, g->stream, b->ctl, (const SlotCtl *)b->sc, k);

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "mg_internal.h"
+#include "routes.h"
 
 #define MG_HIP(call)                                                                              \
     do {                                                                                          \
@@ -265,7 +266,6 @@ constexpr int DENSE_T = 2048, DENSE_T_MIN = 512;
 constexpr int DENSE_TASKS = 8192;
 constexpr int DENSE_V = 256;
 constexpr int DENSE_RANGE_MAX = 8 * DENSE_T;
-enum { KIND_BFS = 0, KIND_SSSP = 1, KIND_PR = 2, KIND_GAS = 3, KIND_BATCH = 4, KIND_BATCH_SSSP = 5, NKINDS = 8 };
 
 struct StepGraph {
     hipGraphExec_t exec = nullptr;                        // STEPS_PER_GRAPH steps

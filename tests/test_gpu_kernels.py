@@ -479,3 +479,13 @@ def test_batch_teams_grow(mg, oracle, device, depth, k):
             assert np.array_equal(got, sssp)
             assert st.vertices_reached == k * n
         assert np.array_equal(dg.bfs_batch(srcs[:5]), bfs[:5])
+
+
+def test_batch_pull_falls_back_whatever_the_bucket_width(mg, oracle, device):
+    # the pushed route's steps beside the pulled route's, at a width that once named both
+    g = _clique_chain(mg, 60, 20)
+    g.values = mg.hash_weights(g, 2, 30)
+    srcs = np.array([0, g.n // 2, g.n - 1], np.int32)
+    with mg.Graph(g, symmetric=True) as dg:
+        for got, s in zip(dg.sssp_batch(srcs, mg.options(sssp_delta=0x9011 + len(srcs))), srcs):
+            assert np.array_equal(got, oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)))
