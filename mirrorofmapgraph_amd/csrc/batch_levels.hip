@@ -420,7 +420,7 @@ int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32
     a.G = b.G;
     // the result: the caller's device buffer, else rows of our own
     int *out = depth_out;
-    if (!o.out_on_device || !out) {
+    if (!plan_delivery(g, depth_out, 4 * (size_t)k * g->n, o.out_on_device).by_kernel) {
         if (!b.rows_out) {
             if ((rc = alloc_i32(&b.rows_out, (size_t)b.S * g->n + 1))) return rc;
             b.bytes += 4LL * b.S * g->n + 4;
@@ -471,7 +471,7 @@ int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32
         stats->vertices_reached = b.h_ctl->reached;
         stats->device_ms = ms;
     }
-    if (out != depth_out && (rc = deliver(g, depth_out, out, 4 * (size_t)k * g->n, false))) return rc;
+    if (out != depth_out && (rc = deliver(g, depth_out, out, 4 * (size_t)k * g->n, o.out_on_device))) return rc;
     if (stats) stats->host_ms = timer.ms();
     return MG_OK;
 }

@@ -461,7 +461,7 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
         p.live = reinterpret_cast<uint32_t *>(l);
         p.bytes += (int64_t)sizeof(Ctl) + (int64_t)sizeof(LevelPart) * PART_GROUPS + 96 + 16LL * g->n;
     }
-    const bool direct = o.out_on_device && out;
+    const bool direct = plan_delivery(g, out, 4 * (size_t)k * g->n, o.out_on_device).by_kernel;
     auto grow = [&](int **buf, int64_t *cap, int64_t need) -> int {
         if (*cap >= need) return MG_OK;
         MG_HIP(hipStreamSynchronize(g->stream));

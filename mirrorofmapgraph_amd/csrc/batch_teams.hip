@@ -309,7 +309,7 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
         t.pairs_cap = (int64_t)pairs.size();
     }
     const int64_t cells = (int64_t)k * g->n;
-    const bool direct = o.out_on_device && out;
+    const bool direct = plan_delivery(g, out, 4 * (size_t)cells, o.out_on_device).as_state;
     if (!direct && t.rows_cap < cells) {
         const int64_t had = t.rows_cap;
         t.rows_cap = 0;

@@ -656,11 +656,13 @@ int print_trace(mg_graph *g, const char *what, const char *dir0, const char *dir
 // Where a result goes.  by_kernel: device memory of the graph's own device, written by the
 // kernels that end the search; early: host memory, copied ahead of the wait that the search
 // ends with, up to EARLY_BYTES (that wait may come before the search is over, and the copy is
-// then made again).  Otherwise it is copied after the wait.
+// then made again).  Otherwise it is copied after the wait.  as_state: by_kernel, and memory
+// of the default kind, which a search may use as its own rows (atomics, lines shared through
+// an XCD's L2); fine-grained and uncached memory is cached otherwise.
 constexpr size_t EARLY_BYTES = 1 << 20;
 struct Delivery {
     void *out = nullptr;
-    bool on_device = false, by_kernel = false, early = false;
+    bool on_device = false, by_kernel = false, as_state = false, early = false;
 };
 Delivery plan_delivery(const mg_graph *g, void *out, size_t bytes, bool out_on_device);
 // Queues what follows a finished search: the result back to the caller's ids (a twin's

@@ -256,6 +256,7 @@ Delivery plan_delivery(const mg_graph *g, void *out, size_t bytes, bool out_on_d
         return d;
     }
     d.by_kernel = at.type == hipMemoryTypeDevice && at.device == g->device && (uintptr_t)out % 4 == 0;
+    d.as_state = d.by_kernel && (at.allocationFlags & hipDeviceMallocUncached) == 0;  // (its bits: fine-grained or uncached)
     return d;
 }
 

@@ -489,3 +489,58 @@ def test_batch_pull_falls_back_whatever_the_bucket_width(mg, oracle, device):
     with mg.Graph(g, symmetric=True) as dg:
         for got, s in zip(dg.sssp_batch(srcs, mg.options(sssp_delta=0x9011 + len(srcs))), srcs):
             assert np.array_equal(got, oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)))
+
+
+# ---------------------------------------------------------------- where batched results go
+@pytest.mark.parametrize("relabel", [False, True])
+@pytest.mark.parametrize("which", ["sparse", "dense", "wide"])
+def test_batched_results_reach_every_kind_of_output(mg, oracle, device, which, relabel):
+    # the routes by teams, by levels and by pulling, and the general one: device memory at even and odd
+    # addresses, fine-grained device memory, managed and pinned memory named as device pointers, host memory
+    import ctypes as C
+
+    if which == "sparse":
+        g = mg.grid_graph(61, 37, seed=5, weight_max=9)
+    elif which == "dense":
+        g = random_graph(mg, 1501, 12000, 6, wmax=30)
+    else:
+        g = random_graph(mg, 120000, 350000, 3, wmax=20)
+    k, n = 3, g.n
+    srcs = np.array([0, n // 2, n - 1], np.int32)
+    size, I32P = 4 * k * n, C.POINTER(C.c_int32)
+    hip = C.CDLL("libamdhip64.so")
+    kinds = {"device": lambda p: hip.hipMalloc(p, C.c_size_t(size + 8)),
+             "fine-grained": lambda p: hip.hipExtMallocWithFlags(p, C.c_size_t(size + 8), C.c_uint(1)),
+             "managed": lambda p: hip.hipMallocManaged(p, C.c_size_t(size + 8), C.c_uint(1)),
+             "pinned": lambda p: hip.hipHostMalloc(p, C.c_size_t(size + 8), C.c_uint(0))}
+    mem = {}
+    for kind, alloc in kinds.items():
+        mem[kind] = C.c_void_p()
+        assert alloc(C.byref(mem[kind])) == 0
+    with mg.Graph(g, symmetric=True, relabel=relabel) as dg:
+        for name, one in (("mg_bfs_batch", lambda s: oracle.bfs(g.row_offsets, g.col_idx, s)),
+                          ("mg_sssp_batch", lambda s: oracle.sssp(g.row_offsets, g.col_idx, g.values, s))):
+            exp = np.stack([one(int(s)) for s in srcs])
+            raw = np.empty(size + 8, np.uint8)
+
+            def call(ptr, on_device):
+                o, st = mg.options(out_on_device=on_device), mg.Stats()
+                mg.check(getattr(mg.lib(), name)(dg.handle, srcs.ctypes.data_as(I32P), k, C.c_void_p(ptr), C.byref(o),
+                                                 C.byref(st)))
+                assert st.vertices_reached == int(((exp >= 0) & (exp != 2**31 - 1)).sum())
+
+            host = np.zeros((k, n), np.int32)
+            call(host.ctypes.data, 0)
+            assert np.array_equal(host, exp)
+            for kind, p in mem.items():
+                for at in (0, 4, 1):
+                    raw[:] = 0xA5
+                    assert hip.hipMemcpy(p, raw.ctypes.data_as(C.c_void_p), C.c_size_t(raw.nbytes), 4) == 0
+                    call(p.value + at, 1)
+                    assert hip.hipMemcpy(raw.ctypes.data_as(C.c_void_p), p, C.c_size_t(raw.nbytes), 4) == 0
+                    assert np.array_equal(raw[at:at + size].copy().view(np.int32).reshape(k, n), exp), (name, kind, at)
+                    assert np.all(raw[:at] == 0xA5) and np.all(raw[at + size:] == 0xA5), (name, kind, at)
+            call(None, 0)
+            call(None, 1)
+    for kind, p in mem.items():
+        (hip.hipHostFree if kind == "pinned" else hip.hipFree)(p)
