@@ -143,6 +143,7 @@ struct BatchDev {
     int *D = nullptr;                            // SSSP distances, n x KS
     int *rows = nullptr;                         // S x n results
     int *rows_out = nullptr;                     // on a degree-ordered twin: rows in the caller's ids
+    int64_t rows_out_cap = 0;                    // other graphs: cells of rows_out (batch_levels.hip; grown)
     bool deep = false;                           // BFS: a search outgrew the levels (batch_levels.hip)
     int2 *pairs = nullptr;                       // SSSP: (vertex, slot) pairs of sparse vertices
     int64_t pair_cap = 0;
@@ -202,6 +203,10 @@ int batch_release_slots(BatchDev &b, hipStream_t st, const uint32_t mask[8]);
 
 int batch_alpha(const mg_options &o);
 int batch_beta(const mg_options &o);
+// The routes below (levels, teams, pulls) need memory that the general ones do not: refused
+// there (MG_ERR_OOM, before anything is queued), the call takes the general route.  True then,
+// with the error cleared.
+bool route_refused(int rc);
 // Batched BFS by whole levels (batch_levels.hip).
 constexpr int LEVELS_ALPHA = 16;
 int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32_t *srcs, int32_t npairs, int32_t k,
@@ -210,6 +215,10 @@ int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32
 // Batched searches by teams (batch_teams.hip), on graphs that teams_wanted() names: sparse
 // ones, until a search there turns out wide (then *wide is set and nothing delivered).
 bool teams_wanted(const mg_graph *g, bool sssp);
+// Runs the call that way when it is wanted; *done says whether it did (with the status
+// returned), else the call goes on to the other routes.
+int teams_try(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k, int32_t *out,
+              const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *done);
 int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
                 int32_t *out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *wide);
 

@@ -701,6 +701,13 @@ int finish_batch(mg_graph *g, BatchDev &b, mg_stats *stats, void *out, size_t by
     return MG_OK;
 }
 
+bool route_refused(int rc) {
+    if (rc != MG_ERR_OOM) return false;
+    clear_error();
+    (void)hipGetLastError();  // the allocation's: the next launch check would report it
+    return true;
+}
+
 int batch_alpha(const mg_options &o) { return o.batch_alpha > 0 ? o.batch_alpha : 4; }
 int batch_beta(const mg_options &o) { return o.batch_beta > 0 ? o.batch_beta : 16; }
 
@@ -741,9 +748,9 @@ static int bfs_batch_run(mg_graph *g, const int32_t *slot_of, const int32_t *src
         int rc;
         if (!b->deep && g->m >= LEVELS_DEGREE * (int64_t)g->n) {
             bool deep = false;
-            if ((rc = bfs_levels_run(g, *b, slot_of, srcs, npairs, k, depth_out, o, stats, timer, &deep)) || !deep)
-                return rc;
-            b->deep = true;
+            rc = bfs_levels_run(g, *b, slot_of, srcs, npairs, k, depth_out, o, stats, timer, &deep);
+            if (deep) b->deep = true;
+            else if (!route_refused(rc)) return rc;
         }
         MG_HIP(hipEventRecord(g->ev0, g->stream));
         if ((rc = bfs_batch_reset(*b, g, g->stream, o.iter_num, batch_alpha(o), batch_beta(o), 0))) return rc;
@@ -779,10 +786,9 @@ extern "C" int mg_bfs_batch(mg_graph *g, const int32_t *srcs, int32_t k, int32_t
         return set_error(MG_ERR_UNSUPPORTED, "mg_bfs_batch: directed=0 needs a symmetric graph");
     int32_t rows[MG_BATCH_MAX], tsrc[MG_BATCH_MAX];
     for (int s = 0; s < k; ++s) rows[s] = s;
-    if (teams_wanted(g, false)) {
-        bool wide = false;
-        if ((rc = teams_batch(g, false, rows, srcs, k, k, depth_out, o, stats, timer, &wide)) || !wide) return rc;
-    }
+    bool done = false;
+    rc = teams_try(g, false, rows, srcs, k, k, depth_out, o, stats, timer, &done);
+    if (done) return rc;
     mg_graph *sg = batch_graph(g, o, srcs, k, tsrc);  // the degree-ordered twin, when the graph keeps one
     if (sg != g && (rc = ensure_workspace(sg))) return rc;
     return bfs_batch_run(sg, rows, sg != g ? tsrc : srcs, k, k, depth_out, o, stats, timer);
@@ -798,10 +804,9 @@ extern "C" int mg_bfs_batch_sets(mg_graph *g, const int32_t *row_of, const int32
     if ((rc = check_batch_sets("mg_bfs_batch_sets", g, row_of, srcs, npairs, k))) return rc;
     if (o.directed == 0 && !(g->flags & MG_GRAPH_SYMMETRIC))
         return set_error(MG_ERR_UNSUPPORTED, "mg_bfs_batch_sets: directed=0 needs a symmetric graph");
-    if (teams_wanted(g, false)) {
-        bool wide = false;
-        if ((rc = teams_batch(g, false, row_of, srcs, npairs, k, depth_out, o, stats, timer, &wide)) || !wide) return rc;
-    }
+    bool done = false;
+    rc = teams_try(g, false, row_of, srcs, npairs, k, depth_out, o, stats, timer, &done);
+    if (done) return rc;
     std::vector<int32_t> tsrc((size_t)npairs);
     mg_graph *sg = batch_graph(g, o, srcs, npairs, tsrc.data());
     if (sg != g && (rc = ensure_workspace(sg))) return rc;

@@ -421,9 +421,15 @@ int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32
     // the result: the caller's device buffer, else rows of our own
     int *out = depth_out;
     if (!plan_delivery(g, depth_out, 4 * (size_t)k * g->n, o.out_on_device).by_kernel) {
-        if (!b.rows_out) {
-            if ((rc = alloc_i32(&b.rows_out, (size_t)b.S * g->n + 1))) return rc;
-            b.bytes += 4LL * b.S * g->n + 4;
+        const int64_t cells = (int64_t)k * g->n;
+        if (!g->perm && b.rows_out_cap < cells) {  // (a twin's context has rows for every slot)
+            free_dev(b.rows_out);
+            b.rows_out = nullptr;
+            b.bytes -= 4 * b.rows_out_cap;
+            b.rows_out_cap = 0;
+            if ((rc = alloc_i32(&b.rows_out, (size_t)cells))) return rc;
+            b.rows_out_cap = cells;
+            b.bytes += 4 * cells;
         }
         out = b.rows_out;
     }

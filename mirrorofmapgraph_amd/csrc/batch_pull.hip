@@ -384,6 +384,7 @@ __global__ __launch_bounds__(BLK) void pull_rows(PullArgs a, int ks, const int *
 void pull_release(mg_graph *g) {
     PullDev *&p = g->steps->pull;
     if (!p) return;
+    invalidate_steps(g, KIND_BATCH_PULL);  // captured rounds point at these buffers
     free_dev(p->ctl);
     if (p->h_ctl) (void)hipHostFree(p->h_ctl);
     free_dev(p->part);
@@ -465,7 +466,7 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
     auto grow = [&](int **buf, int64_t *cap, int64_t need) -> int {
         if (*cap >= need) return MG_OK;
         MG_HIP(hipStreamSynchronize(g->stream));
-        invalidate_steps(g);  // captured rounds point at the old buffer
+        invalidate_steps(g, KIND_BATCH_PULL);  // captured rounds point at the old buffer
         free_dev(*buf);
         *buf = nullptr;
         p.bytes -= 4 * *cap;

@@ -648,7 +648,9 @@ static int sssp_batch_run(mg_graph *g, const int32_t *slot_of, const int32_t *sr
     int rc;
     if (pull_wanted(g)) {
         bool deep = false;
-        if ((rc = pull_batch(g, slot_of, srcs, npairs, k, dist_out, o, stats, timer, &deep)) || !deep) return rc;
+        rc = pull_batch(g, slot_of, srcs, npairs, k, dist_out, o, stats, timer, &deep);
+        if (route_refused(rc)) pull_release(g);  // room for the general route
+        else if (!deep) return rc;
     }
     BatchDev *b = nullptr;
     if ((rc = graph_batch_dev(g, true, &b))) return rc;
@@ -702,10 +704,9 @@ extern "C" int mg_sssp_batch(mg_graph *g, const int32_t *srcs, int32_t k, int32_
     if ((rc = sssp_batch_checks("mg_sssp_batch", g, o))) return rc;
     int32_t rows[MG_BATCH_MAX], tsrc[MG_BATCH_MAX];
     for (int s = 0; s < k; ++s) rows[s] = s;
-    if (teams_wanted(g, true)) {
-        bool wide = false;
-        if ((rc = teams_batch(g, true, rows, srcs, k, k, dist_out, o, stats, timer, &wide)) || !wide) return rc;
-    }
+    bool done = false;
+    rc = teams_try(g, true, rows, srcs, k, k, dist_out, o, stats, timer, &done);
+    if (done) return rc;
     mg_graph *sg = batch_graph(g, o, srcs, k, tsrc);  // the degree-ordered twin, when the graph keeps one
     if (sg != g && (rc = ensure_workspace(sg))) return rc;
     return sssp_batch_run(sg, rows, sg != g ? tsrc : srcs, k, k, dist_out, o, stats, timer);
@@ -720,10 +721,9 @@ extern "C" int mg_sssp_batch_sets(mg_graph *g, const int32_t *row_of, const int3
     std::lock_guard<std::mutex> lock(g->mu);
     if ((rc = check_batch_sets("mg_sssp_batch_sets", g, row_of, srcs, npairs, k))) return rc;
     if ((rc = sssp_batch_checks("mg_sssp_batch_sets", g, o))) return rc;
-    if (teams_wanted(g, true)) {
-        bool wide = false;
-        if ((rc = teams_batch(g, true, row_of, srcs, npairs, k, dist_out, o, stats, timer, &wide)) || !wide) return rc;
-    }
+    bool done = false;
+    rc = teams_try(g, true, row_of, srcs, npairs, k, dist_out, o, stats, timer, &done);
+    if (done) return rc;
     std::vector<int32_t> tsrc((size_t)npairs);
     mg_graph *sg = batch_graph(g, o, srcs, npairs, tsrc.data());
     if (sg != g && (rc = ensure_workspace(sg))) return rc;

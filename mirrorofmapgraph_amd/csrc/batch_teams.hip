@@ -287,10 +287,8 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
         t.teams = 0;
         if ((rc = teams_buf(t, &t.team, had * (int64_t)sizeof(TeamCtl), teams * (int64_t)sizeof(TeamCtl))) ||
             (rc = teams_buf(t, &t.recs, had * 8 * (int64_t)TEAM_RECS, teams * 8 * (int64_t)TEAM_RECS)) ||
-            (rc = teams_buf(t, &t.bits, had * 16 * (int64_t)nwords, teams * 16 * (int64_t)nwords))) {
-            teams_release(g);
+            (rc = teams_buf(t, &t.bits, had * 16 * (int64_t)nwords, teams * 16 * (int64_t)nwords)))
             return rc;
-        }
         t.teams = teams;
     }
     // the sources by row
@@ -370,6 +368,20 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
     if (!direct && (rc = deliver(g, out, t.rows, 4 * (size_t)cells, o.out_on_device))) return rc;
     if (stats) stats->host_ms = timer.ms();
     return MG_OK;
+}
+
+int teams_try(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k, int32_t *out,
+              const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *done) {
+    *done = false;
+    if (!teams_wanted(g, sssp)) return MG_OK;
+    bool wide = false;
+    const int rc = teams_batch(g, sssp, row_of, srcs, npairs, k, out, o, stats, timer, &wide);
+    if (route_refused(rc)) {
+        teams_release(g);  // room for the general route
+        return MG_OK;
+    }
+    *done = !wide;
+    return rc;
 }
 
 }  // namespace mg

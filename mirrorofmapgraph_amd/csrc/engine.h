@@ -219,6 +219,8 @@ int grow_chunk_queue(mg_graph *g);
 // Destroys every captured step graph of g (their kernel arguments hold buffer
 // pointers; they are captured again on next use).
 void invalidate_steps(mg_graph *g);
+// The same for one kind of steps.
+void invalidate_steps(mg_graph *g, int kind);
 int ensure_pr_workspace(mg_graph *g);
 int ensure_team(mg_graph *g);
 int alloc_i32(int32_t **p, size_t n);

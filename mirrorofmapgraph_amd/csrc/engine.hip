@@ -166,16 +166,17 @@ int64_t queue_capacity(int64_t need, double max_queue_sizing) {
     return c < 64 ? 64 : c > 4e18 ? (int64_t)4e18 : (int64_t)c;
 }
 
-void invalidate_steps(mg_graph *g) {
+void invalidate_steps(mg_graph *g, int kind) {
     if (!g->steps) return;
-    for (StepGraph &s : g->steps->sg) {
-        if (s.exec) (void)hipGraphExecDestroy(s.exec);
-        for (hipGraphExec_t &x : s.part) {
-            if (x) (void)hipGraphExecDestroy(x);
-            x = nullptr;
-        }
-        s = StepGraph();
-    }
+    StepGraph &s = g->steps->sg[kind];
+    if (s.exec) (void)hipGraphExecDestroy(s.exec);
+    for (hipGraphExec_t x : s.part)
+        if (x) (void)hipGraphExecDestroy(x);
+    s = StepGraph();
+}
+
+void invalidate_steps(mg_graph *g) {
+    for (int kind = 0; kind < NKINDS; ++kind) invalidate_steps(g, kind);
 }
 
 static int set_chunk_cap(mg_graph *g, int64_t cap) {

@@ -544,3 +544,29 @@ def test_batched_results_reach_every_kind_of_output(mg, oracle, device, which, r
             call(None, 1)
     for kind, p in mem.items():
         (hip.hipHostFree if kind == "pinned" else hip.hipFree)(p)
+
+
+@pytest.mark.parametrize("which", ["teams", "levels", "pull"])
+@pytest.mark.parametrize("kth", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_batched_routes_refused_memory_go_the_general_way(mg, oracle, device, monkeypatch, which, kth):
+    # the kth allocation of a call is refused: one that only a faster route needs fails no call
+    import ctypes as C
+
+    g = mg.grid_graph(61, 37, seed=5, weight_max=9) if which == "teams" else random_graph(mg, 1501, 12000, 6, wmax=30)
+    srcs = np.array([0, g.n // 2, g.n - 1], np.int32)
+    bfs = np.stack([oracle.bfs(g.row_offsets, g.col_idx, int(s)) for s in srcs])
+    sssp = np.stack([oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)) for s in srcs])
+    with mg.Graph(g, symmetric=True) as dg:
+        if which == "levels":  # the context, which both routes need, without the rows of a host result
+            hip, p, o = C.CDLL("libamdhip64.so"), C.c_void_p(), mg.options(out_on_device=1)
+            assert hip.hipMalloc(C.byref(p), C.c_size_t(12 * g.n)) == 0
+            mg.check(mg.lib().mg_bfs_batch(dg.handle, srcs.ctypes.data_as(C.POINTER(C.c_int32)), 3, p, C.byref(o), None))
+            hip.hipFree(p)
+        monkeypatch.setenv("MG_FAIL_ALLOC_AT", str(kth))
+        rows = dg.sssp_batch(srcs) if which == "pull" else dg.bfs_batch(srcs)
+        monkeypatch.delenv("MG_FAIL_ALLOC_AT")
+        assert np.array_equal(rows, sssp if which == "pull" else bfs)
+        for _ in range(2):
+            assert np.array_equal(dg.bfs_batch(srcs), bfs) and np.array_equal(dg.sssp_batch(srcs), sssp)
+        more = np.concatenate([srcs, srcs + 1, srcs[:1]])[:6] % g.n  # a larger call on the same state
+        assert np.array_equal(dg.bfs_batch(more)[:3], bfs) and np.array_equal(dg.sssp_batch(more)[:3], sssp)
