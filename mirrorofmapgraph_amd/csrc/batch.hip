@@ -749,8 +749,15 @@ static int bfs_batch_run(mg_graph *g, const int32_t *slot_of, const int32_t *src
         if (!b->deep && g->m >= LEVELS_DEGREE * (int64_t)g->n) {
             bool deep = false;
             rc = bfs_levels_run(g, *b, slot_of, srcs, npairs, k, depth_out, o, stats, timer, &deep);
-            if (deep) b->deep = true;
-            else if (!route_refused(rc)) return rc;
+            if (deep) {
+                b->deep = true;
+                if (!g->perm) {  // the levels' rows for host results: not needed again
+                    free_dev(b->rows_out);
+                    b->rows_out = nullptr;
+                    b->bytes -= 4 * b->rows_out_cap;
+                    b->rows_out_cap = 0;
+                }
+            } else if (!route_refused(rc)) return rc;
         }
         MG_HIP(hipEventRecord(g->ev0, g->stream));
         if ((rc = bfs_batch_reset(*b, g, g->stream, o.iter_num, batch_alpha(o), batch_beta(o), 0))) return rc;

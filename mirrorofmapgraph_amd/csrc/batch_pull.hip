@@ -65,7 +65,6 @@ struct PullDev {
     int ntasks = 0;
     int *D = nullptr, *rows = nullptr;
     int64_t d_cap = 0, rows_cap = 0, bytes = 0;
-    bool deep = false;
 };
 
 // Rows of INT_MAX (0 past slot k), nothing changed, every slot live.
@@ -401,7 +400,7 @@ int64_t pull_dev_size(const PullDev *p) { return p->bytes; }
 
 bool pull_wanted(const mg_graph *g) {
     return g->m >= PULL_DEGREE * (int64_t)g->n && ((g->flags & MG_GRAPH_SYMMETRIC) || g->col_off) &&
-           !(g->steps->pull && g->steps->pull->deep);
+           !g->steps->pull_deep;
 }
 
 // The wave tasks over the in-lists: runs of consecutive vertices with at most PULL_T
@@ -524,7 +523,8 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
     const StepKey sk = batch_pull_steps(k);
     if ((rc = drive(g, step, PULL_ROUNDS + 2, sk.kind, sk.key, p.ctl, p.h_ctl))) return rc;
     if (p.h_ctl->changed & PULL_DEEP) {
-        p.deep = *deep = true;
+        g->steps->pull_deep = *deep = true;
+        pull_release(g);  // not taken again
         return MG_OK;
     }
     int *dst = direct ? out : p.rows;

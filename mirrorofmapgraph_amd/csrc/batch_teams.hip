@@ -52,8 +52,6 @@ struct TeamsDev {
     int64_t rows_cap = 0;
     int *pairs = nullptr;      // row starts (MG_BATCH_MAX + 1), then the sources by row
     int64_t pairs_cap = 0;
-    bool wide[2] = {false, false};  // a BFS / SSSP row was too wide for the largest team
-    int wgs[2] = {0, 0};            // least workgroups of a team, since smaller ones were outgrown (0: none yet)
     int64_t bytes = 0;
 };
 
@@ -264,7 +262,7 @@ static int teams_buf(TeamsDev &t, T **p, int64_t old_bytes, int64_t need) {
 }
 
 bool teams_wanted(const mg_graph *g, bool sssp) {
-    return g->m < TEAMS_DEGREE * (int64_t)g->n && !(g->steps->teams && g->steps->teams->wide[sssp]);
+    return g->m < TEAMS_DEGREE * (int64_t)g->n && !g->steps->teams_wide[sssp];
 }
 
 int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
@@ -277,7 +275,7 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
     const int nwords = ((g->n + 63) / 64) * 2;
     const int room = TEAM_SEG * (BLK / WAVE);  // records a workgroup queues
     const int front = (int)std::min(1e6, (sssp ? 2 : 1) * TEAMS_FRONT * std::sqrt((double)g->n));
-    const int least = std::min(TEAM_WGS, std::max(t.wgs[sssp], (front + room - 1) / room));
+    const int least = std::min(TEAM_WGS, std::max(g->steps->teams_wgs[sssp], (front + room - 1) / room));
     const int per_xcd = std::min({(k + XCDS - 1) / XCDS, TEAMS_MAX / XCDS, TEAMS_GRID / XCDS / least}), teams = per_xcd * XCDS;
     if (!t.ctl && (rc = teams_buf(t, &t.ctl, 0, sizeof(TeamsCtl)))) return rc;
     if (!t.h_ctl && hipHostMalloc((void **)&t.h_ctl, sizeof(TeamsCtl), hipHostMallocDefault) != hipSuccess)
@@ -348,11 +346,12 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
     MG_HIP(hipMemcpyAsync(t.h_ctl, t.ctl, sizeof(TeamsCtl), hipMemcpyDeviceToHost, g->stream));
     MG_HIP(hipStreamSynchronize(g->stream));
     if (t.h_ctl->wide && a.wgs < TEAM_WGS) {
-        t.wgs[sssp] = 2 * a.wgs;
+        g->steps->teams_wgs[sssp] = 2 * a.wgs;
         return teams_batch(g, sssp, row_of, srcs, npairs, k, out, o, stats, timer, wide);
     }
     if (t.h_ctl->wide) {
-        t.wide[sssp] = *wide = true;
+        g->steps->teams_wide[sssp] = *wide = true;
+        teams_release(g);  // (searches of the other kind make it again)
         return MG_OK;
     }
     float ms = 0;

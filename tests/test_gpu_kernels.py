@@ -570,3 +570,39 @@ def test_batched_routes_refused_memory_go_the_general_way(mg, oracle, device, mo
             assert np.array_equal(dg.bfs_batch(srcs), bfs) and np.array_equal(dg.sssp_batch(srcs), sssp)
         more = np.concatenate([srcs, srcs + 1, srcs[:1]])[:6] % g.n  # a larger call on the same state
         assert np.array_equal(dg.bfs_batch(more)[:3], bfs) and np.array_equal(dg.sssp_batch(more)[:3], sssp)
+
+
+@pytest.mark.parametrize("which", ["teams-bfs", "teams-sssp", "levels", "pull"])
+def test_batched_routes_given_up_hold_no_memory(mg, oracle, device, monkeypatch, which):
+    # after a search that its route could not hold, the graph holds what the general route needs
+    import ctypes as C
+
+    if which.startswith("teams"):
+        g = random_graph(mg, 120000, 350000, 3, wmax=20)
+    else:
+        g = _clique_chain(mg, 60, 20)
+        g.values = mg.hash_weights(g, 2, 30)
+    srcs = np.array([0, g.n // 2, g.n - 1], np.int32)
+    sssp = which in ("teams-sssp", "pull")
+    one = (lambda s: oracle.sssp(g.row_offsets, g.col_idx, g.values, s)) if sssp else (
+        lambda s: oracle.bfs(g.row_offsets, g.col_idx, s))
+    exp = np.stack([one(int(s)) for s in srcs])
+
+    def grown(general):
+        with mg.Graph(g, symmetric=True) as dg:
+            before = dg.device_bytes()
+            if not general:
+                for _ in range(2):
+                    assert np.array_equal(dg.sssp_batch(srcs) if sssp else dg.bfs_batch(srcs), exp)
+            elif which == "levels":  # (a device result needs no rows)
+                hip, p, o = C.CDLL("libamdhip64.so"), C.c_void_p(), mg.options(out_on_device=1)
+                assert hip.hipMalloc(C.byref(p), C.c_size_t(12 * g.n)) == 0
+                mg.check(mg.lib().mg_bfs_batch(dg.handle, srcs.ctypes.data_as(C.POINTER(C.c_int32)), 3, p, C.byref(o), None))
+                hip.hipFree(p)
+            else:
+                monkeypatch.setenv("MG_FAIL_ALLOC_AT", "1")  # the faster route's first allocation is refused
+                assert np.array_equal(dg.sssp_batch(srcs) if sssp else dg.bfs_batch(srcs), exp)
+                monkeypatch.delenv("MG_FAIL_ALLOC_AT")
+            return dg.device_bytes() - before
+
+    assert grown(False) == grown(True)
