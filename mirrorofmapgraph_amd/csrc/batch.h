@@ -212,15 +212,11 @@ constexpr int LEVELS_ALPHA = 16;
 int bfs_levels_run(mg_graph *g, BatchDev &b, const int32_t *slot_of, const int32_t *srcs, int32_t npairs, int32_t k,
                    int32_t *depth_out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *deep);
 
-// Batched searches by teams (batch_teams.hip), on graphs that teams_wanted() names: sparse
-// ones, until a search there turns out wide (then *wide is set and nothing delivered).
-bool teams_wanted(const mg_graph *g, bool sssp);
-// Runs the call that way when it is wanted; *done says whether it did (with the status
-// returned), else the call goes on to the other routes.
+// Batched searches by teams (batch_teams.hip), on sparse graphs.  Runs the call that way when
+// it is wanted (TeamsRule); *done says whether it did (with the status returned), else the
+// call goes on to the other routes.
 int teams_try(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k, int32_t *out,
               const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *done);
-int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
-                int32_t *out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *wide);
 
 // Batched SSSP by pulling (batch_pull.hip), on graphs that pull_wanted() names: mean degree 8
 // and more with an in-edge view, until a search there takes too many rounds (then *deep is

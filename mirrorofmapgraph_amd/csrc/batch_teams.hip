@@ -7,15 +7,16 @@
 // 512^2 grid are 1850 rounds of about 10,000 (vertex, source) pairs, 41 us each.  Here up to
 // TEAMS_MAX teams take rows from a counter and run each to its end in one launch, the
 // level boundary being a meeting of the team (about 1 us); a row is the team's depth or
-// distance array itself.  The teams share TEAMS_GRID workgroups.  A row whose
-// frontier outgrows a team's queues raises `wide`, every team stops at its next row and
-// the call is run again the shared way, as are all later ones on the graph.
+// distance array itself.  The teams share TEAMS_GRID workgroups.  A row whose frontier
+// outgrows a team's queues says why in TeamsCtl::end, every team stops at its next row and
+// the call is run again, by larger teams or the shared way (TeamsRule).
 //
 // Bound by each team's chain of accesses and meetings, 4 to 5 us a level with 64 teams.
 // 64 SSSP sources on a 512^2 grid 76 -> 6.0 ms (93 before the shared batches' slices fitted
 // the grid); with 1024 workgroups 6.4 ms.  256 sources: SSSP 13.8 ms with 256 teams of two
 // workgroups, 17.8 with 128 of eight, 24 with 64 of 16; BFS 11.3 / 12.2 / 13.8 ms.
 #include <cmath>
+#include <cstdlib>
 
 #include "batch.h"
 #include "team_search.h"
@@ -37,7 +38,7 @@ constexpr int TEAMS_FRONT = 4;
 
 struct TeamsCtl {
     int arrived[16];             // workgroups that came, by XCD
-    int next, wide, levels, pad;  // next row; a row was too wide; most levels of a row
+    int next, end, levels, pad;  // next row; TEAMS_DONE or why a row ended (no team takes another then); most levels of a row
     unsigned long long edges, te, nr;  // edges relaxed; TEPS count and reached vertices
 };
 
@@ -122,7 +123,7 @@ __device__ __forceinline__ int teams_next(const TeamsArgs &a, const TeamSeat &t,
     uint64_t word = team_word(it, false, 0, 0, 0);
     if (t.rank == 0) {
         int row = 0;
-        if (lane == 0) row = ld_dev(&a.ctl->wide) ? a.k : atomicAdd(&a.ctl->next, 1);
+        if (lane == 0) row = ld_dev(&a.ctl->end) ? a.k : atomicAdd(&a.ctl->next, 1);
         row = __builtin_amdgcn_readfirstlane(row);
         if (row < a.k) {
             TeamOut out(t.recs, it, 0);
@@ -142,7 +143,7 @@ __device__ __forceinline__ int teams_next(const TeamsArgs &a, const TeamSeat &t,
                 if (firsts) out.queue(first, firsts, v, o);
             }
             // the out-edges' field carries the row
-            word = team_over(out.word(it)) ? team_word(it, true, 0, 0, row + 1)
+            word = team_over(out.word(it)) ? team_word(it, true, out.hub, 0, row + 1)
                                            : team_word(it, false, out.nrec, min(out.nf, 0xffff), row + 1);
         }
     }
@@ -152,10 +153,10 @@ __device__ __forceinline__ int teams_next(const TeamsArgs &a, const TeamSeat &t,
     return (int)(low & 0xfffff) - 1;
 }
 
-__device__ __forceinline__ void teams_row_done(const TeamsArgs &a, const TeamSeat &t, int L, bool over) {
+__device__ __forceinline__ void teams_row_done(const TeamsArgs &a, const TeamSeat &t, int L, bool over, bool hub) {
     if (t.rank != 0 || lane_id() != 0) return;
     atomicMax(&a.ctl->levels, L);
-    if (over) __hip_atomic_store(&a.ctl->wide, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (over) atomicMax(&a.ctl->end, hub ? TEAMS_HUB : t.size < a.wgs * (BLK / WAVE) ? TEAMS_SHORT : TEAMS_OUTGROWN);
 }
 
 __global__ __launch_bounds__(BLK) void teams_bfs(TeamsArgs a) {
@@ -167,12 +168,13 @@ __global__ __launch_bounds__(BLK) void teams_bfs(TeamsArgs a) {
         const int row = teams_next<false>(a, t, visited, it);
         if (row < 0) return;
         int L = 0;
-        bool over = false;
+        bool over = false, hub = false;
         team_bfs(t, a.off, a.adj, visited, a.rows + (int64_t)row * a.n, L, it, [&](uint64_t w) {
             over = wave_ballot(team_over(w)) != 0;
+            hub = over && team_hub(w);
             return over || wave_ballot(team_nf(w) != 0) == 0 || L >= a.limit;
         });
-        teams_row_done(a, t, L, over);
+        teams_row_done(a, t, L, over, hub);
         if (!over) teams_clear(visited, a.nwords, t);
     }
 }
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(BLK) void teams_sssp(TeamsArgs a) {
         s.thr = a.delta;
         int L = 0;
         const bool done = team_sssp(t, s, L, it, [](uint64_t) {}, [](uint64_t) { return false; });
-        teams_row_done(a, t, L, !done);
+        teams_row_done(a, t, L, !done, s.hub);
         if (done && L >= a.limit) {  // stopped short: the frontier and the far vertices are left
             teams_clear(s.bm0, a.nwords, t);
             teams_clear(s.bm1, a.nwords, t);
@@ -261,21 +263,25 @@ static int teams_buf(TeamsDev &t, T **p, int64_t old_bytes, int64_t need) {
     return MG_OK;
 }
 
-bool teams_wanted(const mg_graph *g, bool sssp) {
-    return g->m < TEAMS_DEGREE * (int64_t)g->n && !g->steps->teams_wide[sssp];
+// Workgroups launched for a team of wgs; fewer with MG_TEAM_LAUNCH in the environment, for
+// tests of teams that close short, as on a busy GPU.
+static int teams_launch(int wgs) {
+    const char *e = getenv("MG_TEAM_LAUNCH");
+    return e && *e ? std::clamp(atoi(e), 1, wgs) : wgs;
 }
 
-int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
-                int32_t *out, const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *wide) {
+// Runs the call; *end says whether its rows were finished (else nothing is delivered) and
+// *wgs how many workgroups a team was to have.
+static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
+                       int32_t *out, const mg_options &o, mg_stats *stats, const CallTimer &timer, int *end, int *wgs) {
     int rc;
-    *wide = false;
     TeamsDev *&tp = g->steps->teams;
     if (!tp && !(tp = new (std::nothrow) TeamsDev())) return set_error(MG_ERR_OOM, "host allocation failed");
     TeamsDev &t = *tp;
     const int nwords = ((g->n + 63) / 64) * 2;
     const int room = TEAM_SEG * (BLK / WAVE);  // records a workgroup queues
     const int front = (int)std::min(1e6, (sssp ? 2 : 1) * TEAMS_FRONT * std::sqrt((double)g->n));
-    const int least = std::min(TEAM_WGS, std::max(g->steps->teams_wgs[sssp], (front + room - 1) / room));
+    const int least = std::min(TEAM_WGS, std::max(g->steps->teams_rule[sssp].wgs, (front + room - 1) / room));
     const int per_xcd = std::min({(k + XCDS - 1) / XCDS, TEAMS_MAX / XCDS, TEAMS_GRID / XCDS / least}), teams = per_xcd * XCDS;
     if (!t.ctl && (rc = teams_buf(t, &t.ctl, 0, sizeof(TeamsCtl)))) return rc;
     if (!t.h_ctl && hipHostMalloc((void **)&t.h_ctl, sizeof(TeamsCtl), hipHostMallocDefault) != hipSuccess)
@@ -336,8 +342,9 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
     MG_HIP(hipMemcpyAsync(t.pairs, pairs.data(), 4 * pairs.size(), hipMemcpyHostToDevice, g->stream));
     hipLaunchKernelGGL(teams_init, dim3(grid_blocks_cap(std::max<int64_t>(cells / 4, 4LL * teams * nwords), BLK, 4 * MAX_GRID)),
                        dim3(BLK), 0, g->stream, a, unreached);
-    if (sssp) hipLaunchKernelGGL(teams_sssp, dim3(teams * a.wgs), dim3(BLK), 0, g->stream, a);
-    else hipLaunchKernelGGL(teams_bfs, dim3(teams * a.wgs), dim3(BLK), 0, g->stream, a);
+    const int grid = teams * teams_launch(a.wgs);
+    if (sssp) hipLaunchKernelGGL(teams_sssp, dim3(grid), dim3(BLK), 0, g->stream, a);
+    else hipLaunchKernelGGL(teams_bfs, dim3(grid), dim3(BLK), 0, g->stream, a);
     if (stats)
         hipLaunchKernelGGL(teams_stats, dim3(std::max(1, std::min(64, grid_blocks(g->n, BLK))), k), dim3(BLK), 0,
                            g->stream, a, unreached);
@@ -345,15 +352,9 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
     MG_HIP(hipEventRecord(g->ev1, g->stream));
     MG_HIP(hipMemcpyAsync(t.h_ctl, t.ctl, sizeof(TeamsCtl), hipMemcpyDeviceToHost, g->stream));
     MG_HIP(hipStreamSynchronize(g->stream));
-    if (t.h_ctl->wide && a.wgs < TEAM_WGS) {
-        g->steps->teams_wgs[sssp] = 2 * a.wgs;
-        return teams_batch(g, sssp, row_of, srcs, npairs, k, out, o, stats, timer, wide);
-    }
-    if (t.h_ctl->wide) {
-        g->steps->teams_wide[sssp] = *wide = true;
-        teams_release(g);  // (searches of the other kind make it again)
-        return MG_OK;
-    }
+    *wgs = a.wgs;
+    *end = t.h_ctl->end;
+    if (*end != TEAMS_DONE) return MG_OK;
     float ms = 0;
     MG_HIP(hipEventElapsedTime(&ms, g->ev0, g->ev1));
     if (stats) {
@@ -372,15 +373,22 @@ int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *sr
 int teams_try(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k, int32_t *out,
               const mg_options &o, mg_stats *stats, const CallTimer &timer, bool *done) {
     *done = false;
-    if (!teams_wanted(g, sssp)) return MG_OK;
-    bool wide = false;
-    const int rc = teams_batch(g, sssp, row_of, srcs, npairs, k, out, o, stats, timer, &wide);
-    if (route_refused(rc)) {
-        teams_release(g);  // room for the general route
-        return MG_OK;
+    TeamsRule &rule = g->steps->teams_rule[sssp];
+    if (g->m >= TEAMS_DEGREE * (int64_t)g->n || !rule.wanted()) return MG_OK;
+    for (bool again = false;;) {
+        int end = TEAMS_DONE, wgs = 0;
+        const int rc = teams_batch(g, sssp, row_of, srcs, npairs, k, out, o, stats, timer, &end, &wgs);
+        if (route_refused(rc)) break;
+        if (rc || end == TEAMS_DONE) {
+            *done = true;
+            if (!rc) rule.succeeded();
+            return rc;
+        }
+        if (!rule.retry(end, wgs, TEAM_WGS, again)) break;
+        again = again || end == TEAMS_SHORT;
     }
-    *done = !wide;
-    return rc;
+    teams_release(g);  // room for the general route
+    return MG_OK;
 }
 
 }  // namespace mg

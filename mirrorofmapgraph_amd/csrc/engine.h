@@ -340,8 +340,7 @@ struct mg_graph_steps {
     mg::PullDev *pull = nullptr;                 // batched SSSP by pulling
     // What batched searches found out about the graph (kept when the routes' state is released)
     bool pull_deep = false;              // SSSP took too many rounds to be pulled
-    bool teams_wide[2] = {false, false};  // a BFS / SSSP row was too wide for the largest team
-    int teams_wgs[2] = {0, 0};            // least workgroups of a team, since smaller ones were outgrown (0: none yet)
+    mg::TeamsRule teams_rule[2];         // BFS, SSSP
 };
 
 // Queues steps until the device reports `done`.  Steps run from a captured HIP graph

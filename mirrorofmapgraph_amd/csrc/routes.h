@@ -20,4 +20,42 @@ struct StepKey {
 inline StepKey batch_sssp_steps(long long delta) { return {KIND_BATCH_SSSP, mix64((uint64_t)delta)}; }
 inline StepKey batch_pull_steps(int k) { return {KIND_BATCH_PULL, (uint64_t)k}; }
 
+// How a launch of teams ended (TeamsCtl::end, the largest of its rows').
+enum {
+    TEAMS_DONE = 0,
+    TEAMS_SHORT = 1,     // a row outgrew a team of fewer workgroups than it was to have (a busy GPU)
+    TEAMS_OUTGROWN = 2,  // a row outgrew a whole team
+    TEAMS_HUB = 3,       // a row reached a vertex of more out-edges than a team queues
+};
+
+// What a graph's batched searches of one kind found out about teams.
+struct TeamsRule {
+    int wgs = 0;        // least workgroups of a team, since smaller ones were outgrown (0: none yet)
+    int skip = 0;       // calls to come that don't try
+    int wait = 0;       // how many the last failure made it
+
+    // Whether this call tries (called once a call).
+    bool wanted() {
+        if (skip == 0) return true;
+        --skip;
+        return false;
+    }
+    // After a launch of teams of `wgs_now` workgroups that ended short of its rows: whether to
+    // run the call again by teams, else the general route takes it.  A larger team helps only
+    // where a whole one was outgrown; a short one says nothing about the graph, and gets one
+    // more try (`again`: it had that).  A failure that belongs to the graph and the sources is
+    // not repeated at once: the next 16 calls, then 64, 256, ... don't try.
+    bool retry(int end, int wgs_now, int wgs_most, bool again) {
+        if (end == TEAMS_SHORT) return !again;
+        if (end == TEAMS_OUTGROWN && wgs_now < wgs_most) {
+            wgs = 2 * wgs_now;
+            return true;
+        }
+        wait = wait == 0 ? 16 : wait < 1 << 20 ? 4 * wait : wait;
+        skip = wait;
+        return false;
+    }
+    void succeeded() { wait = 0; }
+};
+
 }  // namespace mg

@@ -53,7 +53,7 @@ __device__ __forceinline__ int rec_len(uint64_t r) { return (int)(r >> 62) + 1; 
 
 // What a member posts after a level (of its part of the next frontier): tag (the
 // meeting's number, 11 bits), overflow, records, vertices, out-edges.  A member
-// whose counts do not fit posts the overflow bit.
+// whose counts do not fit posts the overflow bit, and one record if a vertex has too many edges.
 __host__ __device__ constexpr uint64_t team_word(int tag, bool over, int rec, int nf, int mf) {
     return ((uint64_t)(tag & 0x7ff) << 53) | ((uint64_t)over << 52) | ((uint64_t)rec << 36) | ((uint64_t)nf << 20) |
            (uint64_t)mf;
@@ -75,6 +75,9 @@ struct TeamCtl {
 // The XCD this wave runs on (hardware register XCC_ID).
 __device__ __forceinline__ int xcd_id() { return (int)__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15; }
 
+// The whole wave: a vertex of too many edges is among what overflowed.
+__device__ __forceinline__ bool team_hub(uint64_t w) { return wave_ballot(team_over(w) && team_rec(w) != 0) != 0; }
+
 // Before the launch that forms the team (one workgroup of at least 2 * TEAM_SIZE threads):
 // nobody has joined, nothing is posted (meetings are numbered from 1).
 template <int = 0>
@@ -83,9 +86,10 @@ __global__ void team_open(TeamCtl *t) {
     if (threadIdx.x == 0) t->leader = t->joined = t->size = 0;
 }
 
-// Whole workgroup: joins the team of up to `wgs` (<= TEAM_WGS) workgroups.  False for workgroups that take no part; else this
-// wave's number among the team's `size` waves (a workgroup's waves lie `size` /
-// (BLK / WAVE) apart, so the first few members are on different CUs).
+// Whole workgroup: joins the team of up to `wgs` (<= TEAM_WGS) workgroups.  False for
+// workgroups that take no part; else this wave's number among the team's `size` waves (a
+// workgroup's waves lie `size` / (BLK / WAVE) apart, so the first few members are on
+// different CUs).
 __device__ __forceinline__ bool team_join(TeamCtl *t, int wgs, int &rank, int &size) {
     __shared__ int s_rank, s_size;
     if (threadIdx.x == 0) {
@@ -216,14 +220,14 @@ struct TeamSeat {
 struct TeamOut {
     uint64_t *recs;
     int nrec = 0, nf = 0, mf = 0;
-    bool over = false;
+    bool hub = false;
     __device__ TeamOut(uint64_t *all, int meeting, int rank)
         : recs(all + ((size_t)(meeting & 1) * TEAM_SIZE + rank) * TEAM_SEG) {}
     // Whole wave: queues vertex v with edge slots o.a..o.b for every lane with `first`
     // (`firsts`, not empty).
     __device__ __forceinline__ void queue(bool first, uint64_t firsts, int v, IntPair o) {
         const int deg = first ? o.b - o.a : 0;
-        if (wave_ballot(deg > TEAM_DEG)) over = true;
+        if (wave_ballot(deg > TEAM_DEG)) hub = true;
         // records and edges, one scan for both
         const int mine = min(deg, TEAM_DEG), mrec = (mine + TEAM_EDGES - 1) / TEAM_EDGES;
         const int sum = wave_scan_add(mrec << 16 | mine);
@@ -237,8 +241,8 @@ struct TeamOut {
         mf += all & 0xffff;
     }
     __device__ __forceinline__ uint64_t word(int meeting) const {
-        const bool o = over || nrec > TEAM_SEG || nf > 0xffff || mf > 0xfffff;
-        return o ? team_word(meeting, true, 0, 0, 0) : team_word(meeting, false, nrec, nf, mf);
+        const bool o = hub || nrec > TEAM_SEG || nf > 0xffff || mf > 0xfffff;
+        return o ? team_word(meeting, true, hub, 0, 0) : team_word(meeting, false, nrec, nf, mf);
     }
 };
 

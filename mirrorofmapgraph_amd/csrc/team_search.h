@@ -85,6 +85,7 @@ struct TeamSssp {
     int nwords, limit;
     long long delta, thr, unbucketed;  // no distance reaches a bound of `unbucketed`
     long long ex = 0;                  // edges this lane relaxed
+    bool hub = false;                  // overflowed at a vertex of too many edges
 };
 
 // Runs from meeting `it` (posted, frontier L) until the search ends or reaches its level
@@ -107,7 +108,10 @@ __device__ __forceinline__ bool team_sssp(const TeamSeat &t, TeamSssp &s, int &L
         const TeamIn in = team_in(t.recs, it, w);
         long long sweep_from = -1;  // >= 0: sweep, dropping waiting distances below this
         // the same decisions in every wave
-        if (wave_ballot(team_over(w)) != 0) break;
+        if (wave_ballot(team_over(w)) != 0) {
+            s.hub = team_hub(w);
+            break;
+        }
         if (!swept) closed(w);
         if (L >= limit) {
             done = true;

@@ -606,3 +606,61 @@ def test_batched_routes_given_up_hold_no_memory(mg, oracle, device, monkeypatch,
             return dg.device_bytes() - before
 
     assert grown(False) == grown(True)
+
+
+def _widening(mg, first, doublings):
+    """A tree: `first` vertices below the root, then twice as many a level; the last level holds most."""
+    src, dst, at, level = [np.zeros(first, np.int64)], [np.arange(1, first + 1)], first + 1, np.arange(1, first + 1)
+    for _ in range(doublings):
+        kids = np.arange(at, at + 2 * len(level))
+        src.append(np.repeat(level, 2)), dst.append(kids)
+        at, level = at + len(kids), kids
+    g = mg.csr_from_edges(at, np.concatenate(src).astype(np.int32), np.concatenate(dst).astype(np.int32),
+                          mg.MG_CSR_SYMMETRIZE | mg.MG_CSR_SORT_COLS)
+    g.values = mg.hash_weights(g, 3, 9)
+    return g
+
+
+@pytest.mark.parametrize("sssp", [False, True])
+def test_batch_teams_short_of_workgroups_are_tried_again(mg, oracle, device, monkeypatch, sssp):
+    # the last level needs most of a team's sixteen workgroups; here teams close with one
+    g = _widening(mg, 6, 12)
+    srcs = np.zeros(8, np.int32)
+    one = oracle.sssp(g.row_offsets, g.col_idx, g.values, 0) if sssp else oracle.bfs(g.row_offsets, g.col_idx, 0)
+    o = mg.options(sssp_delta=-1)
+    with mg.Graph(g, symmetric=True) as dg:
+        monkeypatch.setenv("MG_TEAM_LAUNCH", "1")
+        for _ in range(3):
+            for row in dg.sssp_batch(srcs, o) if sssp else dg.bfs_batch(srcs):
+                assert np.array_equal(row, one)
+        monkeypatch.delenv("MG_TEAM_LAUNCH")
+        before = dg.device_bytes()  # the general route's state: the teams' was released
+        for row in dg.sssp_batch(srcs, o) if sssp else dg.bfs_batch(srcs):
+            assert np.array_equal(row, one)
+        assert dg.device_bytes() > before  # the teams' state is there: they took the call
+
+
+@pytest.mark.parametrize("sssp", [False, True])
+def test_batch_teams_beside_a_hub_in_another_component(mg, oracle, device, sssp):
+    # a vertex that no team queues in one component; searches of the other one are taken by teams again
+    a, b = mg.grid_graph(40, 30, seed=3), mg.grid_graph(50, 40, seed=4)
+    n, hub = a.n + b.n + 1500, 7
+    src = np.concatenate([np.repeat(np.arange(a.n), np.diff(a.row_offsets)),
+                          np.repeat(np.arange(b.n), np.diff(b.row_offsets)) + a.n, np.full(1500, hub)])
+    dst = np.concatenate([a.col_idx, b.col_idx + a.n, np.arange(a.n + b.n, n)])
+    g = mg.csr_from_edges(n, src.astype(np.int32), dst.astype(np.int32),
+                          mg.MG_CSR_SYMMETRIZE | mg.MG_CSR_DEDUPE | mg.MG_CSR_SORT_COLS)
+    g.values = mg.hash_weights(g, 3, 9)
+    one = (lambda s: oracle.sssp(g.row_offsets, g.col_idx, g.values, s)) if sssp else (
+        lambda s: oracle.bfs(g.row_offsets, g.col_idx, s))
+    near, far = np.array([0, hub, a.n - 1], np.int32), np.arange(a.n, a.n + 3, dtype=np.int32)
+    with mg.Graph(g, symmetric=True) as dg:
+        batch = dg.sssp_batch if sssp else dg.bfs_batch
+        assert np.array_equal(batch(near), np.stack([one(int(s)) for s in near]))
+        before, exp = dg.device_bytes(), np.stack([one(int(s)) for s in far])
+        for calls in range(40):
+            assert np.array_equal(batch(far), exp)
+            if dg.device_bytes() > before:  # the teams' state is there again
+                break
+        assert calls < 39
+        assert np.array_equal(batch(near), np.stack([one(int(s)) for s in near]))

@@ -39,3 +39,39 @@ def test_pushed_and_pulled_batches_never_share_steps(tmp_path):
     printf("%ld", same);
     """)
     assert out == "0"
+
+
+def test_teams_grow_only_where_a_whole_team_was_outgrown(tmp_path):
+    out = run(tmp_path, """
+    {   // short of workgroups: one more try, and nothing to remember, however often it happens
+        TeamsRule r;
+        for (int call = 0; call < 100; ++call)
+            if (!r.wanted() || !r.retry(TEAMS_SHORT, 16, 16, false) || r.retry(TEAMS_SHORT, 16, 16, true)) return 1;
+        if (r.wgs || r.skip || r.wait) return 2;
+    }
+    {   // a vertex no team takes: no larger teams
+        TeamsRule r;
+        if (!r.wanted() || r.retry(TEAMS_HUB, 2, 16, false) || r.wgs) return 3;
+    }
+    {   // outgrown: doubled up to the largest, then the general route
+        TeamsRule r;
+        int wgs = 2, tries = 0;
+        while (r.retry(TEAMS_OUTGROWN, wgs, 16, false)) wgs = r.wgs, ++tries;
+        if (wgs != 16 || tries != 3 || r.wanted()) return 4;
+    }
+    // tries of a graph whose calls all fail, and the calls until one that would not fail is tried
+    TeamsRule r;
+    int tries = 0;
+    for (int call = 0; call < 100000; ++call)
+        if (r.wanted()) {
+            ++tries;
+            r.retry(TEAMS_HUB, 16, 16, false);
+        }
+    TeamsRule s;
+    s.retry(TEAMS_HUB, 16, 16, false);
+    int until = 1;
+    while (!s.wanted()) ++until;
+    s.succeeded();
+    printf("%d %d %d", tries, until, s.wanted());
+    """)
+    assert out == "8 17 1"  # 16 + 64 + 256 + ... calls between them
