@@ -32,7 +32,7 @@ struct BfsArgs {
     uint32_t *visited;
     int *hard;
     int G;               // workgroups of the level kernels
-    int team;            // narrow searches pause for a team (bfs_team)
+    int team;            // narrow searches pause for a team (bfs_team), at first after so many levels; 0: they don't
 };
 
 // Visit of edge (v, u) at level L: claim u through the visited bitmap, label it and
@@ -112,6 +112,7 @@ __global__ void bfs_begin(BfsArgs a, int src, int iter_limit, int can_bu, int al
     Ctl *c = a.fa.ctl;
     a.fa.q[0][0] = src;
     ctl_reset(c, a.fa.n, iter_limit, 1);
+    c->team_after = a.team;
     const long long d = view_degree(a.fa, src);
     c->can_bu = can_bu;
     c->alpha = alpha > 0 ? alpha : 14;
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(SMALL_BLK) void bfs_small(BfsArgs a) {
     __shared__ int s_q[SMALL_Q];
     __shared__ int s_big[SMALL_BIG];
     __shared__ int s_bpre[SMALL_BIG], s_bbeg[SMALL_BIG], s_bwave[SMALL_BLK / WAVE];
-    __shared__ int s_go, s_L, s_cnt, s_nbig, s_levels, s_dir, s_canbu, s_alpha, s_limit, s_narrow;
+    __shared__ int s_go, s_L, s_cnt, s_nbig, s_levels, s_dir, s_canbu, s_alpha, s_limit, s_after;
     __shared__ long long s_mu;
     if (c->pending) {
         const int L = c->level;
@@ -156,7 +157,7 @@ __global__ __launch_bounds__(SMALL_BLK) void bfs_small(BfsArgs a) {
     int n0 = 0, qv = 0;
     if (threadIdx.x == 0) {
         const int L = c->level;
-        s_narrow = c->small_levels;
+        s_after = c->team_after;
         s_go = !c->done && c->dir == DIR_TD && c->qsize[L % 3] <= SMALL_Q && c->mf_cur <= SMALL_E;
         s_L = L;
         s_mu = c->m_unexplored;
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(SMALL_BLK) void bfs_small(BfsArgs a) {
             s_levels++;
             const bool go = nf > 0 && nf <= SMALL_Q && dir == DIR_TD && mf <= SMALL_E && L + 1 < s_limit;
             // a search that stays narrow is handed to a team
-            const bool to_team = go && a.team && s_narrow + s_levels >= TEAM_AFTER;
+            const bool to_team = go && a.team && s_levels >= s_after;
             s_go = to_team ? 2 : go;
             s_L = L + 1;
             if (!go || to_team) {
@@ -468,6 +469,7 @@ __global__ __launch_bounds__(BLK) void bfs_team(BfsArgs a, TeamCtl *team, uint64
     if (lead) {
         c->m_unexplored = mu;
         c->small_levels += L - L0;
+        c->team_after = team_after_next(c->team_after, L - L0);
         c->level = L - 1;
         c->pending = 1;
         c->qvalid = 0;
@@ -682,7 +684,7 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
     a.hard = ws.hard;
     a.G = o.level_grid > 0 ? o.level_grid : level_blocks(g->n, g->m, 64, MAX_GRID);
     // (search views serve graphs that are not thin, within a byte budget: no team there)
-    a.team = a.fa.nviews == 1 && !g->arrays_borrowed;
+    a.team = a.fa.nviews == 1 && !g->arrays_borrowed ? g->steps->team_after[0] : 0;
     const long long m_views = g->m * a.fa.nviews;
 
     MG_HIP(hipEventRecord(g->ev0, g->stream));
@@ -713,6 +715,7 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
                     tail, &tail_queued, team)))
         return rc;
     rc = finish_search(g, stats, ws.vals, -1, ws.vals, 4 * (size_t)g->n, to, timer, tail_queued);
+    if (a.team) g->steps->team_after[0] = team_after_start(ws.h_ctl->team_after);
     if (rc == MG_OK && o.verbose) rc = print_trace(g, "bfs", "top-down", "bottom-up");
     return rc;
 }

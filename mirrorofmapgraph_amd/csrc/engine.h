@@ -87,6 +87,7 @@ struct Ctl {
     int pair_end;             // batched SSSP: pair slots below this are valid this iteration
     long long fmin;           // SSSP: a lower bound on the distances of the current frontier
     int team_step;            // BFS / SSSP: steps run when the first team took over (0: none did)
+    int team_after;           // narrow levels in a row before a team is asked for (team_after_next)
 };
 
 struct TeamCtl;
@@ -341,6 +342,7 @@ struct mg_graph_steps {
     // What batched searches found out about the graph (kept when the routes' state is released)
     bool pull_deep = false;              // SSSP took too many rounds to be pulled
     mg::TeamsRule teams_rule[2];         // BFS, SSSP
+    int team_after[2] = {mg::TEAM_AFTER, mg::TEAM_AFTER};  // where the next BFS / SSSP starts (team_after_start)
 };
 
 // Queues steps until the device reports `done`.  Steps run from a captured HIP graph

@@ -617,6 +617,7 @@ __device__ __forceinline__ void ctl_reset(Ctl *c, int n, int iter_limit, int fro
     c->dsum = 0;
     c->mf_cur = 0;
     c->team_step = 0;
+    c->team_after = 0;
 }
 
 // Advances the control block past level L given the next frontier's size nf and

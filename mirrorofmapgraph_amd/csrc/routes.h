@@ -20,6 +20,20 @@ struct StepKey {
 inline StepKey batch_sssp_steps(long long delta) { return {KIND_BATCH_SSSP, mix64((uint64_t)delta)}; }
 inline StepKey batch_pull_steps(int k) { return {KIND_BATCH_PULL, (uint64_t)k}; }
 
+// Narrow levels in a row that the single workgroup runs before a team takes over (team.h): at
+// first, after a team that ran `levels` levels when it was asked for after `after`, and at the
+// start of the graph's next search.  The hand-over and the way back cost some ten levels of
+// the single workgroup (the steps queued behind the pause, a wait of the host, the frontier
+// rebuilt from the depths), so a team that soon outgrows its queues or meets a hub has to be
+// waited for four times as long.  Asking again after a single narrow level, searches that
+// alternate took up to nine times as long as without teams (300 stars of 1100 leaves on a
+// path: SSSP 9.4 -> 82 ms, so 9.6).
+constexpr int TEAM_AFTER = 8;
+constexpr int team_after_next(int after, int levels) {
+    return levels >= 4 * TEAM_AFTER || after >= 1 << 20 ? after : 4 * after;
+}
+constexpr int team_after_start(int last) { return last / 4 > TEAM_AFTER ? last / 4 : TEAM_AFTER; }
+
 // How a launch of teams ended (TeamsCtl::end, the largest of its rows').
 enum {
     TEAMS_DONE = 0,

@@ -44,7 +44,7 @@ struct SsspArgs {
     int bucketed;
     long long bucket_edges;
     int wmin;  // smallest edge weight (>= 0)
-    int team;  // narrow searches pause for a team (sssp_team)
+    int team;  // narrow searches pause for a team (sssp_team), at first after so many levels; 0: they don't
 };
 
 constexpr long long UNBUCKETED = LLONG_MAX / 4;  // a bucket bound no distance reaches
@@ -625,6 +625,7 @@ __global__ void sssp_begin(SsspArgs a, int src, int iter_limit, int can_pull, lo
     Ctl *c = a.fa.ctl;
     a.fa.q[0][0] = src;
     ctl_reset(c, a.fa.n, iter_limit, 1);
+    c->team_after = a.team;
     c->thr = a.delta;  // the first bucket: [0, delta)
     c->fmin = 0;
     c->mf_cur = view_degree(a.fa, src);
@@ -673,7 +674,7 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
     __shared__ int s_beg[2 * SMALL_Q];       // list starts
     __shared__ int s_d[SMALL_Q];             // frontier distances
     __shared__ int s_wave[SMALL_BLK / WAVE];
-    __shared__ int s_go, s_L, s_cnt, s_levels, s_limit, s_canpull, s_alpha, s_nfar, s_keep, s_qv, s_nq, s_narrow;
+    __shared__ int s_go, s_L, s_cnt, s_levels, s_limit, s_canpull, s_alpha, s_nfar, s_keep, s_qv, s_nq, s_after;
     __shared__ long long s_m, s_thr;
     if (c->pending) {
         const int L = c->level;
@@ -689,7 +690,7 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
     }
     if (threadIdx.x == 0) {
         const int L = c->level;
-        s_narrow = c->small_levels;
+        s_after = c->team_after;
         s_go = !c->done && c->dir == DIR_PUSH && c->qsize[L % 3] <= SMALL_Q && c->mf_cur <= SSSP_SMALL_E;
         s_L = L;
         s_cnt = c->qsize[L % 3];
@@ -959,7 +960,7 @@ __global__ __launch_bounds__(SMALL_BLK) void sssp_small(SsspArgs a) {
             const bool go = nf > 0 && nf <= SMALL_Q && !(s_canpull && mf * s_alpha > s_m) && mf <= SSSP_SMALL_E &&
                             L + 1 < s_limit;
             // a search that stays narrow is handed to a team
-            s_go = go && a.team && s_narrow + s_levels >= TEAM_AFTER ? 2 : go;
+            s_go = go && a.team && s_levels >= s_after ? 2 : go;
             s_L = L + 1;
             s_keep = nf;
         }
@@ -1104,6 +1105,7 @@ __global__ __launch_bounds__(BLK) void sssp_team(SsspArgs a, TeamCtl *team, uint
     write_part<BLK>(fa, nf, mf, s.ex, mn);
     if (lead) {
         c->small_levels += L - L0;
+        c->team_after = team_after_next(c->team_after, L - L0);
         c->level = L - 1;
         c->thr = s.thr;
         c->pending = 1;
@@ -1199,7 +1201,7 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     a.farbm = ws.visited;
     a.wmin = g->min_weight;
     // (search views serve graphs that are not thin, within a byte budget: no team there)
-    a.team = a.fa.nviews == 1 && !g->arrays_borrowed;
+    a.team = a.fa.nviews == 1 && !g->arrays_borrowed ? g->steps->team_after[1] : 0;
     const int in_view = a.fa.off[2] != nullptr && a.fa.nviews == 1 && o.engine != MG_ENGINE_GAS;
     // pull levels relax every vertex from all its in-edges: unbucketed searches only
     const int can_pull = in_view && !a.bucketed;
@@ -1246,6 +1248,7 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     if ((rc = drive(g, step, max_steps, KIND_SSSP, key, nullptr, nullptr, tail, &tail_queued, team)))
         return rc;
     rc = finish_search(g, stats, ws.vals, INT_MAX, ws.vals, 4 * (size_t)g->n, to, timer, tail_queued);
+    if (a.team) g->steps->team_after[1] = team_after_start(ws.h_ctl->team_after);
     if (rc == MG_OK && o.verbose) rc = print_trace(g, "sssp", "push", "pull");
     return rc;
 }

@@ -37,7 +37,6 @@ constexpr int TEAM_EDGES = 4;        // edges per record, a lane each
 constexpr int TEAM_PIECE = WAVE / TEAM_EDGES;  // records a wave takes at a time
 constexpr int TEAM_DEG = 1020;       // out-edges of a vertex a team queues (64 fit team_word's fields)
 constexpr int TEAM_GATHER = 1000;    // ticks (100 MHz) the first member waits for others
-constexpr int TEAM_AFTER = 8;        // narrow levels run by the single workgroup before a team takes over
 constexpr int TEAM_CLOSED = 1 << 29;
 
 // Records: 1..TEAM_EDGES consecutive edge slots of a frontier vertex, TEAM_SEG records

@@ -664,3 +664,13 @@ def test_batch_teams_beside_a_hub_in_another_component(mg, oracle, device, sssp)
                 break
         assert calls < 39
         assert np.array_equal(batch(near), np.stack([one(int(s)) for s in near]))
+
+
+@pytest.mark.parametrize("leaves,length", [(1100, 3), (1100, 12), (3000, 9)])
+def test_searches_that_alternate_between_teams_and_the_single_workgroup(mg, oracle, device, leaves, length):
+    # every star sends a team back; later searches of the graph start from what the earlier ones found
+    g = _chain(mg, [length] * 40, [leaves] * 39 + [0], 6)
+    with mg.Graph(g, symmetric=True) as dg:
+        for src in (0, g.n - 1, g.n // 2, 0, 0):
+            assert np.array_equal(dg.bfs(src), oracle.bfs(g.row_offsets, g.col_idx, src))
+            assert np.array_equal(dg.sssp(src), oracle.sssp(g.row_offsets, g.col_idx, g.values, src))

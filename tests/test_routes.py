@@ -75,3 +75,31 @@ def test_teams_grow_only_where_a_whole_team_was_outgrown(tmp_path):
     printf("%d %d %d", tries, until, s.wanted());
     """)
     assert out == "8 17 1"  # 16 + 64 + 256 + ... calls between them
+
+
+def test_a_team_that_soon_hands_back_is_asked_for_less_often(tmp_path):
+    # pauses of searches of 100,000 narrow levels whose teams run a given number of levels each: the
+    # graph's first search, a later one, and one whose teams run long again after them
+    out = run(tmp_path, """
+    for (int levels : {0, 4, 31, 32, 1000}) {
+        int start = TEAM_AFTER;
+        auto search = [&](int levels) {
+            long at = 0, pauses = 0;
+            int after = start;
+            for (; (at += after) < 100000; at += levels) {
+                ++pauses;
+                after = team_after_next(after, levels);
+            }
+            start = team_after_start(after);
+            return pauses;
+        };
+        printf("%ld ", search(levels));
+        printf("%ld ", search(levels));
+        for (int i = 0; i < 10; ++i) search(1000);
+        printf("%ld ", search(1000));
+    }
+    """)
+    rows = [tuple(map(int, out.split()[3 * i: 3 * i + 3])) for i in range(5)]
+    assert all(r[0] <= 7 and r[1] <= 2 for r in rows[:3])
+    assert rows[3][:2] == (2500, 2500) and rows[4][0] <= 100
+    assert all(r[2] == rows[4][0] for r in rows)
