@@ -704,8 +704,6 @@ static int bfs_run(mg_graph *g, int src, int *depth_out, const mg_options &o, mg
     const Delivery to = plan_delivery(g, depth_out, 4 * (size_t)g->n, o.out_on_device);
     auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, -1, ws.vals, 4 * (size_t)g->n, to); };
     auto team = [&]() -> int {
-        const int trc = ensure_team(g);
-        if (trc) return trc;
         hipLaunchKernelGGL(team_open<>, dim3(1), dim3(2 * TEAM_SIZE), 0, g->stream, ws.team);
         hipLaunchKernelGGL(bfs_team, dim3(TEAM_GRID), dim3(BLK), 0, g->stream, a, ws.team, ws.team_rec);
         MG_HIP(hipGetLastError());

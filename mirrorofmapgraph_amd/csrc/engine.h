@@ -106,8 +106,8 @@ struct Workspace {
     uint32_t *visited = nullptr;
     uint32_t *bm[3] = {nullptr, nullptr, nullptr};
     ChunkRec *chunks = nullptr;
-    LevelPart *part = nullptr;  // 3 * BIG_GRID slots
-    TeamCtl *team = nullptr;  // team of the narrow levels and its queues (team.h; on first use)
+    LevelPart *part = nullptr;  // PART_GROUPS slots
+    TeamCtl *team = nullptr;  // team of the narrow levels and its queues (team.h; not on search views)
     uint64_t *team_rec = nullptr;
     Ctl *ctl = nullptr;
     Ctl *h_ctl = nullptr;     // pinned host mirror
@@ -223,7 +223,6 @@ void invalidate_steps(mg_graph *g);
 // The same for one kind of steps.
 void invalidate_steps(mg_graph *g, int kind);
 int ensure_pr_workspace(mg_graph *g);
-int ensure_team(mg_graph *g);
 int alloc_i32(int32_t **p, size_t n);
 int alloc_f32(float **p, size_t n);
 int alloc_chunks(ChunkRec **p, size_t n);

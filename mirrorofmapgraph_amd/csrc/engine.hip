@@ -117,9 +117,10 @@ int ensure_workspace(mg_graph *g) {
         (rc = dalloc(&ws.q[2], n)) || (rc = dalloc(&ws.hard, n)) || (rc = dalloc(&ws.visited, ws.nwords)) ||
         (rc = dalloc(&ws.bm[0], ws.nwords)) || (rc = dalloc(&ws.bm[1], ws.nwords)) ||
         (rc = dalloc(&ws.bm[2], ws.nwords)) || (rc = dalloc(&ws.chunks, ws.chunk_cap)) ||
-        (rc = dalloc(&ws.part, 3 * BIG_GRID)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2 * TAIL_WGS)) ||
+        (rc = dalloc(&ws.part, PART_GROUPS)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2 * TAIL_WGS)) ||
         (rc = dalloc(&ws.tail_cnt, LAST_WG_INTS)) ||
-        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP))) {
+        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP)) ||
+        (!g->arrays_borrowed && ((rc = dalloc(&ws.team, 1)) || (rc = dalloc(&ws.team_rec, TEAM_RECS))))) {
         free_workspace(ws);
         return rc;
     }
@@ -133,14 +134,6 @@ int ensure_workspace(mg_graph *g) {
         return set_error(MG_ERR_OOM, "hipHostMalloc failed: %s", hipGetErrorString(e));
     }
     return MG_OK;
-}
-
-int ensure_team(mg_graph *g) {
-    Workspace &ws = g->ws;
-    if (ws.team) return MG_OK;
-    int rc = 0;
-    if ((rc = dalloc(&ws.team, 1)) || (rc = dalloc(&ws.team_rec, TEAM_RECS))) dfree(ws.team);
-    return rc;
 }
 
 int ensure_pr_workspace(mg_graph *g) {

@@ -1238,8 +1238,6 @@ static int sssp_run(mg_graph *g, int src, int *dist_out, const mg_options &o, mg
     const Delivery to = plan_delivery(g, dist_out, 4 * (size_t)g->n, o.out_on_device);
     auto tail = [&]() { return queue_finish(g, stats != nullptr, ws.vals, INT_MAX, ws.vals, 4 * (size_t)g->n, to); };
     auto team = [&]() -> int {
-        const int trc = ensure_team(g);
-        if (trc) return trc;
         hipLaunchKernelGGL(team_open<>, dim3(1), dim3(2 * TEAM_SIZE), 0, g->stream, ws.team);
         hipLaunchKernelGGL(sssp_team, dim3(TEAM_GRID), dim3(BLK), 0, g->stream, a, ws.team, ws.team_rec);
         MG_HIP(hipGetLastError());

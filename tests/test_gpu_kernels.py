@@ -674,3 +674,14 @@ def test_searches_that_alternate_between_teams_and_the_single_workgroup(mg, orac
         for src in (0, g.n - 1, g.n // 2, 0, 0):
             assert np.array_equal(dg.bfs(src), oracle.bfs(g.row_offsets, g.col_idx, src))
             assert np.array_equal(dg.sssp(src), oracle.sssp(g.row_offsets, g.col_idx, g.values, src))
+
+
+def test_a_search_needs_no_memory_for_its_team(mg, oracle, device, monkeypatch):
+    g = mg.grid_graph(90, 70, seed=2, weight_max=16)
+    with mg.Graph(g, symmetric=True) as dg:
+        dg.sssp(0, mg.options(iter_num=2))  # (the tasks of the dense levels, made by the first search)
+        for fn, exp in ((dg.bfs, oracle.bfs(g.row_offsets, g.col_idx, 0)),
+                        (dg.sssp, oracle.sssp(g.row_offsets, g.col_idx, g.values, 0))):
+            monkeypatch.setenv("MG_FAIL_ALLOC_AT", "1")
+            assert np.array_equal(fn(0), exp)
+            monkeypatch.delenv("MG_FAIL_ALLOC_AT")
