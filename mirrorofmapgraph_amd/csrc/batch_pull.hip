@@ -83,6 +83,7 @@ __global__ void pull_init(PullArgs a, int lanes, int iter_limit) {
     if (threadIdx.x != 0) return;
     ctl_reset(a.ctl, a.n, iter_limit, 1);
     a.ctl->fmin = 0;
+    a.ctl->aux = a.k;
 }
 
 __global__ void pull_seed(PullArgs a, int lanes, SeedList sl) {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(BLK) void pull_round(PullArgs a) {
     const int *low = a.low[L % 3];
     int *low_next = a.low[(L + 1) % 3], *low_clear = a.low[(L + 2) % 3];
     uint4 *D4 = reinterpret_cast<uint4 *>(a.D);
-    const bool used = 4 * gl < a.k;
+    const bool used = 4 * gl < c->aux;  // (a.k is the capturing call's)
     // this lane's live slots, as masks over their distances
     const uint32_t lw = a.live[8 * (L % 3) + gl / 8] >> (4 * (gl % 8));
     const uint4 on = make_uint4(lw & 1 ? ~0u : 0u, lw & 2 ? ~0u : 0u, lw & 4 ? ~0u : 0u, lw & 8 ? ~0u : 0u);
@@ -380,10 +381,15 @@ __global__ __launch_bounds__(BLK) void pull_rows(PullArgs a, int ks, const int *
 
 // ---------------------------------------------------------------- host side
 
+// The captured rounds, which point at the state's buffers.
+static void pull_drop_steps(mg_graph *g) {
+    for (int w = 0; w < 4; ++w) invalidate_steps(g, KIND_BATCH_PULL + w);
+}
+
 void pull_release(mg_graph *g) {
     PullDev *&p = g->steps->pull;
     if (!p) return;
-    invalidate_steps(g, KIND_BATCH_PULL);  // captured rounds point at these buffers
+    pull_drop_steps(g);
     free_dev(p->ctl);
     if (p->h_ctl) (void)hipHostFree(p->h_ctl);
     free_dev(p->part);
@@ -446,7 +452,7 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
     PullDev *&pp = g->steps->pull;
     if (!pp && !(pp = new (std::nothrow) PullDev())) return set_error(MG_ERR_OOM, "host allocation failed");
     PullDev &p = *pp;
-    const int lanes = k <= 32 ? 8 : k <= 64 ? 16 : k <= 128 ? 32 : 64, ks = 4 * lanes;
+    const int lanes = pull_lanes(k), ks = 4 * lanes;
     if (!p.ctl) {
         int *c = nullptr, *l = nullptr;
         if ((rc = alloc_i32(&c, sizeof(Ctl) / 4)) || (rc = alloc_parts(&p.part, PART_GROUPS)) ||
@@ -465,7 +471,7 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
     auto grow = [&](int **buf, int64_t *cap, int64_t need) -> int {
         if (*cap >= need) return MG_OK;
         MG_HIP(hipStreamSynchronize(g->stream));
-        invalidate_steps(g, KIND_BATCH_PULL);  // captured rounds point at the old buffer
+        pull_drop_steps(g);
         free_dev(*buf);
         *buf = nullptr;
         p.bytes -= 4 * *cap;
@@ -519,7 +525,6 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
         MG_HIP(hipGetLastError());
         return MG_OK;
     };
-    // the captured rounds read k and the row width from their arguments
     const StepKey sk = batch_pull_steps(k);
     if ((rc = drive(g, step, PULL_ROUNDS + 2, sk.kind, sk.key, p.ctl, p.h_ctl))) return rc;
     if (p.h_ctl->changed & PULL_DEEP) {

@@ -74,7 +74,7 @@ struct Ctl {
     int changed;        // generic "something changed" counter / overflow flag (bit 30)
     int pending;        // a multi-workgroup level finished and awaits its close
     int qvalid;         // bit i: queue q[i] lists the frontier of bitmap bm[i]
-    int aux;            // search-specific (CC: root of the sampled large component)
+    int aux;            // search-specific (CC: root of the sampled large component; pulled SSSP: sources)
     long long mf_next;        // sum of out-degrees of vertices found this level
     long long m_unexplored;   // out-edges of unreached vertices
     long long edges_traversed;// reference TEPS count

@@ -7,8 +7,9 @@
 
 namespace mg {
 
-// Kinds of captured steps a graph keeps, one executable graph each.
-enum { KIND_BFS = 0, KIND_SSSP = 1, KIND_PR = 2, KIND_GAS = 3, KIND_BATCH = 4, KIND_BATCH_SSSP = 5, KIND_BATCH_PULL = 6, NKINDS = 8 };
+// Kinds of captured steps a graph keeps, one executable graph each (KIND_BATCH_PULL: four, by
+// row width).
+enum { KIND_BFS = 0, KIND_SSSP = 1, KIND_PR = 2, KIND_GAS = 3, KIND_BATCH = 4, KIND_BATCH_SSSP = 5, KIND_BATCH_PULL = 6, NKINDS = 10 };
 
 // What a batched search's captured steps are kept under.  Two routes whose steps work on
 // different state never share one: a search that found the other route's steps would replay
@@ -18,7 +19,13 @@ struct StepKey {
     uint64_t key;
 };
 inline StepKey batch_sssp_steps(long long delta) { return {KIND_BATCH_SSSP, mix64((uint64_t)delta)}; }
-inline StepKey batch_pull_steps(int k) { return {KIND_BATCH_PULL, (uint64_t)k}; }
+// Pulled rows: 32, 64, 128 or 256 distances a vertex, four a lane.  k itself is read from
+// device memory, so calls of any sizes replay the rounds of their width: keyed on k, a caller
+// whose batches vary captured them again on each call (R-MAT scale 16, 17 to 28 sources: 968
+// us a call, 796 with k fixed).
+inline int pull_width(int k) { return k <= 32 ? 0 : k <= 64 ? 1 : k <= 128 ? 2 : 3; }
+inline int pull_lanes(int k) { return 8 << pull_width(k); }
+inline StepKey batch_pull_steps(int k) { return {KIND_BATCH_PULL + pull_width(k), 0}; }
 
 // Narrow levels in a row that the single workgroup runs before a team takes over (team.h): at
 // first, after a team that ran `levels` levels when it was asked for after `after`, and at the

@@ -685,3 +685,14 @@ def test_a_search_needs_no_memory_for_its_team(mg, oracle, device, monkeypatch):
             monkeypatch.setenv("MG_FAIL_ALLOC_AT", "1")
             assert np.array_equal(fn(0), exp)
             monkeypatch.delenv("MG_FAIL_ALLOC_AT")
+
+
+def test_batch_pull_sizes_that_share_a_row_width(mg, oracle, device):
+    # larger and smaller calls in turn on one graph, as many columns as the width has and one
+    g = random_graph(mg, 1501, 12000, 6, wmax=30)
+    srcs = np.random.default_rng(1).integers(0, g.n, 64).astype(np.int32)
+    exp = np.stack([oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)) for s in srcs])
+    with mg.Graph(g, symmetric=True) as dg:
+        for k in (1, 32, 3, 31, 32, 4, 33, 64, 35, 64, 5):
+            for lo in (0, 64 - k):
+                assert np.array_equal(dg.sssp_batch(srcs[lo:lo + k]), exp[lo:lo + k]), (k, lo)

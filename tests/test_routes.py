@@ -103,3 +103,17 @@ def test_a_team_that_soon_hands_back_is_asked_for_less_often(tmp_path):
     assert all(r[0] <= 7 and r[1] <= 2 for r in rows[:3])
     assert rows[3][:2] == (2500, 2500) and rows[4][0] <= 100
     assert all(r[2] == rows[4][0] for r in rows)
+
+
+def test_pulled_batches_of_one_row_width_share_their_steps(tmp_path):
+    out = run(tmp_path, """
+    int changes = 0;
+    for (int k = 1; k <= MG_BATCH_MAX; ++k) {
+        const StepKey a = batch_pull_steps(k), b = batch_pull_steps(k > 1 ? k - 1 : 1);
+        if (4 * pull_lanes(k) < k || 64 % pull_lanes(k) || a.kind >= NKINDS || a.kind < KIND_BATCH_PULL) return 1;
+        changes += a.kind != b.kind;
+        if (a.key != b.key || (a.kind != b.kind) != (pull_lanes(k) != pull_lanes(k > 1 ? k - 1 : 1))) return 2;
+    }
+    printf("%d", changes);
+    """)
+    assert out == "3"  # one slot a width, so calls of several widths do not capture in turn either
