@@ -315,9 +315,10 @@ typedef struct mg_server_config {
                                  (0 = 5000; -1 = runs to the end in one launch)          */
     int32_t ppr_gate_us;      /* personalized PageRank cohorts: an idle engine starts when
                                  ppr_batch_min queries wait or the oldest has waited this
-                                 long (0 = 20000, or 70000 while queries of other engines
-                                 run; -1 = every query starts on arrival)               */
-    int32_t ppr_batch_min;    /* (0 = 8, or 16 while others run; at most 64)             */
+                                 long (0 = 20000, or 70000 while at least 64 queries of
+                                 other engines run or wait; -1 = every query starts on
+                                 arrival)                                               */
+    int32_t ppr_batch_min;    /* (0 = 8, or 16 beside those 64; at most 64)              */
     int32_t plain_kinds;      /* bit k set (1 << MG_Q_BFS, 1 << MG_Q_SSSP): those queries on
                                  graphs that are not thin run as whole-GPU searches
                                  (mg_bfs / mg_sssp, the graph's twin included), two at a

@@ -406,14 +406,8 @@ static int thin_round(Server &s, Engine &e, bool *queued) {
 // loaded engine sweeping nonstop for one or two queries at a time.  An idle engine
 // starts when ppr_batch_min queries wait or the oldest has waited ppr_gate_us, and a
 // running cohort takes new queries during its first PPR_JOIN iterations only; the
-// others start the next cohort.  By default a gate is longer while other engines run: a
-// faster sweep otherwise ends sooner, starts again for fewer queries and keeps the memory
-// as busy (benchmark mix of 2000 queries/s, 20 ms and 8 queries / 70 ms and 16: median of
-// all queries 74 / 39 ms, 99th percentile 440 / 330, SSSP at R-MAT scale 22 20 / 12.5 ms
-// of service).
+// others start the next cohort (ppr_gate).
 constexpr int PPR_JOIN = 8;
-constexpr int PPR_GATE_US = 20000, PPR_BATCH = 8;              // alone
-constexpr int PPR_GATE_BUSY_US = 70000, PPR_BATCH_BUSY = 16;   // beside running queries of other engines
 static bool ppr_admits(const Server &s, const Engine &e) {
     if (s.cfg.ppr_gate_us < 0 || e.waiting.empty()) return true;
     if (e.running > 0) {
@@ -422,11 +416,11 @@ static bool ppr_admits(const Server &s, const Engine &e) {
             if (r) most = std::max(most, s.cfg.ppr_iters - r->iters_left);
         return most < PPR_JOIN;
     }
-    bool busy = false;
-    for (const auto &o : s.engines) busy = busy || (o && o.get() != &e && o->running > 0);
-    const int batch = s.cfg.ppr_batch_min > 0 ? s.cfg.ppr_batch_min : busy ? PPR_BATCH_BUSY : PPR_BATCH;
-    const double gate_ms = (s.cfg.ppr_gate_us > 0 ? s.cfg.ppr_gate_us : busy ? PPR_GATE_BUSY_US : PPR_GATE_US) / 1000.0;
-    return (int)e.waiting.size() >= batch || s.now() - e.waiting.front()->t_submit >= gate_ms;
+    int64_t others = 0;
+    for (const auto &o : s.engines)
+        if (o && o.get() != &e) others += o->running + (int64_t)o->waiting.size();
+    const PprGate gate = ppr_gate(s.cfg.ppr_gate_us, s.cfg.ppr_batch_min, others);
+    return (int)e.waiting.size() >= gate.batch || s.now() - e.waiting.front()->t_submit >= gate.us / 1000.0;
 }
 
 // One round of an engine; returns true if it queued work.  Called with s.mu held.

@@ -117,3 +117,14 @@ def test_pulled_batches_of_one_row_width_share_their_steps(tmp_path):
     printf("%d", changes);
     """)
     assert out == "3"  # one slot a width, so calls of several widths do not capture in turn either
+
+
+def test_a_lightly_loaded_server_does_not_hold_pagerank_queries_back(tmp_path):
+    out = run(tmp_path, """
+    for (long others : {0, 1, 10, 63, 64, 1000}) {
+        const PprGate d = ppr_gate(0, 0, others), own = ppr_gate(5, 3, others);
+        if (own.us != 5 || own.batch != 3) return 1;
+        printf("%d/%d ", d.us, d.batch);
+    }
+    """)
+    assert out.split() == 4 * ["20000/8"] + 2 * ["70000/16"]
