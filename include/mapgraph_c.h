@@ -131,7 +131,10 @@ typedef struct mg_options {
     double  max_queue_sizing; /* reference "max_queue_sizing" (queue = sizing * n)         */
     int32_t alpha;          /* BFS top-down -> bottom-up switch (frontier edges > unexplored/alpha) */
     int32_t beta;           /* BFS bottom-up -> top-down switch (frontier < n/beta)        */
-    int32_t batch_alpha;    /* mg_bfs_batch push -> pull switch (frontier edges > m/batch_alpha); 0 = 4 */
+    int32_t batch_alpha;    /* mg_bfs_batch push -> pull switch (frontier edges > m/batch_alpha); 0 = 16
+                               on graphs of mean degree 8 and more, 4 on others and in searches
+                               of more than 30 levels (sparse graphs, whose rows run side by side,
+                               do not pull)                                                */
     int32_t batch_beta;     /* mg_bfs_batch pull -> push switch (frontier edges < m/batch_beta); 0 = 16  */
     int32_t sssp_delta;     /* SSSP bucket width: relax only distances below the current
                                bucket bound, raised by sssp_delta when no such distance is
@@ -141,7 +144,9 @@ typedef struct mg_options {
                                whole-GPU levels unbucketed (dense levels pull); -1 =
                                unbucketed.  Batched searches: the width of every level, 0 =
                                about 4 x the mean weight (4 x the largest on sparse graphs,
-                               whose rows run side by side), -1 = unbucketed               */
+                               whose rows run side by side), -1 = unbucketed; without effect on
+                               graphs of mean degree 8 and more with in-edges, whose rounds
+                               pull every vertex (searches of up to 48 rounds)             */
     int32_t ppr_iters;      /* personalized PageRank iterations (0 = 20)                   */
     int32_t sssp_bucket_edges; /* mg_sssp: once the pending vertices of a whole-GPU level
                                have fewer out-edges than this, the bucket bound is lifted
@@ -259,7 +264,8 @@ int mg_ppr_batch(mg_graph *g, const int32_t *srcs, int32_t k, float *rank_out,
  *   MG_TUNE_BFS         alpha, beta, level_grid            (mg_bfs)
  *   MG_TUNE_SSSP        sssp_delta, sssp_bucket_edges, level_grid   (mg_sssp)
  *   MG_TUNE_BFS_BATCH   batch_alpha, batch_beta             (mg_bfs_batch)
- *   MG_TUNE_SSSP_BATCH  sssp_delta                          (mg_sssp_batch)
+ *   MG_TUNE_SSSP_BATCH  sssp_delta                          (mg_sssp_batch; kept as *start
+ *                       where the search pulls, which has no bucket width)
  * Coordinate descent from *start (NULL: the defaults) over candidate values, two
  * passes: each setting is timed on the sample sources (device time, median of reps
  * runs after a warm-up; single-source kinds: up to 64 sources, summed; batched kinds:

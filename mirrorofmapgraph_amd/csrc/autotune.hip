@@ -12,12 +12,14 @@
 // `reps` runs after a warm-up run) and kept when it is at least 3% faster than the
 // best so far; two passes over the parameters.  Every candidate's results must be
 // bit-identical to the starting setting's (they are unique answers), otherwise the
-// tuner stops with MG_ERR_DEVICE: a parameter must never change a result.
+// tuner stops with MG_ERR_DEVICE: a parameter must never change a result.  A batched SSSP
+// that is pulled (batch_pull.hip) has no bucket width: its candidates are the same search, so
+// none is kept for what are differences between runs.
 #include <algorithm>
 #include <cstring>
 #include <vector>
 
-#include "engine.h"
+#include "batch.h"
 
 namespace mg {
 namespace {
@@ -142,7 +144,8 @@ extern "C" int mg_autotune(mg_graph *g, int32_t what, const int32_t *srcs, int32
                 o.*p.field = v;
                 double ms = 0;
                 if ((rc = t.measure(o, &ms))) return rc;
-                if (ms < 0.97 * t_best) {
+                const bool same = what == MG_TUNE_SSSP_BATCH && pull_wanted(search_graph(g, o, nullptr));
+                if (!same && ms < 0.97 * t_best) {
                     t_best = ms;
                     cur = o;
                     moved = true;

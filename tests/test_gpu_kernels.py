@@ -696,3 +696,12 @@ def test_batch_pull_sizes_that_share_a_row_width(mg, oracle, device):
         for k in (1, 32, 3, 31, 32, 4, 33, 64, 35, 64, 5):
             for lo in (0, 64 - k):
                 assert np.array_equal(dg.sssp_batch(srcs[lo:lo + k]), exp[lo:lo + k]), (k, lo)
+
+
+def test_the_tuner_keeps_no_bucket_width_for_a_pulled_batch(mg, device):
+    g = mg.rmat_graph(12, 16, seed=3, weight_max=64)
+    with mg.Graph(g, symmetric=True) as dg:
+        for start in (0, 7):
+            for _ in range(3):
+                best, _ = dg.autotune("sssp_batch", mg.pick_sources(g, 4, seed=1), start=mg.options(sssp_delta=start), reps=1)
+                assert best.sssp_delta == start
