@@ -705,3 +705,24 @@ def test_the_tuner_keeps_no_bucket_width_for_a_pulled_batch(mg, device):
             for _ in range(3):
                 best, _ = dg.autotune("sssp_batch", mg.pick_sources(g, 4, seed=1), start=mg.options(sssp_delta=start), reps=1)
                 assert best.sssp_delta == start
+
+
+@pytest.mark.parametrize("symmetric", [False, True])
+@pytest.mark.parametrize("n", [255, 257, 65537, 262145, 524321])
+def test_frontier_slices_of_the_general_batches(mg, oracle, device, monkeypatch, n, symmetric):
+    # as above for both directions, with batches on the shared frontier: the memory of the other route
+    # for sparse graphs is refused
+    g = random_graph(mg, n, 3 * n if symmetric else 6 * n, seed=n + 1, symmetric=symmetric, wmax=16)
+    assert g.m < 8 * n
+    srcs = np.array([int(np.argmax(g.degrees())), n - 1, 0], np.int32)
+    bfs = [oracle.bfs(g.row_offsets, g.col_idx, int(s)) for s in srcs]
+    sssp = [oracle.sssp(g.row_offsets, g.col_idx, g.values, int(s)) for s in srcs]
+    with mg.Graph(g, symmetric=symmetric) as dg:
+        assert np.array_equal(dg.bfs(int(srcs[0])), bfs[0]) and np.array_equal(dg.sssp(int(srcs[0])), sssp[0])
+        for batch, exp, at in ((dg.bfs_batch, bfs, "1"), (dg.sssp_batch, sssp, "01")):
+            before = dg.device_bytes()
+            monkeypatch.setenv("MG_FAIL_ALLOC_AT", at)  # the first allocation from here on
+            for got, row in zip(batch(srcs), exp):
+                assert np.array_equal(got, row)
+            monkeypatch.delenv("MG_FAIL_ALLOC_AT")
+            assert dg.device_bytes() >= before + 4 * mg.MG_BATCH_MAX * n  # the general route's rows
