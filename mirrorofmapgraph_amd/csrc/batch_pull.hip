@@ -64,7 +64,7 @@ struct PullDev {
     ChunkRec *tasks = nullptr;
     int ntasks = 0;
     int *D = nullptr, *rows = nullptr;
-    int64_t d_cap = 0, rows_cap = 0, bytes = 0;
+    int64_t d_cap = 0, rows_cap = 0;
 };
 
 // Rows of INT_MAX (0 past slot k), nothing changed, every slot live.
@@ -400,9 +400,8 @@ void pull_release(mg_graph *g) {
     free_dev(p->rows);
     delete p;
     p = nullptr;
+    g->steps->pull_bytes = 0;
 }
-
-int64_t pull_dev_size(const PullDev *p) { return p->bytes; }
 
 bool pull_wanted(const mg_graph *g) {
     return g->m >= PULL_DEGREE * (int64_t)g->n && ((g->flags & MG_GRAPH_SYMMETRIC) || g->col_off) &&
@@ -433,7 +432,7 @@ static int pull_tasks(mg_graph *g, PullDev &p, const int *d_in_off) {
         copy_on(g->stream, p.tasks, t.data(), sizeof(ChunkRec) * t.size(), hipMemcpyHostToDevice) != hipSuccess)
         return set_error(MG_ERR_DEVICE, "task copy failed");
     p.ntasks = (int)t.size();
-    p.bytes += (int64_t)(sizeof(ChunkRec) * t.size());
+    g->steps->pull_bytes += (int64_t)(sizeof(ChunkRec) * t.size());
     return MG_OK;
 }
 
@@ -465,7 +464,7 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
         }
         p.ctl = reinterpret_cast<Ctl *>(c);
         p.live = reinterpret_cast<uint32_t *>(l);
-        p.bytes += (int64_t)sizeof(Ctl) + (int64_t)sizeof(LevelPart) * PART_GROUPS + 96 + 16LL * g->n;
+        g->steps->pull_bytes += (int64_t)sizeof(Ctl) + (int64_t)sizeof(LevelPart) * PART_GROUPS + 96 + 16LL * g->n;
     }
     const bool direct = plan_delivery(g, out, 4 * (size_t)k * g->n, o.out_on_device).by_kernel;
     auto grow = [&](int **buf, int64_t *cap, int64_t need) -> int {
@@ -474,12 +473,12 @@ int pull_batch(mg_graph *g, const int32_t *row_of, const int32_t *srcs, int32_t 
         pull_drop_steps(g);
         free_dev(*buf);
         *buf = nullptr;
-        p.bytes -= 4 * *cap;
+        g->steps->pull_bytes -= 4 * *cap;
         *cap = 0;
         const int arc = alloc_i32(buf, (size_t)need);
         if (arc) return arc;
         *cap = need;
-        p.bytes += 4 * need;
+        g->steps->pull_bytes += 4 * need;
         return MG_OK;
     };
     if ((rc = grow(&p.D, &p.d_cap, (int64_t)ks * g->n))) return rc;

@@ -53,7 +53,6 @@ struct TeamsDev {
     int64_t rows_cap = 0;
     int *pairs = nullptr;      // row starts (MG_BATCH_MAX + 1), then the sources by row
     int64_t pairs_cap = 0;
-    int64_t bytes = 0;
 };
 
 struct TeamsArgs {
@@ -245,21 +244,20 @@ void teams_release(mg_graph *g) {
     free_dev(t->pairs);
     delete t;
     t = nullptr;
+    g->steps->teams_bytes = 0;
 }
-
-int64_t teams_dev_size(const TeamsDev *t) { return t->bytes; }
 
 // A device buffer of at least `need` bytes (an old one is too small and freed).
 template <class T>
-static int teams_buf(TeamsDev &t, T **p, int64_t old_bytes, int64_t need) {
+static int teams_buf(mg_graph *g, T **p, int64_t old_bytes, int64_t need) {
     free_dev(*p);
     *p = nullptr;
-    t.bytes -= old_bytes;
+    g->steps->teams_bytes -= old_bytes;
     if (alloc_refused() || hipMalloc((void **)p, (size_t)std::max<int64_t>(need, 16)) != hipSuccess) {
         *p = nullptr;
         return set_error(MG_ERR_OOM, "batched search state of %lld bytes: allocation failed", (long long)need);
     }
-    t.bytes += need;
+    g->steps->teams_bytes += need;
     return MG_OK;
 }
 
@@ -283,15 +281,15 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
     const int front = (int)std::min(1e6, (sssp ? 2 : 1) * TEAMS_FRONT * std::sqrt((double)g->n));
     const int least = std::min(TEAM_WGS, std::max(g->steps->teams_rule[sssp].wgs, (front + room - 1) / room));
     const int per_xcd = std::min({(k + XCDS - 1) / XCDS, TEAMS_MAX / XCDS, TEAMS_GRID / XCDS / least}), teams = per_xcd * XCDS;
-    if (!t.ctl && (rc = teams_buf(t, &t.ctl, 0, sizeof(TeamsCtl)))) return rc;
+    if (!t.ctl && (rc = teams_buf(g, &t.ctl, 0, sizeof(TeamsCtl)))) return rc;
     if (!t.h_ctl && hipHostMalloc((void **)&t.h_ctl, sizeof(TeamsCtl), hipHostMallocDefault) != hipSuccess)
         return set_error(MG_ERR_OOM, "hipHostMalloc failed");
     if (t.teams < teams) {
         const int64_t had = t.teams;
         t.teams = 0;
-        if ((rc = teams_buf(t, &t.team, had * (int64_t)sizeof(TeamCtl), teams * (int64_t)sizeof(TeamCtl))) ||
-            (rc = teams_buf(t, &t.recs, had * 8 * (int64_t)TEAM_RECS, teams * 8 * (int64_t)TEAM_RECS)) ||
-            (rc = teams_buf(t, &t.bits, had * 16 * (int64_t)nwords, teams * 16 * (int64_t)nwords)))
+        if ((rc = teams_buf(g, &t.team, had * (int64_t)sizeof(TeamCtl), teams * (int64_t)sizeof(TeamCtl))) ||
+            (rc = teams_buf(g, &t.recs, had * 8 * (int64_t)TEAM_RECS, teams * 8 * (int64_t)TEAM_RECS)) ||
+            (rc = teams_buf(g, &t.bits, had * 16 * (int64_t)nwords, teams * 16 * (int64_t)nwords)))
             return rc;
         t.teams = teams;
     }
@@ -307,7 +305,7 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
     if (t.pairs_cap < (int64_t)pairs.size()) {
         const int64_t had = t.pairs_cap;
         t.pairs_cap = 0;
-        if ((rc = teams_buf(t, &t.pairs, 4 * had, 4 * (int64_t)pairs.size()))) return rc;
+        if ((rc = teams_buf(g, &t.pairs, 4 * had, 4 * (int64_t)pairs.size()))) return rc;
         t.pairs_cap = (int64_t)pairs.size();
     }
     const int64_t cells = (int64_t)k * g->n;
@@ -315,7 +313,7 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
     if (!direct && t.rows_cap < cells) {
         const int64_t had = t.rows_cap;
         t.rows_cap = 0;
-        if ((rc = teams_buf(t, &t.rows, 4 * had, 4 * cells))) return rc;
+        if ((rc = teams_buf(g, &t.rows, 4 * had, 4 * cells))) return rc;
         t.rows_cap = cells;
     }
     TeamsArgs a{};

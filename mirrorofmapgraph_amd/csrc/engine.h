@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstring>
 #include <mutex>
@@ -321,9 +322,7 @@ void gas_release(mg_graph *g);
 void batch_release(mg_graph *g);
 void ppr_release(mg_graph *g);
 void teams_release(mg_graph *g);
-int64_t teams_dev_size(const TeamsDev *t);
 void pull_release(mg_graph *g);
-int64_t pull_dev_size(const PullDev *p);
 int64_t batch_dev_size(const BatchDev *b);  // device bytes held by a batch context
 int64_t ppr_dev_size(const PprDev *p);
 // SSSP bucket width for options o on graph g (a huge value when unbucketed).
@@ -338,6 +337,8 @@ struct mg_graph_steps {
     mg::PprDev *pdev = nullptr;                  // batched personalized PageRank context
     mg::TeamsDev *teams = nullptr;               // batched searches by teams
     mg::PullDev *pull = nullptr;                 // batched SSSP by pulling
+    // Device bytes of the last two, which a running call may release (read without the lock)
+    std::atomic<int64_t> teams_bytes{0}, pull_bytes{0};
     // What batched searches found out about the graph (kept when the routes' state is released)
     bool pull_deep = false;              // SSSP took too many rounds to be pulled
     mg::TeamsRule teams_rule[2];         // BFS, SSSP

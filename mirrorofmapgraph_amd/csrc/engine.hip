@@ -598,8 +598,7 @@ int mg_graph_device_bytes(const mg_graph *g, int64_t *bytes) {
         for (const BatchDev *p : g->steps->bdev)
             if (p) b += batch_dev_size(p);
     if (g->steps && g->steps->pdev) b += ppr_dev_size(g->steps->pdev);
-    if (g->steps && g->steps->teams) b += teams_dev_size(g->steps->teams);
-    if (g->steps && g->steps->pull) b += pull_dev_size(g->steps->pull);
+    if (g->steps) b += g->steps->teams_bytes + g->steps->pull_bytes;
     if (g->perm) b += 8LL * g->n;
     if (g->twin) {
         int64_t tb = 0;

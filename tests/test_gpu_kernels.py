@@ -726,3 +726,28 @@ def test_frontier_slices_of_the_general_batches(mg, oracle, device, monkeypatch,
                 assert np.array_equal(got, row)
             monkeypatch.delenv("MG_FAIL_ALLOC_AT")
             assert dg.device_bytes() >= before + 4 * mg.MG_BATCH_MAX * n  # the general route's rows
+
+
+def test_device_bytes_beside_calls_that_release_state(mg, oracle, device):
+    # asked for from another thread while batches make, grow and release their routes' state
+    import threading
+
+    g = _clique_chain(mg, 60, 20)
+    g.values = mg.hash_weights(g, 2, 30)
+    sparse = random_graph(mg, 120000, 350000, 3, wmax=20)
+    stop, seen = threading.Event(), []
+    with mg.Graph(g, symmetric=True) as a, mg.Graph(sparse, symmetric=True) as b:
+        def ask():
+            while not stop.is_set():
+                seen.extend((a.device_bytes(), b.device_bytes()))
+
+        t = threading.Thread(target=ask)
+        t.start()
+        for k in (1, 40, 100):
+            srcs = np.arange(k, dtype=np.int32)
+            for dg, h in ((a, g), (b, sparse)):
+                assert np.array_equal(dg.sssp_batch(srcs)[0], oracle.sssp(h.row_offsets, h.col_idx, h.values, 0))
+                assert np.array_equal(dg.bfs_batch(srcs)[-1], oracle.bfs(h.row_offsets, h.col_idx, k - 1))
+        stop.set()
+        t.join()
+    assert seen and min(seen) > 0 and max(seen) < 1 << 34
