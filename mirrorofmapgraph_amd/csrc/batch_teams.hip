@@ -382,7 +382,10 @@ int teams_try(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs
             if (!rc) rule.succeeded();
             return rc;
         }
-        if (!rule.retry(end, wgs, TEAM_WGS, again)) break;
+        if (!rule.retry(end, wgs, TEAM_WGS, again)) {
+            if (rule.skip == 0) return MG_OK;  // the next call tries again
+            break;
+        }
         again = again || end == TEAMS_SHORT;
     }
     teams_release(g);  // room for the general route
