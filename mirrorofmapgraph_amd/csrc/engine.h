@@ -108,7 +108,7 @@ struct Workspace {
     uint32_t *bm[3] = {nullptr, nullptr, nullptr};
     ChunkRec *chunks = nullptr;
     LevelPart *part = nullptr;  // PART_GROUPS slots
-    TeamCtl *team = nullptr;  // team of the narrow levels and its queues (team.h; not on search views)
+    TeamCtl *team = nullptr;  // team of the narrow levels and its queues (team.h; behind part; not on search views)
     uint64_t *team_rec = nullptr;
     Ctl *ctl = nullptr;
     Ctl *h_ctl = nullptr;     // pinned host mirror

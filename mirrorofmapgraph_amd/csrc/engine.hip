@@ -79,8 +79,6 @@ static void free_workspace(Workspace &ws) {
     for (auto &p : ws.bm) dfree(p);
     dfree(ws.chunks);
     dfree(ws.part);
-    dfree(ws.team);
-    dfree(ws.team_rec);
     dfree(ws.ctl);
     if (ws.h_ctl) (void)hipHostFree(ws.h_ctl);
     if (ws.h_reach) (void)hipHostFree(ws.h_reach);
@@ -112,17 +110,23 @@ int ensure_workspace(mg_graph *g) {
     // lists longer than CHUNK_T in the tile path), over both push views
     ws.chunk_need = 2 * (g->m / TASK + g->m / (LANE_T + 1)) + 2 * (g->m / CHUNK + g->m / CHUNK_T) + 64;
     ws.chunk_cap = ws.chunk_need;
+    // the team's state lies behind the level counters: one allocation, as a twin's first search makes them
+    static_assert(sizeof(TeamCtl) % 128 == 0 && sizeof(LevelPart) * PART_GROUPS % 128 == 0, "cache lines of their own");
+    const size_t team_parts = g->arrays_borrowed ? 0 : (sizeof(TeamCtl) + 8 * TEAM_RECS + sizeof(LevelPart) - 1) / sizeof(LevelPart);
     int rc = 0;
     if ((rc = dalloc(&ws.vals, n)) || (rc = dalloc(&ws.q[0], n)) || (rc = dalloc(&ws.q[1], n)) ||
         (rc = dalloc(&ws.q[2], n)) || (rc = dalloc(&ws.hard, n)) || (rc = dalloc(&ws.visited, ws.nwords)) ||
         (rc = dalloc(&ws.bm[0], ws.nwords)) || (rc = dalloc(&ws.bm[1], ws.nwords)) ||
         (rc = dalloc(&ws.bm[2], ws.nwords)) || (rc = dalloc(&ws.chunks, ws.chunk_cap)) ||
-        (rc = dalloc(&ws.part, PART_GROUPS)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2 * TAIL_WGS)) ||
+        (rc = dalloc(&ws.part, PART_GROUPS + team_parts)) || (rc = dalloc(&ws.ctl, 1)) || (rc = dalloc(&ws.d_reach, 2 * TAIL_WGS)) ||
         (rc = dalloc(&ws.tail_cnt, LAST_WG_INTS)) ||
-        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP)) ||
-        (!g->arrays_borrowed && ((rc = dalloc(&ws.team, 1)) || (rc = dalloc(&ws.team_rec, TEAM_RECS))))) {
+        (rc = dalloc(&ws.trace, 2 * (size_t)TRACE_CAP))) {
         free_workspace(ws);
         return rc;
+    }
+    if (team_parts) {
+        ws.team = reinterpret_cast<TeamCtl *>(ws.part + PART_GROUPS);
+        ws.team_rec = reinterpret_cast<uint64_t *>(ws.team + 1);
     }
     hipError_t e = hipHostMalloc((void **)&ws.h_ctl, sizeof(Ctl), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void **)&ws.h_reach, 2 * sizeof(unsigned long long), hipHostMallocDefault);
