@@ -49,8 +49,8 @@ struct PprArgs {
 // and the contribution array of a 4M-vertex graph is 128 MB instead of 1 GB.
 
 // What bounds an iteration is reading rows that the L2 does not hold: at R-MAT scale 20 (31.4M
-// edges) and W = 8, 28M lines of 128 bytes go from L2 to L1 (92 us at 64 bytes a clock and CU)
-// and 7M from memory to the L2 (4.8 TB/s), at W = 64 4.5 GB (5.7 TB/s).  Below that the
+// edges) and W = 8, 29M lines of 128 bytes go from L2 to L1 (92 us at 64 bytes a clock and CU)
+// and 6.4M from memory to the L2 (4.5 TB/s), at W = 64 4.7 GB (6.4 TB/s).  Below that the
 // address unit is: it takes a quad of lanes a clock whatever the lanes load, so a lane loads
 // four columns (16 bytes) at once, and four sources.  Four columns, a list per group and one
 // launch an iteration, against a column per lane, a list per wave and three launches, us an
