@@ -35,6 +35,10 @@ constexpr int64_t TEAMS_DEGREE = 8;
 // the same.  2048^2 grid, 256 rows (two workgroups a team outgrown, the call run again in
 // general / so): BFS 410 / 159 ms, SSSP 884 / 284; on the 512^2 grid two workgroups do.
 constexpr int TEAMS_FRONT = 4;
+// State kept when the route is given up for a while: freeing what kernels have used takes 0.5
+// ms, half of a small call (one source on a random graph of 100,000 vertices: first call 1.63
+// ms so, 1.07 kept), and the next try would make it again.  Larger ones are released.
+constexpr int64_t TEAMS_KEEP = 64LL << 20;
 
 struct TeamsCtl {
     int arrived[16];             // workgroups that came, by XCD
@@ -42,17 +46,11 @@ struct TeamsCtl {
     unsigned long long edges, te, nr;  // edges relaxed; TEPS count and reached vertices
 };
 
-// Device state of a graph's team batches.
+// Device state of a graph's team batches: one block, laid out anew by each call (nothing in it
+// outlives one).
 struct TeamsDev {
-    int teams = 0;
-    TeamsCtl *ctl = nullptr, *h_ctl = nullptr;
-    TeamCtl *team = nullptr;
-    uint64_t *recs = nullptr;
-    uint32_t *bits = nullptr;  // per team: 4 bitmaps
-    int *rows = nullptr;       // results, when they stay here or go to host memory
-    int64_t rows_cap = 0;
-    int *pairs = nullptr;      // row starts (MG_BATCH_MAX + 1), then the sources by row
-    int64_t pairs_cap = 0;
+    char *block = nullptr;
+    int64_t cap = 0;
 };
 
 struct TeamsArgs {
@@ -235,30 +233,10 @@ __global__ __launch_bounds__(BLK) void teams_stats(TeamsArgs a, int unreached) {
 void teams_release(mg_graph *g) {
     TeamsDev *&t = g->steps->teams;
     if (!t) return;
-    free_dev(t->ctl);
-    if (t->h_ctl) (void)hipHostFree(t->h_ctl);
-    free_dev(t->team);
-    free_dev(t->recs);
-    free_dev(t->bits);
-    free_dev(t->rows);
-    free_dev(t->pairs);
+    free_dev(t->block);
     delete t;
     t = nullptr;
     g->steps->teams_bytes = 0;
-}
-
-// A device buffer of at least `need` bytes (an old one is too small and freed).
-template <class T>
-static int teams_buf(mg_graph *g, T **p, int64_t old_bytes, int64_t need) {
-    free_dev(*p);
-    *p = nullptr;
-    g->steps->teams_bytes -= old_bytes;
-    if (alloc_refused() || hipMalloc((void **)p, (size_t)std::max<int64_t>(need, 16)) != hipSuccess) {
-        *p = nullptr;
-        return set_error(MG_ERR_OOM, "batched search state of %lld bytes: allocation failed", (long long)need);
-    }
-    g->steps->teams_bytes += need;
-    return MG_OK;
 }
 
 // Workgroups launched for a team of wgs; fewer with MG_TEAM_LAUNCH in the environment, for
@@ -272,7 +250,6 @@ static int teams_launch(int wgs) {
 // *wgs how many workgroups a team was to have.
 static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs, int32_t npairs, int32_t k,
                        int32_t *out, const mg_options &o, mg_stats *stats, const CallTimer &timer, int *end, int *wgs) {
-    int rc;
     TeamsDev *&tp = g->steps->teams;
     if (!tp && !(tp = new (std::nothrow) TeamsDev())) return set_error(MG_ERR_OOM, "host allocation failed");
     TeamsDev &t = *tp;
@@ -281,18 +258,6 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
     const int front = (int)std::min(1e6, (sssp ? 2 : 1) * TEAMS_FRONT * std::sqrt((double)g->n));
     const int least = std::min(TEAM_WGS, std::max(g->steps->teams_rule[sssp].wgs, (front + room - 1) / room));
     const int per_xcd = std::min({(k + XCDS - 1) / XCDS, TEAMS_MAX / XCDS, TEAMS_GRID / XCDS / least}), teams = per_xcd * XCDS;
-    if (!t.ctl && (rc = teams_buf(g, &t.ctl, 0, sizeof(TeamsCtl)))) return rc;
-    if (!t.h_ctl && hipHostMalloc((void **)&t.h_ctl, sizeof(TeamsCtl), hipHostMallocDefault) != hipSuccess)
-        return set_error(MG_ERR_OOM, "hipHostMalloc failed");
-    if (t.teams < teams) {
-        const int64_t had = t.teams;
-        t.teams = 0;
-        if ((rc = teams_buf(g, &t.team, had * (int64_t)sizeof(TeamCtl), teams * (int64_t)sizeof(TeamCtl))) ||
-            (rc = teams_buf(g, &t.recs, had * 8 * (int64_t)TEAM_RECS, teams * 8 * (int64_t)TEAM_RECS)) ||
-            (rc = teams_buf(g, &t.bits, had * 16 * (int64_t)nwords, teams * 16 * (int64_t)nwords)))
-            return rc;
-        t.teams = teams;
-    }
     // the sources by row
     std::vector<int32_t> pairs((size_t)MG_BATCH_MAX + 1 + (size_t)npairs, 0);
     int32_t *start = pairs.data(), *list = start + MG_BATCH_MAX + 1;
@@ -302,28 +267,41 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
         std::vector<int32_t> at(start, start + k);
         for (int i = 0; i < npairs; ++i) list[at[(size_t)row_of[i]]++] = srcs[i];
     }
-    if (t.pairs_cap < (int64_t)pairs.size()) {
-        const int64_t had = t.pairs_cap;
-        t.pairs_cap = 0;
-        if ((rc = teams_buf(g, &t.pairs, 4 * had, 4 * (int64_t)pairs.size()))) return rc;
-        t.pairs_cap = (int64_t)pairs.size();
-    }
     const int64_t cells = (int64_t)k * g->n;
     const bool direct = plan_delivery(g, out, 4 * (size_t)cells, o.out_on_device).as_state;
-    if (!direct && t.rows_cap < cells) {
-        const int64_t had = t.rows_cap;
-        t.rows_cap = 0;
-        if ((rc = teams_buf(g, &t.rows, 4 * had, 4 * cells))) return rc;
-        t.rows_cap = cells;
+    int64_t need = 0;
+    auto part = [&](int64_t bytes) {
+        const int64_t at = need;
+        need += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    const int64_t at_ctl = part(sizeof(TeamsCtl)), at_pairs = part(4 * (int64_t)pairs.size()),
+                  at_team = part(teams * (int64_t)sizeof(TeamCtl)), at_recs = part(teams * 8 * (int64_t)TEAM_RECS),
+                  at_bits = part(teams * 16 * (int64_t)nwords), at_rows = part(direct ? 0 : 4 * cells);
+    if (t.cap < need) {
+        free_dev(t.block);
+        t.block = nullptr;
+        t.cap = 0;
+        g->steps->teams_bytes = 0;
+        if (alloc_refused() || hipMalloc((void **)&t.block, (size_t)need) != hipSuccess) {
+            t.block = nullptr;
+            return set_error(MG_ERR_OOM, "batched search state of %lld bytes: allocation failed", (long long)need);
+        }
+        t.cap = need;
+        g->steps->teams_bytes = need;
     }
     TeamsArgs a{};
-    a.ctl = t.ctl;
-    a.team = t.team;
-    a.recs = t.recs;
-    a.bits = t.bits;
-    a.rows = direct ? out : t.rows;
-    a.row_start = t.pairs;
-    a.srcs = t.pairs + MG_BATCH_MAX + 1;
+    a.ctl = reinterpret_cast<TeamsCtl *>(t.block + at_ctl);
+    a.team = reinterpret_cast<TeamCtl *>(t.block + at_team);
+    a.recs = reinterpret_cast<uint64_t *>(t.block + at_recs);
+    a.bits = reinterpret_cast<uint32_t *>(t.block + at_bits);
+    int *const own = reinterpret_cast<int *>(t.block + at_rows), *const d_pairs = reinterpret_cast<int *>(t.block + at_pairs);
+    a.rows = direct ? out : own;
+    a.row_start = d_pairs;
+    a.srcs = d_pairs + MG_BATCH_MAX + 1;
+    // (the graph's pinned control block is free between searches)
+    static_assert(sizeof(TeamsCtl) <= sizeof(Ctl), "copied to the pinned block");
+    TeamsCtl *const h = reinterpret_cast<TeamsCtl *>(g->ws.h_ctl);
     a.off = g->row_off;
     a.adj = g->col;
     a.w = g->w;
@@ -337,7 +315,7 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
     a.delta = o.sssp_delta < 0 ? LLONG_MAX / 4 : o.sssp_delta > 0 ? o.sssp_delta : std::max<long long>(1, 4LL * g->max_weight);
     const int unreached = sssp ? INT_MAX : -1;
     MG_HIP(hipEventRecord(g->ev0, g->stream));
-    MG_HIP(hipMemcpyAsync(t.pairs, pairs.data(), 4 * pairs.size(), hipMemcpyHostToDevice, g->stream));
+    MG_HIP(hipMemcpyAsync(d_pairs, pairs.data(), 4 * pairs.size(), hipMemcpyHostToDevice, g->stream));
     hipLaunchKernelGGL(teams_init, dim3(grid_blocks_cap(std::max<int64_t>(cells / 4, 4LL * teams * nwords), BLK, 4 * MAX_GRID)),
                        dim3(BLK), 0, g->stream, a, unreached);
     const int grid = teams * teams_launch(a.wgs);
@@ -348,22 +326,23 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
                            g->stream, a, unreached);
     MG_HIP(hipGetLastError());
     MG_HIP(hipEventRecord(g->ev1, g->stream));
-    MG_HIP(hipMemcpyAsync(t.h_ctl, t.ctl, sizeof(TeamsCtl), hipMemcpyDeviceToHost, g->stream));
+    MG_HIP(hipMemcpyAsync(h, a.ctl, sizeof(TeamsCtl), hipMemcpyDeviceToHost, g->stream));
     MG_HIP(hipStreamSynchronize(g->stream));
     *wgs = a.wgs;
-    *end = t.h_ctl->end;
+    *end = h->end;
     if (*end != TEAMS_DONE) return MG_OK;
     float ms = 0;
     MG_HIP(hipEventElapsedTime(&ms, g->ev0, g->ev1));
     if (stats) {
         std::memset(stats, 0, sizeof *stats);
-        stats->iterations = t.h_ctl->levels;
-        stats->edges_examined = (int64_t)t.h_ctl->edges;
-        stats->edges_traversed = (int64_t)t.h_ctl->te;
-        stats->vertices_reached = (int64_t)t.h_ctl->nr;
+        stats->iterations = h->levels;
+        stats->edges_examined = (int64_t)h->edges;
+        stats->edges_traversed = (int64_t)h->te;
+        stats->vertices_reached = (int64_t)h->nr;
         stats->device_ms = ms;
     }
-    if (!direct && (rc = deliver(g, out, t.rows, 4 * (size_t)cells, o.out_on_device))) return rc;
+    if (!direct)
+        if (const int rc = deliver(g, out, own, 4 * (size_t)cells, o.out_on_device)) return rc;
     if (stats) stats->host_ms = timer.ms();
     return MG_OK;
 }
@@ -383,8 +362,8 @@ int teams_try(mg_graph *g, bool sssp, const int32_t *row_of, const int32_t *srcs
             return rc;
         }
         if (!rule.retry(end, wgs, TEAM_WGS, again)) {
-            if (rule.skip == 0) return MG_OK;  // the next call tries again
-            break;
+            if (rule.skip > 0 && g->steps->teams_bytes > TEAMS_KEEP) teams_release(g);  // (else the next call tries again)
+            return MG_OK;
         }
         again = again || end == TEAMS_SHORT;
     }

@@ -65,14 +65,14 @@ struct TeamsRule {
     // run the call again by teams, else the general route takes it.  A larger team helps only
     // where a whole one was outgrown; a short one says nothing about the graph, and gets one
     // more try (`again`: it had that).  A failure that belongs to the graph and the sources is
-    // not repeated at once: the next 16 calls, then 64, 256, ... don't try.
+    // not repeated at once: the next 32 calls, then 128, 512, ... don't try.
     bool retry(int end, int wgs_now, int wgs_most, bool again) {
         if (end == TEAMS_SHORT) return !again;
         if (end == TEAMS_OUTGROWN && wgs_now < wgs_most) {
             wgs = 2 * wgs_now;
             return true;
         }
-        wait = wait == 0 ? 16 : wait < 1 << 20 ? 4 * wait : wait;
+        wait = wait == 0 ? 32 : wait < 1 << 20 ? 4 * wait : wait;
         skip = wait;
         return false;
     }

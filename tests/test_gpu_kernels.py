@@ -572,9 +572,11 @@ def test_batched_routes_refused_memory_go_the_general_way(mg, oracle, device, mo
         assert np.array_equal(dg.bfs_batch(more)[:3], bfs) and np.array_equal(dg.sssp_batch(more)[:3], sssp)
 
 
+@pytest.mark.parametrize("k", [3, 256])
 @pytest.mark.parametrize("which", ["teams-bfs", "teams-sssp", "levels", "pull"])
-def test_batched_routes_given_up_hold_no_memory(mg, oracle, device, monkeypatch, which):
-    # after a search that its route could not hold, the graph holds what the general route needs
+def test_batched_routes_given_up_hold_no_memory(mg, oracle, device, monkeypatch, which, k):
+    # after a search that its route could not hold, the graph holds what the general route needs, and of
+    # the teams at most 64 MB
     import ctypes as C
 
     if which.startswith("teams"):
@@ -582,11 +584,11 @@ def test_batched_routes_given_up_hold_no_memory(mg, oracle, device, monkeypatch,
     else:
         g = _clique_chain(mg, 60, 20)
         g.values = mg.hash_weights(g, 2, 30)
-    srcs = np.array([0, g.n // 2, g.n - 1], np.int32)
+    srcs = np.resize(np.array([0, g.n // 2, g.n - 1], np.int32), k)
     sssp = which in ("teams-sssp", "pull")
     one = (lambda s: oracle.sssp(g.row_offsets, g.col_idx, g.values, s)) if sssp else (
         lambda s: oracle.bfs(g.row_offsets, g.col_idx, s))
-    exp = np.stack([one(int(s)) for s in srcs])
+    exp = np.resize(np.stack([one(int(s)) for s in srcs[:3]]), (k, g.n))
 
     def grown(general):
         with mg.Graph(g, symmetric=True) as dg:
@@ -596,8 +598,8 @@ def test_batched_routes_given_up_hold_no_memory(mg, oracle, device, monkeypatch,
                     assert np.array_equal(dg.sssp_batch(srcs) if sssp else dg.bfs_batch(srcs), exp)
             elif which == "levels":  # (a device result needs no rows)
                 hip, p, o = C.CDLL("libamdhip64.so"), C.c_void_p(), mg.options(out_on_device=1)
-                assert hip.hipMalloc(C.byref(p), C.c_size_t(12 * g.n)) == 0
-                mg.check(mg.lib().mg_bfs_batch(dg.handle, srcs.ctypes.data_as(C.POINTER(C.c_int32)), 3, p, C.byref(o), None))
+                assert hip.hipMalloc(C.byref(p), C.c_size_t(4 * k * g.n)) == 0
+                mg.check(mg.lib().mg_bfs_batch(dg.handle, srcs.ctypes.data_as(C.POINTER(C.c_int32)), k, p, C.byref(o), None))
                 hip.hipFree(p)
             else:
                 monkeypatch.setenv("MG_FAIL_ALLOC_AT", "1")  # the faster route's first allocation is refused
@@ -605,7 +607,8 @@ def test_batched_routes_given_up_hold_no_memory(mg, oracle, device, monkeypatch,
                 monkeypatch.delenv("MG_FAIL_ALLOC_AT")
             return dg.device_bytes() - before
 
-    assert grown(False) == grown(True)
+    kept = grown(False) - grown(True)
+    assert kept == 0 or (which.startswith("teams") and k == 3 and 0 < kept <= 64 << 20)
 
 
 def _widening(mg, first, doublings):
@@ -653,16 +656,16 @@ def test_batch_teams_beside_a_hub_in_another_component(mg, oracle, device, sssp)
     g.values = mg.hash_weights(g, 3, 9)
     one = (lambda s: oracle.sssp(g.row_offsets, g.col_idx, g.values, s)) if sssp else (
         lambda s: oracle.bfs(g.row_offsets, g.col_idx, s))
-    near, far = np.array([0, hub, a.n - 1], np.int32), np.arange(a.n, a.n + 3, dtype=np.int32)
+    near, far = np.array([0, hub, a.n - 1], np.int32), np.arange(a.n, a.n + 20, dtype=np.int32)
     with mg.Graph(g, symmetric=True) as dg:
         batch = dg.sssp_batch if sssp else dg.bfs_batch
         assert np.array_equal(batch(near), np.stack([one(int(s)) for s in near]))
         before, exp = dg.device_bytes(), np.stack([one(int(s)) for s in far])
-        for calls in range(40):
+        for calls in range(60):
             assert np.array_equal(batch(far), exp)
-            if dg.device_bytes() > before:  # the teams' state is there again
+            if dg.device_bytes() > before:  # state for more teams: they took the call
                 break
-        assert calls < 39
+        assert calls < 59
         assert np.array_equal(batch(near), np.stack([one(int(s)) for s in near]))
 
 

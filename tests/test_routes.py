@@ -74,7 +74,7 @@ def test_teams_grow_only_where_a_whole_team_was_outgrown(tmp_path):
     s.succeeded();
     printf("%d %d %d", tries, until, s.wanted());
     """)
-    assert out == "8 17 1"  # 16 + 64 + 256 + ... calls between them
+    assert out == "7 33 1"  # 32 + 128 + 512 + ... calls between them
 
 
 def test_a_team_that_soon_hands_back_is_asked_for_less_often(tmp_path):
