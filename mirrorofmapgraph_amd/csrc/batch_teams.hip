@@ -140,7 +140,8 @@ __device__ __forceinline__ int teams_next(const TeamsArgs &a, const TeamSeat &t,
                 if (firsts) out.queue(first, firsts, v, o);
             }
             // the out-edges' field carries the row
-            word = team_over(out.word(it)) ? team_word(it, true, out.hub, 0, row + 1)
+            if (out.hub) team_set_hub(t.ctl);
+            word = team_over(out.word(it)) ? team_word(it, true, 0, 0, row + 1)
                                            : team_word(it, false, out.nrec, min(out.nf, 0xffff), row + 1);
         }
     }
@@ -150,10 +151,10 @@ __device__ __forceinline__ int teams_next(const TeamsArgs &a, const TeamSeat &t,
     return (int)(low & 0xfffff) - 1;
 }
 
-__device__ __forceinline__ void teams_row_done(const TeamsArgs &a, const TeamSeat &t, int L, bool over, bool hub) {
+__device__ __forceinline__ void teams_row_done(const TeamsArgs &a, const TeamSeat &t, int L, bool over) {
     if (t.rank != 0 || lane_id() != 0) return;
     atomicMax(&a.ctl->levels, L);
-    if (over) atomicMax(&a.ctl->end, hub ? TEAMS_HUB : t.size < a.wgs * (BLK / WAVE) ? TEAMS_SHORT : TEAMS_OUTGROWN);
+    if (over) atomicMax(&a.ctl->end, ld_dev(&t.ctl->hub) ? TEAMS_HUB : t.size < a.wgs * (BLK / WAVE) ? TEAMS_SHORT : TEAMS_OUTGROWN);
 }
 
 __global__ __launch_bounds__(BLK) void teams_bfs(TeamsArgs a) {
@@ -165,13 +166,12 @@ __global__ __launch_bounds__(BLK) void teams_bfs(TeamsArgs a) {
         const int row = teams_next<false>(a, t, visited, it);
         if (row < 0) return;
         int L = 0;
-        bool over = false, hub = false;
-        team_bfs(t, a.off, a.adj, visited, a.rows + (int64_t)row * a.n, L, it, [&](uint64_t w) {
+        bool over = false;
+        team_bfs<true>(t, a.off, a.adj, visited, a.rows + (int64_t)row * a.n, L, it, [&](uint64_t w) {
             over = wave_ballot(team_over(w)) != 0;
-            hub = over && team_hub(w);
             return over || wave_ballot(team_nf(w) != 0) == 0 || L >= a.limit;
         });
-        teams_row_done(a, t, L, over, hub);
+        teams_row_done(a, t, L, over);
         if (!over) teams_clear(visited, a.nwords, t);
     }
 }
@@ -198,8 +198,8 @@ __global__ __launch_bounds__(BLK) void teams_sssp(TeamsArgs a) {
         s.dist = a.rows + (int64_t)row * a.n;
         s.thr = a.delta;
         int L = 0;
-        const bool done = team_sssp(t, s, L, it, [](uint64_t) {}, [](uint64_t) { return false; });
-        teams_row_done(a, t, L, !done, s.hub);
+        const bool done = team_sssp<true>(t, s, L, it, [](uint64_t) {}, [](uint64_t) { return false; });
+        teams_row_done(a, t, L, !done);
         if (done && L >= a.limit) {  // stopped short: the frontier and the far vertices are left
             teams_clear(s.bm0, a.nwords, t);
             teams_clear(s.bm1, a.nwords, t);
@@ -272,7 +272,7 @@ static int teams_batch(mg_graph *g, bool sssp, const int32_t *row_of, const int3
     int64_t need = 0;
     auto part = [&](int64_t bytes) {
         const int64_t at = need;
-        need += (bytes + 255) / 256 * 256;
+        need += (bytes + 4095) / 4096 * 4096;
         return at;
     };
     const int64_t at_ctl = part(sizeof(TeamsCtl)), at_pairs = part(4 * (int64_t)pairs.size()),

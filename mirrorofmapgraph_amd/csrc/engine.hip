@@ -111,7 +111,7 @@ int ensure_workspace(mg_graph *g) {
     ws.chunk_need = 2 * (g->m / TASK + g->m / (LANE_T + 1)) + 2 * (g->m / CHUNK + g->m / CHUNK_T) + 64;
     ws.chunk_cap = ws.chunk_need;
     // the team's state lies behind the level counters: one allocation, as a twin's first search makes them
-    static_assert(sizeof(TeamCtl) % 128 == 0 && sizeof(LevelPart) * PART_GROUPS % 128 == 0, "cache lines of their own");
+    static_assert(sizeof(LevelPart) * PART_GROUPS % 4096 == 0 && 8 * TEAM_RECS % 4096 == 0, "aligned as allocations of their own");
     const size_t team_parts = g->arrays_borrowed ? 0 : (sizeof(TeamCtl) + 8 * TEAM_RECS + sizeof(LevelPart) - 1) / sizeof(LevelPart);
     int rc = 0;
     if ((rc = dalloc(&ws.vals, n)) || (rc = dalloc(&ws.q[0], n)) || (rc = dalloc(&ws.q[1], n)) ||
@@ -125,8 +125,8 @@ int ensure_workspace(mg_graph *g) {
         return rc;
     }
     if (team_parts) {
-        ws.team = reinterpret_cast<TeamCtl *>(ws.part + PART_GROUPS);
-        ws.team_rec = reinterpret_cast<uint64_t *>(ws.team + 1);
+        ws.team_rec = reinterpret_cast<uint64_t *>(ws.part + PART_GROUPS);
+        ws.team = reinterpret_cast<TeamCtl *>(ws.team_rec + TEAM_RECS);
     }
     hipError_t e = hipHostMalloc((void **)&ws.h_ctl, sizeof(Ctl), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void **)&ws.h_reach, 2 * sizeof(unsigned long long), hipHostMallocDefault);

@@ -52,7 +52,7 @@ __device__ __forceinline__ int rec_len(uint64_t r) { return (int)(r >> 62) + 1; 
 
 // What a member posts after a level (of its part of the next frontier): tag (the
 // meeting's number, 11 bits), overflow, records, vertices, out-edges.  A member
-// whose counts do not fit posts the overflow bit, and one record if a vertex has too many edges.
+// whose counts do not fit posts the overflow bit.
 __host__ __device__ constexpr uint64_t team_word(int tag, bool over, int rec, int nf, int mf) {
     return ((uint64_t)(tag & 0x7ff) << 53) | ((uint64_t)over << 52) | ((uint64_t)rec << 36) | ((uint64_t)nf << 20) |
            (uint64_t)mf;
@@ -66,16 +66,14 @@ __device__ __forceinline__ int team_mf(uint64_t w) { return (int)w & 0xfffff; }
 struct TeamCtl {
     int leader, pad0[31];  // XCD of the team + 1 (0: none yet)
     int joined, pad1[31];
-    int size, pad2[31];    // workgroups, once closed
+    int size;              // workgroups, once closed
+    int hub, pad2[30];     // batches: a member overflowed at a vertex of more than TEAM_DEG edges
     uint64_t word[2][TEAM_SIZE];  // posts, by meeting parity
     int least[2][TEAM_SIZE];      // SSSP: a member's smallest waiting distance, by meeting parity
 };
 
 // The XCD this wave runs on (hardware register XCC_ID).
 __device__ __forceinline__ int xcd_id() { return (int)__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15; }
-
-// The whole wave: a vertex of too many edges is among what overflowed.
-__device__ __forceinline__ bool team_hub(uint64_t w) { return wave_ballot(team_over(w) && team_rec(w) != 0) != 0; }
 
 // Before the launch that forms the team (one workgroup of at least 2 * TEAM_SIZE threads):
 // nobody has joined, nothing is posted (meetings are numbered from 1).
@@ -118,6 +116,10 @@ __device__ __forceinline__ bool team_join(TeamCtl *t, int wgs, int &rank, int &s
     rank = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE * s_size + s_rank);
     size = __builtin_amdgcn_readfirstlane(s_size * (BLK / WAVE));
     return true;
+}
+
+__device__ __forceinline__ void team_set_hub(TeamCtl *t) {
+    if (lane_id() == 0) __hip_atomic_store(&t->hub, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Whole wave: everything it wrote has reached the L2, then its post.
@@ -219,7 +221,7 @@ struct TeamSeat {
 struct TeamOut {
     uint64_t *recs;
     int nrec = 0, nf = 0, mf = 0;
-    bool hub = false;
+    bool hub = false;  // a vertex of more than TEAM_DEG edges
     __device__ TeamOut(uint64_t *all, int meeting, int rank)
         : recs(all + ((size_t)(meeting & 1) * TEAM_SIZE + rank) * TEAM_SEG) {}
     // Whole wave: queues vertex v with edge slots o.a..o.b for every lane with `first`
@@ -241,7 +243,7 @@ struct TeamOut {
     }
     __device__ __forceinline__ uint64_t word(int meeting) const {
         const bool o = hub || nrec > TEAM_SEG || nf > 0xffff || mf > 0xfffff;
-        return o ? team_word(meeting, true, hub, 0, 0) : team_word(meeting, false, nrec, nf, mf);
+        return o ? team_word(meeting, true, 0, 0, 0) : team_word(meeting, false, nrec, nf, mf);
     }
 };
 

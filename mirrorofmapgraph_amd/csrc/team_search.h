@@ -14,12 +14,13 @@ namespace mg {
 // BFS: the neighbour id, then its claim (test-and-set of the visited bit) and its offsets
 // together, so a claimed vertex joins the next frontier as records of its edge range and
 // the next level starts at the adjacency.  Runs from meeting `it` (posted, frontier L) until
-// stop(words) says so; it is asked at every meeting, by every wave alike.
+// stop(words) says so; it is asked at every meeting, by every wave alike.  HUB: TeamCtl::hub is
+// set where that is why a member overflows (in the posts it cost the single searches 0.6%).
 // Bound by the chain record -> neighbour -> claim / offsets -> post -> meeting, about 3 us
 // at 1000 vertices a level.  2048^2 grid: 15.6 ms when first written like this, 20.9 ms with
 // a lane per record (four edges each) and workgroup-wide queues; 8 workgroups 22 ms; one /
 // four pieces in step 16.6 / 15.6 ms.
-template <class Stop>
+template <bool HUB = false, class Stop>
 __device__ __forceinline__ void team_bfs(const TeamSeat &t, const int *off, const int *adj, uint32_t *visited,
                                          int *depth, int &L, int &it, Stop stop) {
     const int sub = lane_id() % TEAM_EDGES;
@@ -66,6 +67,7 @@ __device__ __forceinline__ void team_bfs(const TeamSeat &t, const int *off, cons
         for (; p + t.size < in.pieces; p += 2 * t.size) expand(std::integral_constant<int, 2>(), p);
         if (p < in.pieces) expand(std::integral_constant<int, 1>(), p);
         ++L;
+        if (HUB && out.hub) team_set_hub(t.ctl);
         team_post(t.ctl, it + 1, t.rank, out.word(it + 1));
     }
 }
@@ -85,13 +87,12 @@ struct TeamSssp {
     int nwords, limit;
     long long delta, thr, unbucketed;  // no distance reaches a bound of `unbucketed`
     long long ex = 0;                  // edges this lane relaxed
-    bool hub = false;                  // overflowed at a vertex of too many edges
 };
 
 // Runs from meeting `it` (posted, frontier L) until the search ends or reaches its level
 // limit (true), or until a member overflows or wide(words) says so (false; bitmap
 // L % 3 then holds the frontier).  closed(words) is called after each level.
-template <class Closed, class Wide>
+template <bool HUB = false, class Closed, class Wide>
 __device__ __forceinline__ bool team_sssp(const TeamSeat &t, TeamSssp &s, int &L, int &it, Closed closed, Wide wide) {
     const int lane = lane_id(), sub = lane % TEAM_EDGES;
     // (locals: with its fields read in place the struct stayed in scratch memory)
@@ -108,10 +109,7 @@ __device__ __forceinline__ bool team_sssp(const TeamSeat &t, TeamSssp &s, int &L
         const TeamIn in = team_in(t.recs, it, w);
         long long sweep_from = -1;  // >= 0: sweep, dropping waiting distances below this
         // the same decisions in every wave
-        if (wave_ballot(team_over(w)) != 0) {
-            s.hub = team_hub(w);
-            break;
-        }
+        if (wave_ballot(team_over(w)) != 0) break;
         if (!swept) closed(w);
         if (L >= limit) {
             done = true;
@@ -167,6 +165,7 @@ __device__ __forceinline__ bool team_sssp(const TeamSeat &t, TeamSssp &s, int &L
             if (lane == 0)
                 __hip_atomic_store(&t.ctl->least[(it + 1) & 1][t.rank], least, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (HUB && out.hub) team_set_hub(t.ctl);
             team_post(t.ctl, it + 1, t.rank, out.word(it + 1));
             continue;
         }
@@ -228,6 +227,7 @@ __device__ __forceinline__ bool team_sssp(const TeamSeat &t, TeamSssp &s, int &L
         for (; p + t.size < in.pieces; p += 2 * t.size) relax(std::integral_constant<int, 2>(), p);
         if (p < in.pieces) relax(std::integral_constant<int, 1>(), p);
         ++L;
+        if (HUB && out.hub) team_set_hub(t.ctl);
         team_post(t.ctl, it + 1, t.rank, out.word(it + 1));
     }
     s.thr = thr;
